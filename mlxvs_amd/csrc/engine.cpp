@@ -175,6 +175,22 @@ class Arena {
     return p;
   }
 
+  // Whether `bytes` more can be taken (in pieces of any size) without an
+  // allocation that fails: room is made now.  A fixed arena answers no.
+  bool reserve(size_t bytes) {
+    if (fixed_) return false;
+    for (const auto& c : chunks_)
+      if (c.size - c.used >= bytes) return true;
+    const size_t size = std::max<size_t>(bytes, 64u << 20);
+    char* p = nullptr;
+    if (hipMalloc(&p, size) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    chunks_.push_back({p, size, 0});
+    return true;
+  }
+
   void end(hipStream_t s) {
     if (!done_) check_hip(hipEventCreateWithFlags(&done_, hipEventDisableTiming), "hipEventCreate");
     check_hip(hipEventRecord(done_, s), "hipEventRecord");
@@ -460,7 +476,7 @@ int max_merge_segments(int k, int T) {
 // where the levels would each wait on a few workgroups.
 void merge_lists(Arena& ar, hipStream_t s, const uint64_t* part, int nseg, int T, int k,
                  int64_t nq, int metric, const float* qnorm, int dist_mode, int32_t* ids,
-                 float* dists, int* flags) {
+                 float* dists, int* flags, const kern::SplitState* split = nullptr) {
   const int64_t C = (int64_t)nseg * T;
   // (not in a fixed workspace: its survivor buffer, nq * C ranks, is larger
   // than the levels' outputs)
@@ -469,7 +485,7 @@ void merge_lists(Arena& ar, hipStream_t s, const uint64_t* part, int nseg, int T
     uint64_t* surv = ar.take<uint64_t>((size_t)(nq * C));
     uint64_t* tails = flags ? ar.take<uint64_t>((size_t)nq * nseg) : nullptr;
     kern::BoundMergeArgs bm{part, nseg, T, k, (int)nq, metric, qnorm, dist_mode, surv, tails,
-                            ids, dists, flags};
+                            ids, dists, flags, split};
     launch(s, "merge", [&] { return kern::launch_bound_merge(bm, s); });
     return;
   }
@@ -499,7 +515,7 @@ void merge_lists(Arena& ar, hipStream_t s, const uint64_t* part, int nseg, int T
     first = false;
   }
   kern::MergeArgs ma{mpart, mseg, mT, k, (int)nq, metric, qnorm, dist_mode, ids, dists, flags,
-                     sentinel, first ? 1 : 0};
+                     sentinel, first ? 1 : 0, split};
   launch(s, "merge", [&] { return kern::launch_merge(ma, s); });
 }
 
@@ -530,6 +546,127 @@ BoundPlan shared_bound(int k, int T, int slots, int lists) {
   return b;
 }
 
+// Float32 rows (and cosine's unit rows) multiplied as two binary16 pieces
+// each on the fp16 MFMA (SplitState, knn_kernels.h), for batches whose matrix
+// work outweighs the pass that makes the pieces.
+// Where it starts to pay, measured on real values, k = 10, float32 kernels
+// against pieces: 1M x 128 rows, 128 queries 0.44 / 0.49 ms, 256 0.67 / 0.59,
+// 2,048 4.05 / 1.67; 100k x 128, 512 queries 0.182 / 0.197, 2,048 0.49 / 0.27;
+// 100k x 16, 2,048 queries 0.21 / 0.20 (the select costs as much as the matrix
+// work of 32 values, so fewer count as 32).
+constexpr int64_t kSplitMinQueries = 256;
+constexpr double kSplitMinWork = 8e9;  // n nq max(d, 32)
+// Device memory for the pieces and the operands of the float32 route: as
+// much as the rows take, so large collections keep the float32 kernels.
+constexpr size_t kSplitMaxBytes = size_t(16) << 30;
+
+// Returns false when the route does not apply (nothing was enqueued).
+// `allow`: prefilter words as FusedArgs.
+bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, const uint32_t* allow,
+                     int64_t allow_stride, int32_t* ids, float* dists) {
+  Arena& ar = ss.arena();
+  hipStream_t s = ss.stream();
+  const int64_t n = in.n, nq = in.nq;
+  const int d = in.d;
+  const bool cosine = metric == kern::kCosine, l2 = metric == kern::kL2;
+  if (ar.fixed() || (in.f16 && !cosine) || nq < kSplitMinQueries || nq >= (int64_t(1) << 31) ||
+      (double)n * (double)nq * std::max(d, 32) < kSplitMinWork)
+    return false;
+  const int T = allow ? 16 : list_len_float(k);
+  const int sld = round_up(d, 8), ld32 = round_up(d, 4);
+  if (!kern::fused_split_supported(sld, T) || !kern::fused_supported(ld32, T, false)) return false;
+  const int64_t qblocks = (nq + kQueriesPerBlock - 1) / kQueriesPerBlock;
+  const int tile_rows = 2 * kern::kTileRows;
+  const SplitPlan plan = plan_splits(n, qblocks, k, T, 2, tile_rows,
+                                     device_slots(kern::fused_split_blocks_per_cu(sld, T)), true,
+                                     max_merge_segments(k, T));
+  if (!plan.ok || (plan.rows_per_split + tile_rows) * sld * 4 >= (int64_t(1) << 31)) return false;
+  // the float32 route's operands: unit rows (cosine), or the rows in place,
+  // or a padded copy
+  const bool in_place = !cosine && (uintptr_t)in.base % 16 == 0 &&
+                        (uintptr_t)in.queries % 16 == 0 && d % 4 == 0;
+  const size_t rows_all = (size_t)(n + nq);
+  const size_t bytes = rows_all * ((size_t)sld * 4 + (in_place ? 0 : (size_t)ld32 * 4)) + (64u << 10);
+  if (bytes > kSplitMaxBytes || !ar.reserve(bytes)) return false;
+
+  uint16_t* bhi = ar.take<uint16_t>((size_t)n * sld);
+  uint16_t* blo = ar.take<uint16_t>((size_t)n * sld);
+  uint16_t* qhi = ar.take<uint16_t>((size_t)nq * sld);
+  uint16_t* qlo = ar.take<uint16_t>((size_t)nq * sld);
+  auto* st = ar.take<kern::SplitState>(1);
+  const int f16 = in.f16 ? 1 : 0;
+  const void *kbase = in.base, *kq = in.queries;
+  float *bnorm = nullptr, *qnorm = nullptr, *seed = nullptr;
+  float *ubn = nullptr, *uqn = nullptr;  // cosine: |b|^2, |q|^2
+  kern::SplitInitArgs si{(const float*)in.base, (const float*)in.queries, n, nq, d, d,
+                         cosine ? 1 : 0, st};
+  launch(s, "prep", [&] { return kern::launch_split_init(si, s); });
+  if (cosine) {
+    ubn = ar.take<float>((size_t)n);
+    uqn = ar.take<float>((size_t)nq);
+    kern::PrepArgs pb{in.base, n, d, d, f16, ubn, nullptr, nullptr, 0, 0};
+    kern::PrepArgs pq{in.queries, nq, d, d, f16, uqn, nullptr, nullptr, 0, 0};
+    launch(s, "prep", [&] { return kern::launch_norms(pb, s); });
+    launch(s, "prep", [&] { return kern::launch_norms(pq, s); });
+  }
+  if (l2) {
+    bnorm = ar.take<float>((size_t)n);
+    seed = ar.take<float>((size_t)n);
+    qnorm = ar.take<float>((size_t)nq);
+  }
+  kern::SplitRowsArgs sb{in.base, n, d, d, f16, ubn, bnorm, 1, seed, bhi, blo, sld, 0, st};
+  kern::SplitRowsArgs sq{in.queries, nq, d, d, f16, uqn, qnorm, 0, nullptr, qhi, qlo, sld, 1, st};
+  launch(s, "prep", [&] { return kern::launch_split_rows(sb, s); });
+  launch(s, "prep", [&] { return kern::launch_split_rows(sq, s); });
+  if (!in_place) {
+    float* pb = ar.take<float>((size_t)n * ld32);
+    float* pq = ar.take<float>((size_t)nq * ld32);
+    kern::PrepArgs tb{in.base, n, d, d, f16, nullptr, ubn, pb, ld32, 0};
+    kern::PrepArgs tq{in.queries, nq, d, d, f16, nullptr, uqn, pq, ld32, 0};
+    // (the redo of cosine queries reads the unit rows on every route)
+    if (!(cosine && k > T)) tb.split = tq.split = st;
+    launch(s, "prep", [&] { return kern::launch_transform(tb, s); });
+    launch(s, "prep", [&] { return kern::launch_transform(tq, s); });
+    kbase = pb;
+    kq = pq;
+  }
+
+  const int nseg = 2 * plan.nsplit;
+  uint64_t* part = ar.take<uint64_t>((size_t)nq * nseg * T);
+  const int slots = kern::bound_slots_for(T);
+  const BoundPlan bp = shared_bound(k, T, slots, nseg);
+  uint32_t* gkey = ar.take<uint32_t>((size_t)nq * slots);
+  launch(s, "prep", [&] { return kern::launch_bounds_init(gkey, nq, slots, bp.m, s); });
+  // one launch per route: all but the one that the rows take return at once
+  kern::FusedArgs fa{bhi, qhi, seed, n, (int)nq, sld, cosine ? kern::kInnerProduct : metric,
+                     plan.rows_per_split, plan.nsplit, T, k, part, gkey, bp.m, bp.pubj,
+                     (int)qblocks, plan.xcd ? 1 : 0};
+  fa.allow = allow;
+  fa.allow_stride = allow_stride;
+  fa.split = st;
+  fa.base_lo = blo;
+  fa.queries_lo = qlo;
+  fa.route = 1;
+  launch(s, "fused_hi", [&] { return kern::launch_fused_f16(fa, s); });
+  fa.route = 2;
+  launch(s, "fused_split", [&] { return kern::launch_fused_split(fa, s); });
+  fa.route = 0;
+  fa.base = kbase;
+  fa.queries = kq;
+  fa.bnorm = bnorm;
+  fa.ld = ld32;
+  launch(s, "fused_f32", [&] { return kern::launch_fused_f32(fa, s); });
+  int* flags = T < k ? ar.take<int>((size_t)nq) : nullptr;
+  merge_lists(ar, s, part, nseg, T, k, nq, metric, qnorm, 0, ids, dists, flags, st);
+  if (T >= k) return true;
+  kern::RedoArgs ra{cosine ? kbase : in.base, cosine ? kq : in.queries, bnorm, qnorm, flags, n,
+                    (int)nq, cosine ? ld32 : d, d, 0, 0, metric, 0, k, ids, dists};
+  ra.allow = allow;
+  ra.allow_stride = allow_stride;
+  launch(s, "redo", [&] { return kern::launch_redo(ra, s); });
+  return true;
+}
+
 void float_knn(Session& ss, const FloatInputs& in, int k, int metric, int32_t* ids,
                float* dists) {
   Arena& ar = ss.arena();
@@ -553,6 +690,7 @@ void float_knn(Session& ss, const FloatInputs& in, int k, int metric, int32_t* i
     launch(s, "prep", [&] { return kern::launch_filter_rows(in.allow, nq, n, rows_w, s); });
     allow = rows_w;
   }
+  if (float_knn_split(ss, in, k, metric, allow, allow_stride, ids, dists)) return;
   // Operand preparation.  Cosine: unit rows in fp32 (the reference
   // normalises in float32, src/knn.cpp:30-33, also for float16 input,
   // src/utils.h:28).  Otherwise the rows are used in place when they are

@@ -129,23 +129,38 @@ __global__ __launch_bounds__(256) void row_norms_kernel(PrepArgs a) {
   }
 }
 
-// Element-wise row copy into an [n, out_ld] buffer, zero-padded past d:
-// fp32 or binary16 out, optionally divided by max(sqrt(norm), 1e-30)
-// (unit rows, reference src/knn.cpp:30-33).
-__global__ __launch_bounds__(256) void rows_transform_kernel(PrepArgs a) {
-  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (e >= a.n * a.out_ld) return;
-  const int64_t r = e / a.out_ld;
-  const int j = (int)(e % a.out_ld);
-  float v = j < a.d ? load_elem(a.x, a.f16, r * a.ld + j) : 0.0f;
-  if (a.unit_norms) {
-    const float nrm = sqrtf(a.unit_norms[r]);
-    v = v / (nrm > 1e-30f ? nrm : 1e-30f);
+// Row copy into an [n, out_ld] buffer (out_ld a multiple of 4), zero-padded
+// past d: fp32 or binary16 out, optionally divided by max(sqrt(norm), 1e-30)
+// (unit rows, reference src/knn.cpp:30-33).  Four values a lane, its row and
+// column by one division of type Int (32 bits up to 2^32 vectors of four; a
+// 64-bit division per value set the pace before: one query over 166,214 x 708
+// fp32 rows, which are padded to 736, 0.57 -> 0.44 ms a call).
+template <typename Int>
+__global__ __launch_bounds__(256) void rows_transform_kernel(PrepArgs a, Int total) {
+  if (a.split && split_route(a.split->flags) != 0) return;
+  const uint32_t lv = (uint32_t)a.out_ld / 4;
+  // (the host keeps the grid's last step below Int's range)
+  for (Int e = (Int)blockIdx.x * 256 + threadIdx.x; e < total; e += (Int)gridDim.x * 256) {
+    const Int q = e / lv;
+    const int64_t r = (int64_t)q;
+    const int c = 4 * (int)(e - q * lv);
+    float v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = c + u < a.d ? load_elem(a.x, a.f16, r * a.ld + c + u) : 0.0f;
+    if (a.unit_norms) {
+      const float nrm = sqrtf(a.unit_norms[r]);
+      const float den = nrm > 1e-30f ? nrm : 1e-30f;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = v[u] / den;
+    }
+    if (a.out_f16) {
+      typedef _Float16 halfx4 __attribute__((ext_vector_type(4)));
+      *(halfx4*)((_Float16*)a.out + r * a.out_ld + c) =
+          halfx4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+    } else {
+      *(floatx4*)((float*)a.out + r * a.out_ld + c) = floatx4{v[0], v[1], v[2], v[3]};
+    }
   }
-  if (a.out_f16)
-    ((_Float16*)a.out)[e] = (_Float16)v;
-  else
-    ((float*)a.out)[e] = v;
 }
 
 // ---- fused MFMA distance + per-lane top-T -------------------------------------
@@ -235,8 +250,23 @@ constexpr int fused_rb() {
 // lists (ids = buffer columns).  MODE 2: IVF-Flat item, scores written to
 // the candidate buffers.
 // FILT: the dense search with a prefilter (FusedArgs::allow), lists of 16.
-template <bool F16, int DH, int T, bool L2, int MODE = 0, bool FILT = false>
+// NP = 2 (F16): float32 rows as two binary16 pieces (SplitState).  A tile
+// carries both, and each pair of fragments feeds lo x hi, hi x lo and hi x
+// hi; the scores come out in the pieces' scale (the seeds are in it, the
+// merge takes it out again).  Against the float32 MFMA, whose rate is a
+// sixteenth of the fp16 MFMA's, three products cost 3/16 of the matrix time,
+// and a value's product enters the float32 sum with one rounding per eight
+// values instead of one per value.
+template <bool F16, int DH, int T, bool L2, int MODE = 0, bool FILT = false, int NP = 1>
 __global__ __launch_bounds__(256, (fused_min_blocks<F16, DH>())) void fused_kernel(FusedArgs a) {
+  static_assert(NP == 1 || (F16 && MODE == 0), "pieces are binary16");
+  uint32_t sflags = 0;
+  if constexpr (MODE == 0) {
+    if (a.split) {
+      sflags = a.split->flags;
+      if (split_route(sflags) != a.route) return;
+    }
+  }
   using E = typename std::conditional<F16, _Float16, float>::type;
   constexpr int EPV = F16 ? 8 : 4;    // elements per 16-byte vector
   constexpr int D = 2 * DH;           // padded dims of an LDS row
@@ -258,6 +288,8 @@ __global__ __launch_bounds__(256, (fused_min_blocks<F16, DH>())) void fused_kern
   // other and does not wait for them before every read
   __shared__ __align__(16) E tile0[TR * ROWE];
   __shared__ __align__(16) E tile1[TR * ROWE];
+  __shared__ __align__(16) E low0[NP == 2 ? TR * ROWE : 8];  // the lo pieces
+  __shared__ __align__(16) E low1[NP == 2 ? TR * ROWE : 8];
   __shared__ __align__(16) float tnorm0[64];  // 64: a norm load writes 64 lanes
   __shared__ __align__(16) float tnorm1[64];
   // lists of 16 over 64-row tiles (k > 10, often k > 16: many lanes pass)
@@ -354,19 +386,23 @@ __global__ __launch_bounds__(256, (fused_min_blocks<F16, DH>())) void fused_kern
   // row, zero past ld and for lanes without a query (plain global loads: a
   // buffer resource per lane would be looped over the wavefront's queries)
   typedef E vecq __attribute__((ext_vector_type(EPV)));
-  vecq qf[QV];
-  {
-    const E* qr = (const E*)a.queries + (int64_t)(qvalid ? q : 0) * ld;
+  vecq qf[QV], ql[NP == 2 ? QV : 1];
+  auto query_frags = [&](const void* rows, vecq* f) {
+    const E* qr = (const E*)rows + (int64_t)(qvalid ? q : 0) * ld;
 #pragma unroll
     for (int v = 0; v < QV; ++v) {
       u32x4 w = {0u, 0u, 0u, 0u};
       if (qvalid && h * DH + v * EPV < ld) w = *(const u32x4*)(qr + h * DH + v * EPV);
-      qf[v] = __builtin_bit_cast(vecq, w);
+      f[v] = __builtin_bit_cast(vecq, w);
     }
-  }
+  };
+  query_frags(a.queries, qf);
+  if constexpr (NP == 2) query_frags(a.queries_lo, ql);
+  const bool lowlow = NP == 2 && split_low_low(sflags);
+  const char* lbase = NP == 2 ? (const char*)((const E*)a.base_lo + r0 * ld) : nullptr;
 
-  // tile t into (dst, ndst)
-  auto issue_loads = [&](E* dst, float* ndst, int t) {
+  // tile t into (dst, ldst, ndst)
+  auto issue_loads = [&](E* dst, E* ldst, float* ndst, int t) {
     // (the saturating difference is a vector operation: readfirstlane keeps
     // the resource scalar, else the loads would be looped per lane value)
     const uint32_t done = (uint32_t)t * tile_bytes;
@@ -375,6 +411,12 @@ __global__ __launch_bounds__(256, (fused_min_blocks<F16, DH>())) void fused_kern
         __builtin_amdgcn_make_buffer_rsrc((void*)(sbase + done), (short)0, left, 0x00020000);
 #pragma unroll
     for (int j = 0; j < NPF; ++j) load16_to_lds(rb, dst + 64 * (wv * NPF + j) * EPV, voff[j]);
+    if constexpr (NP == 2) {
+      const __amdgpu_buffer_rsrc_t rl =
+          __builtin_amdgcn_make_buffer_rsrc((void*)(lbase + done), (short)0, left, 0x00020000);
+#pragma unroll
+      for (int j = 0; j < NPF; ++j) load16_to_lds(rl, ldst + 64 * (wv * NPF + j) * EPV, voff[j]);
+    }
     if (l2 && wv == 0) {
       const int r = t * TR;
       const uint32_t nleft = __builtin_amdgcn_readfirstlane(r < nrows ? (uint32_t)(nrows - r) * 4u : 0u);
@@ -407,12 +449,12 @@ __global__ __launch_bounds__(256, (fused_min_blocks<F16, DH>())) void fused_kern
   const uint32_t* fw = filt ? a.allow + (int64_t)(qvalid ? q : 0) * a.allow_stride : nullptr;
   const int64_t r1g = r0 + nrows;
 
-  if (ntiles > 0) issue_loads(tile0, tnorm0, 0);
+  if (ntiles > 0) issue_loads(tile0, low0, tnorm0, 0);
   // LATE (the buffered select): the select of tile t runs after the
   // barrier that ends its MFMAs, and tile t + 2 is fetched into tile t's
   // buffers after it, so two tiles are fetched ahead here
   constexpr bool LATE = BUF;
-  if (LATE && ntiles > 0) issue_loads(tile1, tnorm1, 1);
+  if (LATE && ntiles > 0) issue_loads(tile1, low1, tnorm1, 1);
   // nothing may be outstanding at the loop head: the query fragments are
   // read in every iteration, and a pending prologue load would otherwise
   // make each iteration wait for its own tile prefetch as well
@@ -428,7 +470,7 @@ __global__ __launch_bounds__(256, (fused_min_blocks<F16, DH>())) void fused_kern
   auto bound_tile = [](int t) { return (t & 3) == 0 || t < 8; };
   // tile t from (cur, ncur); tile t + 1 into (nxt, nnxt) (LATE: tile t + 2
   // into (cur, ncur), after the select)
-  auto step = [&](E* cur, float* ncur, E* nxt, float* nnxt, int t) {
+  auto step = [&](E* cur, E* lcur, float* ncur, E* nxt, E* lnxt, float* nnxt, int t) {
     // read before the tile prefetch, so that waiting for it (in the
     // epilogue) does not wait for the prefetch
     if constexpr (MODE != 2)
@@ -448,7 +490,7 @@ __global__ __launch_bounds__(256, (fused_min_blocks<F16, DH>())) void fused_kern
     // the next tile into the other buffer (read in the previous tile, which
     // every wavefront has left: the barrier below); unconditional (past the
     // last tile the range is empty and the loads write zeros)
-    if constexpr (!LATE) issue_loads(nxt, nnxt, t + 1);
+    if constexpr (!LATE) issue_loads(nxt, lnxt, nnxt, t + 1);
     __builtin_amdgcn_sched_barrier(0);
     // L2: the accumulators start at the rows' -|b|^2 / 2 (the norms array
     // holds them), so they end at the half score q.b - |b|^2 / 2 with no
@@ -467,21 +509,34 @@ __global__ __launch_bounds__(256, (fused_min_blocks<F16, DH>())) void fused_kern
       // share the swizzle)
       const E* arow = cur + col * ROWE;
       const int sw = col & SWZ;
-      auto frag_at = [&](int r, int v) { return arow + r * 32 * ROWE + EPV * ((h * QV + v) ^ sw); };
+      auto slot_of = [&](int r, int v) { return r * 32 * ROWE + EPV * ((h * QV + v) ^ sw); };
+      auto frag_at = [&](int r, int v) { return arow + slot_of(r, v); };
       // A fragments one step ahead: the LDS reads of step v + 1 are issued
       // before the MFMAs of step v (a scheduling barrier keeps them there),
       // so the MFMA chain does not wait for LDS at every step
       typedef typename std::conditional<F16, halfx8, floatx4>::type fragv;
-      fragv av[2][RB];
+      fragv av[2][RB], al[2][NP == 2 ? RB : 1];
+      const E* lrow = lcur + col * ROWE;
+      auto fetch = [&](int v) {
 #pragma unroll
-      for (int r = 0; r < RB; ++r) av[0][r] = *(const fragv*)frag_at(r, 0);
+        for (int r = 0; r < RB; ++r) {
+          if constexpr (NP == 2) al[v & 1][r] = *(const fragv*)(lrow + slot_of(r, v));
+          av[v & 1][r] = *(const fragv*)frag_at(r, v);
+        }
+      };
+      fetch(0);
 #pragma unroll
       for (int v = 0; v < QV; ++v) {
-        if (v + 1 < QV) {
-#pragma unroll
-          for (int r = 0; r < RB; ++r) av[(v + 1) & 1][r] = *(const fragv*)frag_at(r, v + 1);
-        }
+        if (v + 1 < QV) fetch(v + 1);
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (NP == 2) {
+#pragma unroll
+          for (int r = 0; r < RB; ++r)
+            acc[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[v & 1][r], qf[v], acc[r], 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < RB; ++r)
+            acc[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[v & 1][r], ql[v], acc[r], 0, 0, 0);
+        }
         if constexpr (F16) {
 #pragma unroll
           for (int r = 0; r < RB; ++r)
@@ -493,6 +548,16 @@ __global__ __launch_bounds__(256, (fused_min_blocks<F16, DH>())) void fused_kern
             for (int r = 0; r < RB; ++r)
               acc[r] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[v & 1][r][u], qf[v][u], acc[r], 0,
                                                             0, 0);
+        }
+      }
+      if constexpr (NP == 2) {
+        if (lowlow) {  // (short values, rare: the products that keep their sums exact)
+#pragma unroll
+          for (int v = 0; v < QV; ++v)
+#pragma unroll
+            for (int r = 0; r < RB; ++r)
+              acc[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                  *(const fragv*)(lrow + slot_of(r, v)), ql[v], acc[r], 0, 0, 0);
         }
       }
     }
@@ -558,7 +623,7 @@ __global__ __launch_bounds__(256, (fused_min_blocks<F16, DH>())) void fused_kern
     }
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (LATE) {
-      issue_loads(cur, ncur, t + 2);
+      issue_loads(cur, lcur, ncur, t + 2);
     } else {
       // every wavefront's LDS-direct loads of tile t + 1 have landed, and
       // every wavefront is done with cur
@@ -566,8 +631,8 @@ __global__ __launch_bounds__(256, (fused_min_blocks<F16, DH>())) void fused_kern
     }
   };
   for (int t = 0; t < ntiles; t += 2) {
-    step(tile0, tnorm0, tile1, tnorm1, t);
-    if (t + 1 < ntiles) step(tile1, tnorm1, tile0, tnorm0, t + 1);
+    step(tile0, low0, tnorm0, tile1, low1, tnorm1, t);
+    if (t + 1 < ntiles) step(tile1, low1, tnorm1, tile0, low0, tnorm0, t + 1);
   }
   // LATE: the fetches past the last tile land before the workgroup ends
   if constexpr (LATE) __builtin_amdgcn_s_waitcnt(0);
@@ -1272,6 +1337,7 @@ __global__ __launch_bounds__(256) void merge_wave_kernel(MergeArgs a) {
   }
   const bool l2 = a.metric == kL2;
   const float qn = (l2 && a.dist_mode == 0) ? a.qnorm[q] : 0.0f;
+  const float scale = list_score_scale(a.split);
   // writes rank r as output slot i (id, distance)
   auto emit = [&](int i, uint64_t r) {
     const int64_t o = (int64_t)q * a.k + i;
@@ -1280,7 +1346,7 @@ __global__ __launch_bounds__(256) void merge_wave_kernel(MergeArgs a) {
       if (a.dists) a.dists[o] = (a.dist_mode == 1 || l2) ? INFINITY : -INFINITY;
     } else {
       a.ids[o] = id_of_rank(r);
-      const float sv = score_of_key((uint32_t)(r >> 32));
+      const float sv = score_of_key((uint32_t)(r >> 32)) * scale;
       if (a.dists) {
         if (a.dist_mode == 1) {
           a.dists[o] = -sv;
@@ -1428,7 +1494,8 @@ __global__ __launch_bounds__(256) void merge_kernel(MergeArgs a) {
     if (threadIdx.x == 0) a.flags[q] = s_flag;
   }
   const float qn = (a.metric == kL2 && a.dist_mode == 0) ? a.qnorm[q] : 0.0f;
-  emit_topk<256>(buf, work, a.k, q, a.metric, qn, a.dist_mode, a.ids, a.dists);
+  emit_topk<256>(buf, work, a.k, q, a.metric, qn, a.dist_mode, a.ids, a.dists,
+                 list_score_scale(a.split));
 }
 
 // ---- exhaustive path ------------------------------------------------------------
@@ -1964,6 +2031,57 @@ hipError_t dispatch_t(const FusedArgs& a, hipStream_t s) {
   return hipErrorInvalidValue;
 }
 
+template <int DH, int T>
+hipError_t split_inst(const FusedArgs& a, hipStream_t s) {
+  const dim3 grid(a.nsplit * a.nqb);
+  if constexpr (T == 16) {
+    if (a.allow) {
+      if (a.metric == kL2)
+        hipLaunchKernelGGL((fused_kernel<true, DH, T, true, 0, true, 2>), grid, dim3(256), 0, s, a);
+      else
+        hipLaunchKernelGGL((fused_kernel<true, DH, T, false, 0, true, 2>), grid, dim3(256), 0, s, a);
+      return hipGetLastError();
+    }
+  }
+  if (a.allow) return hipErrorInvalidValue;
+  if (a.metric == kL2)
+    hipLaunchKernelGGL((fused_kernel<true, DH, T, true, 0, false, 2>), grid, dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((fused_kernel<true, DH, T, false, 0, false, 2>), grid, dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+
+template <int DH>
+hipError_t split_t(const FusedArgs& a, hipStream_t s) {
+  switch (a.T) {
+    case 4: return split_inst<DH, 4>(a, s);
+    case 8: return split_inst<DH, 8>(a, s);
+    case 10: return split_inst<DH, 10>(a, s);
+    case 16: return split_inst<DH, 16>(a, s);
+  }
+  return hipErrorInvalidValue;
+}
+
+template <int DH, int T>
+int split_occupancy() {
+  int blocks = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+          &blocks, fused_kernel<true, DH, T, true, 0, false, 2>, 256, 0) != hipSuccess)
+    return 1;
+  return blocks;
+}
+
+template <int DH>
+int split_occupancy_t(int T) {
+  switch (T) {
+    case 4: return split_occupancy<DH, 4>();
+    case 8: return split_occupancy<DH, 8>();
+    case 10: return split_occupancy<DH, 10>();
+    case 16: return split_occupancy<DH, 16>();
+  }
+  return 1;
+}
+
 template <int T>
 int deep_occupancy(bool f16) {
   int blocks = 0;
@@ -2055,6 +2173,20 @@ int fused_blocks_per_cu(int ld, int T, bool f16) {
   return 1;
 }
 
+bool fused_split_supported(int ld, int T) {
+  return t_ok(T) && ld >= 8 && ld % 8 == 0 && ld <= kMaxSplitDim;
+}
+
+int fused_split_blocks_per_cu(int ld, int T) {
+  return ld <= 64 ? split_occupancy_t<32>(T) : split_occupancy_t<64>(T);
+}
+
+hipError_t launch_fused_split(const FusedArgs& a, hipStream_t s) {
+  if (!fused_split_supported(a.ld, a.T) || !a.split || !a.base_lo || !a.queries_lo)
+    return hipErrorInvalidValue;
+  return a.ld <= 64 ? split_t<32>(a, s) : split_t<64>(a, s);
+}
+
 hipError_t launch_norms(const PrepArgs& a, hipStream_t s) {
   if (a.n <= 0) return hipSuccess;
   const dim3 grid((unsigned)((a.n + 255) / 256));
@@ -2071,10 +2203,18 @@ hipError_t launch_norms(const PrepArgs& a, hipStream_t s) {
 }
 
 hipError_t launch_transform(const PrepArgs& a, hipStream_t s) {
-  const int64_t total = a.n * a.out_ld;
-  if (total <= 0) return hipSuccess;
-  hipLaunchKernelGGL(rows_transform_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256),
-                     0, s, a);
+  if (a.n <= 0 || a.out_ld <= 0) return hipSuccess;
+  if (a.out_ld % 4 != 0 || (uintptr_t)a.out % 16 != 0) return hipErrorInvalidValue;
+  const int64_t total = a.n * (a.out_ld / 4);
+  // (a launch that a split call's rows rarely need: few workgroups, which
+  // return at once)
+  const int64_t grid = std::min<int64_t>((total + 255) / 256, a.split ? 2048 : int64_t(1) << 23);
+  if (total + grid * 256 < (int64_t(1) << 32))
+    hipLaunchKernelGGL(rows_transform_kernel<uint32_t>, dim3((unsigned)grid), dim3(256), 0, s, a,
+                       (uint32_t)total);
+  else
+    hipLaunchKernelGGL(rows_transform_kernel<uint64_t>, dim3((unsigned)grid), dim3(256), 0, s, a,
+                       (uint64_t)total);
   return hipGetLastError();
 }
 

@@ -24,6 +24,8 @@ constexpr int kMaxMergeCandidates = 4096;
 // Largest k of the exact selection.
 constexpr int kMaxK = 256;
 
+struct SplitState;
+
 // Row preparation.
 struct PrepArgs {
   const void* x;            // rows [n, ld], first d used; fp32 or binary16
@@ -40,9 +42,80 @@ struct PrepArgs {
                             // scoring kernels read), else |x|^2
   const int* need;          // launch_norms: if set, only the 256-row blocks b with
                             // need[b] != 0 are written
+  const SplitState* split;  // launch_transform: if set, only on the float32 route
 };
 hipError_t launch_norms(const PrepArgs& a, hipStream_t s);
 hipError_t launch_transform(const PrepArgs& a, hipStream_t s);
+
+// Float32 rows as two binary16 pieces: x 2^s = hi + lo, hi the nearest
+// binary16 and lo the nearest to the rest (13 bits at most: lo drops a last
+// bit of 24 at most), so that the products run on the fp16 MFMA, which sums
+// exact products of halves in float32.  One power of two scales all base
+// rows and one all queries (launch_split_init, from a sample); what a call's
+// rows turn out to need is collected on the device in SplitState::flags
+// (launch_split_rows), and every kernel of the call that serves one route
+// returns at once on another's.
+enum SplitFlags : uint32_t {
+  kSplitBaseLow = 1,    // some base row has a nonzero lo piece
+  kSplitQueryLow = 2,   // some query has
+  kSplitBaseLong = 4,   // some base value has more than 16 significant bits
+  kSplitQueryLong = 8,  // some query value has
+  kSplitRows32 = 16,    // the pieces cannot stand for the rows: a value past
+                        // binary16's range or not finite, or a row most of
+                        // whose values lie below its precision
+};
+struct SplitState {
+  uint32_t flags;
+  float sbase, squery;  // 2^s of the base rows and of the queries
+  float inv;            // scores from the pieces times inv are the rows' scores
+};
+// Which kernel a call's rows take: 0 the float32 MFMA, 1 the hi pieces alone
+// (no value has a lo piece: integers, rows that were binary16), 2 both.
+__host__ __device__ inline int split_route(uint32_t flags) {
+  return flags & kSplitRows32 ? 0 : flags & (kSplitBaseLow | kSplitQueryLow) ? 2 : 1;
+}
+// The lo x lo products are at most 2^-24 of a value's product, below half a
+// unit of the float32 sum they would join; they are formed when both sides
+// have lo pieces and one side has short values only (at most 16 bits), whose
+// float32 sums can be exact.
+__host__ __device__ inline bool split_low_low(uint32_t flags) {
+  const uint32_t low = kSplitBaseLow | kSplitQueryLow, lng = kSplitBaseLong | kSplitQueryLong;
+  return (flags & low) == low && (flags & lng) != lng;
+}
+// The factor that takes a call's list scores to the rows' scores.
+__host__ __device__ inline float list_score_scale(const SplitState* st) {
+  return st && split_route(st->flags) != 0 ? st->inv : 1.0f;
+}
+// Sets st: no flags, the scales from a sample of the rows (unit: rows of
+// length at most 1).
+struct SplitInitArgs {
+  const float* base;     // [n, ld], first d used
+  const float* queries;  // [nq, ld]
+  int64_t n, nq;
+  int d, ld;
+  int unit;
+  SplitState* st;
+};
+hipError_t launch_split_init(const SplitInitArgs& a, hipStream_t s);
+// One pass over the rows: squared norms as launch_norms (norm, half_neg), the
+// L2 seeds -|x|^2 / 2 in the scale of the pieces' scores (seed), the pieces
+// (zero past d) and the flags.
+struct SplitRowsArgs {
+  const void* x;            // [n, ld], first d used; fp32 or binary16
+  int64_t n;
+  int d, ld;
+  int f16;
+  const float* unit_norms;  // rows divided by max(sqrt(norm), 1e-30) first (cosine)
+  float* norm;              // [n] or null
+  int half_neg;
+  float* seed;              // [n] or null
+  uint16_t* hi;             // [n, out_ld]
+  uint16_t* lo;             // [n, out_ld]
+  int out_ld;               // a multiple of 8
+  int query;                // the rows are the queries
+  SplitState* st;
+};
+hipError_t launch_split_rows(const SplitRowsArgs& a, hipStream_t s);
 
 // Fused distance + per-lane top-T selection.
 //   grid nsplit * nqb (nqb = ceil(nq / 128)); workgroup 256 threads.
@@ -91,6 +164,12 @@ struct FusedArgs {
   // word-aligned rows of words per query, launch_filter_rows).
   const uint32_t* allow;
   int64_t allow_stride;
+  // Split rows (SplitState): the kernel returns unless the call's rows take
+  // `route`; null: no routes.  launch_fused_split reads the lo pieces too.
+  const SplitState* split;
+  int route;
+  const void* base_lo;
+  const void* queries_lo;
   // Cosine by factors (deep kernel, fp32 rows, metric kCosine): bnorm holds
   // |b|^2 of the rows and qnorm |q|^2 of the queries, and each score is the
   // rows' dot product times 1 / max(|b|, 1e-30) and 1 / max(|q|, 1e-30), the
@@ -99,6 +178,12 @@ struct FusedArgs {
 };
 hipError_t launch_fused_f32(const FusedArgs& a, hipStream_t s);
 hipError_t launch_fused_f16(const FusedArgs& a, hipStream_t s);
+// Both pieces of float32 rows (base / base_lo, queries / queries_lo
+// [.., ld] binary16, ld a multiple of 8 up to kMaxSplitDim).
+constexpr int kMaxSplitDim = 128;
+hipError_t launch_fused_split(const FusedArgs& a, hipStream_t s);
+bool fused_split_supported(int ld, int T);
+int fused_split_blocks_per_cu(int ld, int T);
 // true when the fused kernels have an instance for (ld, T)
 bool fused_supported(int ld, int T, bool f16);
 // resident workgroups per CU of that instance (HIP occupancy query)
@@ -229,6 +314,9 @@ struct MergeArgs {
   // per-list check then uses these instead of the lists' last entries
   const uint64_t* sentinel;
   int sorted;            // 1: each list of T is sorted best first (stream lists)
+  // the lists' scores are split->inv times too large unless the call took
+  // the float32 route (null: they are the scores)
+  const SplitState* split;
 };
 hipError_t launch_merge(const MergeArgs& a, hipStream_t s);
 
@@ -258,6 +346,7 @@ struct BoundMergeArgs {
   int32_t* ids;
   float* dists;
   int* flags;            // [nq] or null (T >= k)
+  const SplitState* split;  // as MergeArgs
 };
 hipError_t launch_bound_merge(const BoundMergeArgs& a, hipStream_t s);
 

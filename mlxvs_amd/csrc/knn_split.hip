@@ -1,0 +1,256 @@
+// Float32 rows as two binary16 pieces (SplitState, knn_kernels.h): the pass
+// that makes them, for the kernels that multiply them on the fp16 MFMA.
+#include <hip/hip_fp16.h>
+#include <hip/hip_runtime.h>
+
+#include "knn_kernels.h"
+
+namespace mlxvs::kern {
+namespace {
+
+typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kSampleThreads = 1024;
+constexpr int kSamplePer = 8;
+// The sample's largest value is scaled to [2^11, 2^12): binary16 ends at
+// 2^16, so values up to 16 times larger still fit, and its spacing below
+// 2^-13 is 2^-24, so a value down to 1/4096 of the largest keeps 24 bits and
+// smaller ones an error of 2^-36 of the largest.
+constexpr int kSampleExp = 11;
+// Unit rows: their values are at most 1 (and a rounding), scaled to 2^15.
+constexpr float kUnitScale = 32768.0f;
+
+// The sample: up to 8,192 values of the base rows and of the queries, 64
+// neighbouring columns of each of 128 rows spread over all of them (the
+// columns by a multiplicative hash).  One workgroup, 16 coalesced loads a lane in
+// flight together (values scattered one by one took it 50 us, not 5).
+__global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArgs a) {
+  __shared__ float wmax[2][kSampleThreads / 64];
+  const int tid = threadIdx.x;
+  float m[2] = {0.0f, 0.0f};
+  if (!a.unit) {
+    float v[2][kSamplePer];
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+      const float* x = side ? a.queries : a.base;
+      const int64_t n = side ? a.nq : a.n;
+#pragma unroll
+      for (int i = 0; i < kSamplePer; ++i) {
+        const uint32_t j = (uint32_t)(i * (kSampleThreads / 64) + (tid >> 6));
+        const int64_t r = (int64_t)j * n / (kSamplePer * kSampleThreads / 64);
+        const uint32_t c = ((j * 2654435761u >> 8) + (tid & 63)) % (uint32_t)a.d;
+        v[side][i] = x[r * a.ld + c];
+      }
+    }
+#pragma unroll
+    for (int side = 0; side < 2; ++side)
+#pragma unroll
+      for (int i = 0; i < kSamplePer; ++i) m[side] = fmaxf(m[side], fabsf(v[side][i]));
+  }
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    m[0] = fmaxf(m[0], __shfl_xor(m[0], o));
+    m[1] = fmaxf(m[1], __shfl_xor(m[1], o));
+  }
+  if ((tid & 63) == 0) {
+    wmax[0][tid >> 6] = m[0];
+    wmax[1][tid >> 6] = m[1];
+  }
+  __syncthreads();
+  if (tid != 0) return;
+  float sc[2];
+  for (int side = 0; side < 2; ++side) {
+    float x = 0.0f;
+    for (int w = 0; w < kSampleThreads / 64; ++w) x = fmaxf(x, wmax[side][w]);
+    // (a sample of zeros, or one past 2^80 either way: any scale will do,
+    // the pass over all rows decides whether it did)
+    int e = 0;
+    const bool usable = x > 0x1p-80f && x < 0x1p80f;
+    if (usable) (void)frexpf(x, &e);  // x = f 2^e, f in [1/2, 1)
+    sc[side] = a.unit ? kUnitScale : usable ? ldexpf(1.0f, kSampleExp + 1 - e) : 1.0f;
+  }
+  a.st->flags = 0;
+  a.st->sbase = sc[0];
+  a.st->squery = sc[1];
+  a.st->inv = 1.0f / (sc[0] * sc[1]);  // powers of two: exact
+}
+
+// 256 rows per workgroup, a 32-value slab at a time through LDS: fetched with
+// coalesced loads (VEC: 16 bytes a lane; else a value a lane), summed row by
+// row in the order of row_norms_kernel (the norms are those), and turned into
+// pieces eight values a thread, 64 contiguous bytes a row and piece.  HBM
+// bound: each row is read once and written once (4 bytes a value both ways).
+template <bool F16, bool VEC>
+__global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs a) {
+  constexpr int SS = 36;  // LDS row stride (floats), as row_norms_kernel
+  __shared__ __align__(16) float sh[256 * SS];
+  const int tid = threadIdx.x;
+  const int64_t row0 = (int64_t)blockIdx.x * 256;
+  const float scale = a.query ? a.st->squery : a.st->sbase;
+  const float seed_scale = a.st->sbase * a.st->squery;
+  float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  constexpr int EPV = F16 ? 8 : 4;
+  constexpr int VPR = 32 / EPV;
+  float pv[VEC ? VPR : 32][VEC ? EPV : 1];
+  auto load_slab = [&](int c0) {
+    if constexpr (VEC) {
+#pragma unroll
+      for (int j = 0; j < VPR; ++j) {
+        const int e = tid + 256 * j;
+        const int r = e / VPR, c = (e % VPR) * EPV;
+        const int64_t row = row0 + r;
+        if (row < a.n && c0 + c < a.d) {
+          if constexpr (F16) {
+            const halfx8 hv = *(const halfx8*)((const _Float16*)a.x + row * a.ld + c0 + c);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) pv[j][u] = (float)hv[u];
+          } else {
+            const floatx4 f = *(const floatx4*)((const float*)a.x + row * a.ld + c0 + c);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) pv[j][u] = f[u];
+          }
+        } else {
+#pragma unroll
+          for (int u = 0; u < EPV; ++u) pv[j][u] = 0.0f;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 32; ++j) {
+        const int e = tid + 256 * j;
+        const int r = e >> 5, c = c0 + (e & 31);
+        const int64_t row = row0 + r;
+        float v = 0.0f;
+        if (row < a.n && c < a.d)
+          v = F16 ? (float)((const _Float16*)a.x)[row * a.ld + c]
+                  : ((const float*)a.x)[row * a.ld + c];
+        pv[j][0] = v;
+      }
+    }
+  };
+  // pieces: thread t converts values 8 (t % 4) .. + 7 of rows t / 4 + 64 j
+  int lossy[4] = {0, 0, 0, 0};
+  uint32_t seen = 0;  // bit 0: a lo piece, 1: a long value, 2: out of range
+  load_slab(0);
+  for (int c0 = 0; c0 < a.out_ld; c0 += 32) {
+    if constexpr (VEC) {
+#pragma unroll
+      for (int j = 0; j < VPR; ++j) {
+        const int e = tid + 256 * j;
+        const int r = e / VPR, c = (e % VPR) * EPV;
+#pragma unroll
+        for (int u = 0; u < EPV; u += 4)
+          *(floatx4*)&sh[r * SS + c + u] = floatx4{pv[j][u], pv[j][u + 1], pv[j][u + 2], pv[j][u + 3]};
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 32; ++j) {
+        const int e = tid + 256 * j;
+        sh[(e >> 5) * SS + (e & 31)] = pv[j][0];
+      }
+    }
+    if (c0 + 32 < a.out_ld) load_slab(c0 + 32);
+    __syncthreads();
+    if (a.norm || a.seed) {
+#pragma unroll
+      for (int j4 = 0; j4 < 32; j4 += 4) {
+        const floatx4 v = *(const floatx4*)&sh[tid * SS + j4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (c0 + j4 + u < a.d) acc[(j4 + u) & 7] += v[u] * v[u];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int r = (tid >> 2) + 64 * j, c = 8 * (tid & 3);
+      const int64_t row = row0 + r;
+      if (row >= a.n || c0 + c >= a.out_ld) continue;
+      float x[8];
+      *(floatx4*)&x[0] = *(const floatx4*)&sh[r * SS + c];
+      *(floatx4*)&x[4] = *(const floatx4*)&sh[r * SS + c + 4];
+      if (a.unit_norms) {
+        const float nrm = sqrtf(a.unit_norms[row]);
+        const float den = nrm > 1e-30f ? nrm : 1e-30f;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = x[u] / den;
+      }
+      halfx8 hi, lo;
+      int lost = 0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float xs = x[u] * scale;
+        const _Float16 hv = (_Float16)xs;
+        const float rest = xs - (float)hv;  // exact
+        const _Float16 lv = (_Float16)rest;
+        hi[u] = hv;
+        lo[u] = lv;
+        const uint16_t lb = __builtin_bit_cast(uint16_t, lv);
+        if (!(fabsf(xs) <= 65504.0f)) seen |= 4u;
+        if (lb & 0x7fffu) seen |= 1u;
+        if ((lb & 0x003fu) && (lb & 0x7c00u)) seen |= 2u;
+        // (rest - lo, exact; a value whose scaling underflowed is lost too)
+        if (fabsf(rest - (float)lv) > fabsf(xs) * 0x1p-23f || (xs == 0.0f && x[u] != 0.0f)) ++lost;
+      }
+      lossy[j] += lost;
+      *(u32x4*)(a.hi + row * a.out_ld + c0 + c) = __builtin_bit_cast(u32x4, hi);
+      *(u32x4*)(a.lo + row * a.out_ld + c0 + c) = __builtin_bit_cast(u32x4, lo);
+    }
+    __syncthreads();
+  }
+  // a row most of whose values the pieces lose bits of (more than an eighth):
+  // its four threads' counts
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    int t = lossy[j];
+    t += __shfl_xor(t, 1);
+    t += __shfl_xor(t, 2);
+    if (8 * t > a.d) seen |= 4u;
+  }
+  if ((a.norm || a.seed) && row0 + tid < a.n) {
+    const float s01 = acc[0] + acc[1], s23 = acc[2] + acc[3];
+    const float s45 = acc[4] + acc[5], s67 = acc[6] + acc[7];
+    const float nn = (s01 + s23) + (s45 + s67);
+    // (squared norms near the ends of float32: their sums are not the
+    // scaled ones)
+    if (!(nn < 0x1p100f) || (nn > 0.0f && nn < 0x1p-100f)) seen |= 4u;
+    const float half = nn > 0.0f ? -0.5f * nn : 0.0f;  // (+0, as row_norms_kernel)
+    if (a.norm) a.norm[row0 + tid] = a.half_neg ? half : nn;
+    if (a.seed) a.seed[row0 + tid] = half * seed_scale;
+  }
+  uint32_t any = (__builtin_amdgcn_ballot_w64(seen & 1u) ? (a.query ? kSplitQueryLow : kSplitBaseLow) : 0u) |
+                 (__builtin_amdgcn_ballot_w64(seen & 2u) ? (a.query ? kSplitQueryLong : kSplitBaseLong) : 0u) |
+                 (__builtin_amdgcn_ballot_w64(seen & 4u) ? kSplitRows32 : 0u);
+  // (read first: thousands of wavefronts would serialise on one word)
+  if ((tid & 63) == 0 && any &&
+      (any & ~__hip_atomic_load(&a.st->flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
+    __hip_atomic_fetch_or(&a.st->flags, any, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+}  // namespace
+
+hipError_t launch_split_init(const SplitInitArgs& a, hipStream_t s) {
+  if (a.n < 1 || a.nq < 1 || a.d < 1) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(split_init_kernel, dim3(1), dim3(kSampleThreads), 0, s, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_split_rows(const SplitRowsArgs& a, hipStream_t s) {
+  if (a.n <= 0) return hipSuccess;
+  if (a.out_ld % 8 != 0 || a.out_ld < a.d) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)((a.n + 255) / 256));
+  const int esize = a.f16 ? 2 : 4;
+  const bool vec = (uintptr_t)a.x % 16 == 0 && ((int64_t)a.ld * esize) % 16 == 0 &&
+                   (a.d * esize) % 16 == 0;
+  if (a.f16) {
+    if (vec) hipLaunchKernelGGL((split_rows_kernel<true, true>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((split_rows_kernel<true, false>), grid, dim3(256), 0, s, a);
+  } else {
+    if (vec) hipLaunchKernelGGL((split_rows_kernel<false, true>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((split_rows_kernel<false, false>), grid, dim3(256), 0, s, a);
+  }
+  return hipGetLastError();
+}
+
+}  // namespace mlxvs::kern

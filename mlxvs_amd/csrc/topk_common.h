@@ -493,9 +493,10 @@ __device__ __forceinline__ int pow2_at_least(int x) {
 }
 
 // emit_topk's writes for k ranks already in the output order (0 = empty).
+// The ranks' scores times `scale` (a power of two) are the rows' scores.
 template <int NT>
 __device__ void emit_ordered(const uint64_t* work, int k, int64_t orow, int metric, float qn,
-                             int dist_mode, int32_t* ids, float* dists) {
+                             int dist_mode, int32_t* ids, float* dists, float scale = 1.0f) {
   const bool l2 = metric == 1;
   for (int i = threadIdx.x; i < k; i += NT) {
     uint64_t r = work[i];
@@ -505,7 +506,7 @@ __device__ void emit_ordered(const uint64_t* work, int k, int64_t orow, int metr
       if (dists) dists[o] = (dist_mode == 1 || l2) ? INFINITY : -INFINITY;
     } else {
       ids[o] = id_of_rank(r);
-      float s = score_of_key((uint32_t)(r >> 32));
+      float s = score_of_key((uint32_t)(r >> 32)) * scale;
       if (dists) {
         if (dist_mode == 1) {
           dists[o] = -s;
@@ -528,12 +529,12 @@ __device__ void emit_ordered(const uint64_t* work, int k, int64_t orow, int metr
 template <int NT>
 __device__ void emit_topk(const uint64_t* best, uint64_t* work, int k,
                           int64_t orow, int metric, float qn, int dist_mode,
-                          int32_t* ids, float* dists) {
+                          int32_t* ids, float* dists, float scale = 1.0f) {
   const int K2 = pow2_at_least(k);
   for (int i = threadIdx.x; i < K2; i += NT) work[i] = i < k ? best[i] : 0;
   __syncthreads();
   bitonic_desc<NT>(work, K2, OutputOrder{});
-  emit_ordered<NT>(work, k, orow, metric, qn, dist_mode, ids, dists);
+  emit_ordered<NT>(work, k, orow, metric, qn, dist_mode, ids, dists, scale);
 }
 
 }  // namespace mlxvs::kern

@@ -1281,7 +1281,8 @@ __global__ __launch_bounds__(256) void bound_merge_kernel(BoundMergeArgs a) {
     if (tid == 0) a.flags[q] = s_flag;
   }
   const float qn = (a.metric == kL2 && a.dist_mode == 0) ? a.qnorm[q] : 0.0f;
-  emit_ordered<NT>(sm.buf, a.k, q, a.metric, qn, a.dist_mode, a.ids, a.dists);
+  emit_ordered<NT>(sm.buf, a.k, q, a.metric, qn, a.dist_mode, a.ids, a.dists,
+                   list_score_scale(a.split));
 }
 
 // ---- exact float scan of a few queries --------------------------------------------

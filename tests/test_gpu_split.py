@@ -1,0 +1,145 @@
+"""Float32 batches on the two-piece fp16 route against the CPU restatement.
+
+Large float32 batches multiply their rows as two binary16 pieces; the rows'
+values decide on the device between the hi pieces alone, both pieces, and
+the float32 kernels.  Every kind of values here must give what the float32
+route gives: integers bit for bit (their sums are exact either way), real
+values to float32 accuracy.
+
+The tolerance on real values: the pieces hold a value to 2^-24 of itself, the
+dropped lo x lo products are below 2^-24 of theirs, and the float32 sums have
+fewer roundings than the float32 kernels' (a multiply-add each: at most d
+2^-24 of the sum of magnitudes), so |error| <= (d + 4) 2^-24 sum |q_i b_i|,
+which Cauchy-Schwarz bounds by |q| |b|; L2 takes it twice and adds its norms'.
+"""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+N, NQ = 66_001, 4_003  # n nq max(d, 32) past the route's least work, ragged tiles and blocks
+SAMPLE = 40            # queries checked: the first, the last and some between
+
+
+def rows_of(kind, n, d, r):
+    if kind == "bytes":        # 8-bit integers: the hi pieces alone
+        return r.integers(0, 256, (n, d)).astype(np.float32)
+    if kind == "halves":       # binary16 values, both signs
+        return r.standard_normal((n, d)).astype(np.float16).astype(np.float32)
+    if kind == "wide ints":    # 12-bit integers with lo pieces on both sides: lo x lo counts
+        x = np.zeros((n, d), np.float32)
+        x[np.arange(n), r.integers(0, min(d, 4), n)] = r.integers(2049, 2800, n)
+        return x
+    x = r.standard_normal((n, d)).astype(np.float32)
+    if kind == "outlier":      # past binary16's range in the sample's scale: the float32 kernels
+        x[n // 2, d // 2] = 3.0e6
+    if kind == "tiny row":     # below the pieces' precision: the float32 kernels
+        x[n // 3] *= np.float32(1e-9)
+    if kind == "small":        # a scale far from 1
+        x *= np.float32(2.0 ** -40)
+    return x
+
+
+def sample(nq):
+    return np.unique(np.concatenate([[0, 1, 127, 128, nq - 1, nq - 2],
+                                     np.linspace(0, nq - 1, SAMPLE).astype(int)]))
+
+
+def check(engine, oracle, base, q, k, metric, exact, **filt):
+    if filt:
+        ids, dist = engine.brute_force_knn_filtered(base, q, k, metric, **filt)
+    else:
+        ids, dist = engine.brute_force_knn(base, q, k, metric)
+    pick = sample(len(q))
+    if filt:
+        oi, od = oracle.knn_filtered(base, q[pick], k, metric, **filt)
+    else:
+        oi, od = oracle.knn(base, q[pick], k, metric)
+    if exact:
+        assert np.array_equal(ids[pick], oi)
+        assert np.array_equal(dist[pick], od)
+        return
+    b64, q64 = base.astype(np.float64), q[pick].astype(np.float64)
+    bn, qn = np.linalg.norm(b64, axis=1), np.linalg.norm(q64, axis=1)
+    u = (base.shape[1] + 4) * 2.0 ** -24
+    for i in range(len(pick)):
+        got, g = ids[pick][i], dist[pick][i].astype(np.float64)
+        s = b64 @ q64[i]
+        mag = qn[i] * bn
+        if metric == "l2":
+            s = ((b64 - q64[i]) ** 2).sum(1)
+            err = u * (qn[i] + bn) ** 2
+        elif metric == "cosine":
+            s, err = s / mag, np.full(len(bn), 2 * u)
+        else:
+            err = u * mag
+        if "bitset" in filt:
+            s = np.where(filt["bitset"], s, np.inf if metric == "l2" else -np.inf)
+        assert len(set(got.tolist())) == k
+        assert (np.abs(g - s[got]) <= err[got]).all(), np.abs(g - s[got]).max()
+        # no row left out is better than the last kept by more than the errors
+        order = s if metric == "l2" else -s
+        left = np.ones(len(s), bool)
+        left[got] = False
+        worst = (order[got] + 2 * err[got]).max()
+        assert ((order + 2 * err)[left] >= worst - 4 * err.max()).all()
+
+
+@pytest.mark.parametrize("kind,metric,d,k,exact", [
+    ("bytes", "l2", 128, 10, True),
+    ("bytes", "l2", 99, 33, True),
+    ("bytes", "inner_product", 64, 4, True),
+    ("halves", "inner_product", 100, 10, False),
+    ("wide ints", "l2", 128, 10, True),
+    ("wide ints", "l2", 20, 8, True),
+    ("float", "l2", 128, 10, False),
+    ("float", "l2", 33, 1, False),
+    ("float", "inner_product", 65, 16, False),
+    ("float", "cosine", 96, 10, False),
+    ("float", "cosine", 27, 40, False),
+    ("float", "l2", 128, 100, False),
+    ("small", "l2", 120, 10, False),
+    ("outlier", "l2", 128, 10, False),
+    ("outlier", "cosine", 128, 20, False),
+    ("tiny row", "inner_product", 99, 10, False),
+    ("tiny row", "l2", 36, 40, False),
+])
+def test_every_kind_of_values(engine, oracle, kind, metric, d, k, exact):
+    r = np.random.default_rng(d + k)
+    base, q = rows_of(kind, N, d, r), rows_of(kind, NQ, d, r)
+    check(engine, oracle, base, q, k, metric, exact)
+
+
+@pytest.mark.parametrize("kind", ["bytes", "float", "outlier"])
+def test_prefilter(engine, oracle, kind):
+    r = np.random.default_rng(7)
+    base, q = rows_of(kind, N, 96, r), rows_of(kind, NQ, 96, r)
+    check(engine, oracle, base, q, 12, "l2", kind == "bytes", bitset=r.random(N) < 0.3)
+
+
+def test_mixed_sides_and_ties(engine, oracle):
+    """Integer rows against real queries (one side has lo pieces), and rows
+    that repeat: the lowest ids come first."""
+    r = np.random.default_rng(3)
+    base = rows_of("bytes", N, 64, r)
+    base[40_000:40_300] = base[100:400]
+    q = rows_of("float", NQ, 64, r) + np.float32(100)
+    check(engine, oracle, base, q, 10, "l2", False)
+    q = base[100:100 + NQ].copy()
+    check(engine, oracle, base, q, 10, "l2", True)
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf])
+def test_infinite_values_take_the_float32_route(engine, oracle, value):
+    r = np.random.default_rng(5)
+    base, q = rows_of("float", N, 64, r), np.abs(rows_of("float", NQ, 64, r))
+    base[123, 5] = value
+    ids, dist = engine.brute_force_knn(base, q, 3, "inner_product")
+    pick = sample(NQ)
+    oi, od = oracle.knn(base, q[pick], 3, "inner_product")
+    assert (ids[pick] == oi).mean() > 0.99
+    if value > 0:
+        assert (ids[:, 0] == 123).all() and np.isposinf(dist[:, 0]).all()
+    else:
+        assert not (ids == 123).any()
