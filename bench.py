@@ -392,10 +392,11 @@ def main() -> int:
         # fused kernels cover all queries in one launch; the exhaustive path
         # splits them over several score launches
         flops = 2.0 * nq * n * d / (cnt / args.steps)
-        # (fused_hi / fused_split multiply float32 rows as binary16 pieces on
-        # the fp16 MFMA: the algorithmic flops against that unit's peak)
+        # (fused_hi, fused_split and fused_tile multiply float32 rows as
+        # binary16 pieces on the fp16 MFMA: the algorithmic flops against that
+        # unit's peak)
         peak = (PEAK_FP16_MFMA if (f16 and kname.startswith("fused"))
-                or kname in ("fused_hi", "fused_split") else PEAK_FP32_MFMA)
+                or kname in ("fused_hi", "fused_split", "fused_tile") else PEAK_FP32_MFMA)
         row_bytes = float(n) * d * base.dtype.itemsize / (cnt / args.steps)
         if flops / row_bytes < peak * 1e12 / (PEAK_HBM * 1e9):
             # below the ridge point: the base rows' bytes bound the kernel

@@ -556,9 +556,36 @@ BoundPlan shared_bound(int k, int T, int slots, int lists) {
 // work of 32 values, so fewer count as 32).
 constexpr int64_t kSplitMinQueries = 256;
 constexpr double kSplitMinWork = 8e9;  // n nq max(d, 32)
+// Longer rows (the tile kernel, a workgroup a CU): 500k x 768, 128 queries 1.11
+// / 1.14 ms, 160 1.82 / 1.24, 700 4.69 / 2.29; 200k x 200, 256 queries 0.317 /
+// 0.301, 1,024 0.96 / 0.50; 20k x 768, 700 queries 0.28 / 0.34.
+constexpr int64_t kTileMinQueries = 129;
+constexpr double kTileMinWork = 1.6e10;  // n nq d
+// Binary16 rows there, against the deep kernel's 128 x 128 tiles: 500k x 768,
+// 300 queries 0.62 / 0.63 ms, 512 0.78 / 0.71, 700 0.99 / 0.86; 500k x 384, 700
+// queries 0.53 / 0.52; 1M x 1536 x 10,000 35.2 / 28.6.
+constexpr int64_t kTileF16MinQueries = 384;
+constexpr double kTileF16MinWork = 1.5e11;  // n nq d
 // Device memory for the pieces and the operands of the float32 route: as
 // much as the rows take, so large collections keep the float32 kernels.
 constexpr size_t kSplitMaxBytes = size_t(16) << 30;
+
+// The deep rows' tile kernel for nq queries: its list length and split plan
+// (not ok: too few rows for k, or rows past its buffer range).
+SplitPlan plan_tile(int64_t n, int64_t nq, int k, int T, int ld, bool pieces) {
+  SplitPlan p;
+  if (!kern::tile_supported(ld, T, pieces) || nq >= (int64_t(1) << 31)) return p;
+  const int64_t qblocks = (nq + kern::kTileQueries - 1) / kern::kTileQueries;
+  p = plan_splits(n, qblocks, k, T, kern::tile_segments(T), kern::kTileKernelRows,
+                  device_slots(kern::tile_blocks_per_cu(T, pieces)), true,
+                  max_merge_segments(k, T));
+  // (the kernel fetches up to two tiles past a split's rows)
+  if (p.ok && (p.rows_per_split + 2 * kern::kTileKernelRows) * ld * (pieces ? 4 : 2) >=
+                  (int64_t(1) << 31))
+    p.ok = false;
+  return p;
+}
+int list_len_tile(int k, bool allow) { return allow || k > 10 ? 16 : 10; }
 
 // Returns false when the route does not apply (nothing was enqueued).
 // `allow`: prefilter words as FusedArgs.
@@ -569,30 +596,49 @@ bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, cons
   const int64_t n = in.n, nq = in.nq;
   const int d = in.d;
   const bool cosine = metric == kern::kCosine, l2 = metric == kern::kL2;
-  if (ar.fixed() || (in.f16 && !cosine) || nq < kSplitMinQueries || nq >= (int64_t(1) << 31) ||
-      (double)n * (double)nq * std::max(d, 32) < kSplitMinWork)
+  // rows longer than two pieces of a query fit in registers: the tile kernel,
+  // on interleaved pieces; the float32 route then runs the fused (up to 256
+  // values) or the deep kernel
+  const bool tile = round_up(d, 8) > kern::kMaxSplitDim;
+  const double work = (double)n * (double)nq * std::max(d, 32);
+  if (ar.fixed() || (in.f16 && !cosine) || nq >= (int64_t(1) << 31) ||
+      nq < (tile ? kTileMinQueries : kSplitMinQueries) ||
+      work < (tile ? kTileMinWork : kSplitMinWork))
     return false;
-  const int T = allow ? 16 : list_len_float(k);
-  const int sld = round_up(d, 8), ld32 = round_up(d, 4);
-  if (!kern::fused_split_supported(sld, T) || !kern::fused_supported(ld32, T, false)) return false;
+  const bool deep32 = d > kern::kMaxFusedDimF32;
+  const int T = tile ? list_len_tile(k, allow != nullptr) : allow ? 16 : list_len_float(k);
+  const int sld = round_up(d, tile ? kern::kTilePieceRun : 8);
+  const int vmul32 = deep32 ? 32 : 4;
+  const int ld32 = round_up(d, vmul32);
+  if (deep32 ? !kern::deep_supported(ld32, T, false) : !kern::fused_supported(ld32, T, false))
+    return false;
   const int64_t qblocks = (nq + kQueriesPerBlock - 1) / kQueriesPerBlock;
-  const int tile_rows = 2 * kern::kTileRows;
-  const SplitPlan plan = plan_splits(n, qblocks, k, T, 2, tile_rows,
-                                     device_slots(kern::fused_split_blocks_per_cu(sld, T)), true,
-                                     max_merge_segments(k, T));
-  if (!plan.ok || (plan.rows_per_split + tile_rows) * sld * 4 >= (int64_t(1) << 31)) return false;
-  // the float32 route's operands: unit rows (cosine), or the rows in place,
-  // or a padded copy
-  const bool in_place = !cosine && (uintptr_t)in.base % 16 == 0 &&
-                        (uintptr_t)in.queries % 16 == 0 && d % 4 == 0;
+  const int lanes = tile ? kern::tile_segments(T) : 2;
+  SplitPlan plan;
+  if (tile) {
+    plan = plan_tile(n, nq, k, T, sld, true);
+  } else if (kern::fused_split_supported(sld, T)) {
+    plan = plan_splits(n, qblocks, k, T, 2, 2 * kern::kTileRows,
+                       device_slots(kern::fused_split_blocks_per_cu(sld, T)), true,
+                       max_merge_segments(k, T));
+  }
+  if (!plan.ok || (plan.rows_per_split + 2 * kern::kTileKernelRows) * std::max(ld32, sld) * 4 >=
+                      (int64_t(1) << 31))
+    return false;
+  // the float32 route's operands: the rows in place, or a padded copy, and
+  // for cosine unit rows, unless the deep kernel scales by the norms
+  const bool cos_factors = cosine && !in.f16 && deep32 && k <= 16 && !allow;
+  const bool in_place = (!cosine || cos_factors) && (uintptr_t)in.base % 16 == 0 &&
+                        (uintptr_t)in.queries % 16 == 0 && d % vmul32 == 0;
   const size_t rows_all = (size_t)(n + nq);
   const size_t bytes = rows_all * ((size_t)sld * 4 + (in_place ? 0 : (size_t)ld32 * 4)) + (64u << 10);
   if (bytes > kSplitMaxBytes || !ar.reserve(bytes)) return false;
 
-  uint16_t* bhi = ar.take<uint16_t>((size_t)n * sld);
-  uint16_t* blo = ar.take<uint16_t>((size_t)n * sld);
-  uint16_t* qhi = ar.take<uint16_t>((size_t)nq * sld);
-  uint16_t* qlo = ar.take<uint16_t>((size_t)nq * sld);
+  // (interleaved pieces: the hi arrays hold both)
+  uint16_t* bhi = ar.take<uint16_t>((size_t)n * sld * (tile ? 2 : 1));
+  uint16_t* blo = tile ? nullptr : ar.take<uint16_t>((size_t)n * sld);
+  uint16_t* qhi = ar.take<uint16_t>((size_t)nq * sld * (tile ? 2 : 1));
+  uint16_t* qlo = tile ? nullptr : ar.take<uint16_t>((size_t)nq * sld);
   auto* st = ar.take<kern::SplitState>(1);
   const int f16 = in.f16 ? 1 : 0;
   const void *kbase = in.base, *kq = in.queries;
@@ -621,8 +667,10 @@ bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, cons
   if (!in_place) {
     float* pb = ar.take<float>((size_t)n * ld32);
     float* pq = ar.take<float>((size_t)nq * ld32);
-    kern::PrepArgs tb{in.base, n, d, d, f16, nullptr, ubn, pb, ld32, 0};
-    kern::PrepArgs tq{in.queries, nq, d, d, f16, nullptr, uqn, pq, ld32, 0};
+    const float* un = cos_factors ? nullptr : ubn;
+    const float* uq = cos_factors ? nullptr : uqn;
+    kern::PrepArgs tb{in.base, n, d, d, f16, nullptr, un, pb, ld32, 0};
+    kern::PrepArgs tq{in.queries, nq, d, d, f16, nullptr, uq, pq, ld32, 0};
     // (the redo of cosine queries reads the unit rows on every route)
     if (!(cosine && k > T)) tb.split = tq.split = st;
     launch(s, "prep", [&] { return kern::launch_transform(tb, s); });
@@ -631,7 +679,7 @@ bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, cons
     kq = pq;
   }
 
-  const int nseg = 2 * plan.nsplit;
+  const int nseg = lanes * plan.nsplit;
   uint64_t* part = ar.take<uint64_t>((size_t)nq * nseg * T);
   const int slots = kern::bound_slots_for(T);
   const BoundPlan bp = shared_bound(k, T, slots, nseg);
@@ -640,22 +688,37 @@ bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, cons
   // one launch per route: all but the one that the rows take return at once
   kern::FusedArgs fa{bhi, qhi, seed, n, (int)nq, sld, cosine ? kern::kInnerProduct : metric,
                      plan.rows_per_split, plan.nsplit, T, k, part, gkey, bp.m, bp.pubj,
-                     (int)qblocks, plan.xcd ? 1 : 0};
+                     (int)qblocks, plan.xcd ? (tile ? 2 : 1) : 0};
   fa.allow = allow;
   fa.allow_stride = allow_stride;
   fa.split = st;
   fa.base_lo = blo;
   fa.queries_lo = qlo;
-  fa.route = 1;
-  launch(s, "fused_hi", [&] { return kern::launch_fused_f16(fa, s); });
-  fa.route = 2;
-  launch(s, "fused_split", [&] { return kern::launch_fused_split(fa, s); });
+  if (tile) {
+    fa.route = 1;  // (both piece routes)
+    fa.nqb = (int)((nq + kern::kTileQueries - 1) / kern::kTileQueries);
+    launch(s, "fused_tile", [&] { return kern::launch_tile(fa, true, s); });
+  } else {
+    fa.route = 1;
+    launch(s, "fused_hi", [&] { return kern::launch_fused_f16(fa, s); });
+    fa.route = 2;
+    launch(s, "fused_split", [&] { return kern::launch_fused_split(fa, s); });
+  }
+  // (its two segments a split: the same lists over finer splits)
   fa.route = 0;
+  fa.nqb = (int)qblocks;
   fa.base = kbase;
   fa.queries = kq;
-  fa.bnorm = bnorm;
+  fa.bnorm = cos_factors ? ubn : bnorm;
+  fa.qnorm = cos_factors ? uqn : nullptr;
+  if (cos_factors) fa.metric = kern::kCosine;
   fa.ld = ld32;
-  launch(s, "fused_f32", [&] { return kern::launch_fused_f32(fa, s); });
+  fa.nsplit = plan.nsplit * (lanes / 2);
+  fa.rows_per_split = plan.rows_per_split / (lanes / 2);
+  if (deep32)
+    launch(s, "fused_deep", [&] { return kern::launch_deep(fa, false, false, s); });
+  else
+    launch(s, "fused_f32", [&] { return kern::launch_fused_f32(fa, s); });
   int* flags = T < k ? ar.take<int>((size_t)nq) : nullptr;
   merge_lists(ar, s, part, nseg, T, k, nq, metric, qnorm, 0, ids, dists, flags, st);
   if (T >= k) return true;
@@ -714,8 +777,16 @@ void float_knn(Session& ss, const FloatInputs& in, int k, int metric, int32_t* i
   // rows longer than the register-resident kernels take go through the
   // deep kernel, which reads them in 128-byte chunks (32 fp32 / 64 fp16 dims)
   const bool deep = d > kern::kMaxFusedDimF32;
+  // binary16 batches: the tile kernel, on rows of whole 64-byte chunks (not in
+  // the no-allocation entry, whose scratch its lists would outgrow)
+  const int tile_T = list_len_tile(k, allow != nullptr);
+  const SplitPlan tplan = deep && kf16 && !ar.fixed() && nq >= kTileF16MinQueries &&
+                                  (double)n * (double)nq * d >= kTileF16MinWork
+                              ? plan_tile(n, nq, k, tile_T, round_up(d, 2 * kern::kTilePieceRun), false)
+                              : SplitPlan{};
+  const bool use_tile = tplan.ok;
   // row padding: whole 16-byte vectors, or whole 128-byte chunks (deep)
-  const int vmul = deep ? (kf16 ? 64 : 32) : (kf16 ? 8 : 4);
+  const int vmul = deep ? (use_tile ? 2 * kern::kTilePieceRun : kf16 ? 64 : 32) : (kf16 ? 8 : 4);
   const void* kbase = in.base;
   const void* kq = in.queries;
   int kld = d;
@@ -800,10 +871,10 @@ void float_knn(Session& ss, const FloatInputs& in, int k, int metric, int32_t* i
     launch(s, "prep", [&] { return kern::launch_norms(pq, s); });
   }
   // lists of 16 with a prefilter (its kernel instances; exact for every k)
-  const int T = allow ? 16 : list_len_float(k);
+  const int T = use_tile ? tile_T : allow ? 16 : list_len_float(k);
   const int64_t qblocks = (nq + kQueriesPerBlock - 1) / kQueriesPerBlock;
-  SplitPlan plan;
-  const bool use_deep = deep && kern::deep_supported(kld, T, kf16);
+  SplitPlan plan = tplan;
+  const bool use_deep = deep && !use_tile && kern::deep_supported(kld, T, kf16);
   // at most 32 queries (fp32): rows streamed straight into registers (not
   // with a prefilter, which the fused and deep kernels apply)
   const bool use_stream = !kf16 && !deep && !allow && kern::stream_supported(kld, T, nq);
@@ -811,12 +882,13 @@ void float_knn(Session& ss, const FloatInputs& in, int k, int metric, int32_t* i
   // row blocks of a tile instead of the queries
   const bool deep_rs = use_deep && nq <= 32;
   // segment lists per split
-  const int lanes = (use_stream || deep_rs) ? 8 : 2;
+  const int lanes = use_tile ? kern::tile_segments(T) : (use_stream || deep_rs) ? 8 : 2;
   // split alignment: whole tiles (deep: 128 rows; fused: 32 or 64; stream:
   // a tile for each of the four wavefronts)
   const int tile_rows = use_deep ? kern::kDeepRows : use_stream ? 4 * kern::kTileRows
                                                                : 2 * kern::kTileRows;
-  if ((use_deep || kern::fused_supported(kld, T, kf16)) && nq < (int64_t(1) << 31)) {
+  if (!use_tile && (use_deep || kern::fused_supported(kld, T, kf16)) &&
+      nq < (int64_t(1) << 31)) {
     const int bpc = use_deep     ? kern::deep_blocks_per_cu(T, kf16)
                     : use_stream ? kern::stream_blocks_per_cu(kld)
                                  : kern::fused_blocks_per_cu(kld, T, kf16);
@@ -881,11 +953,14 @@ void float_knn(Session& ss, const FloatInputs& in, int k, int metric, int32_t* i
   kern::FusedArgs fa{kbase, kq, cos_factors ? cnb : bnorm, n, (int)nq, kld,
                      cos_factors ? kern::kCosine : cosine ? kern::kInnerProduct : metric,
                      plan.rows_per_split, plan.nsplit, T, k, part, gkey, bp.m, bp.pubj,
-                     (int)qblocks, plan.xcd ? (use_deep ? 2 : 1) : 0};
+                     (int)qblocks, plan.xcd ? (use_deep || use_tile ? 2 : 1) : 0};
   fa.allow = allow;
   fa.allow_stride = allow_stride;
   fa.qnorm = cnq;
-  if (use_deep)
+  if (use_tile) fa.nqb = (int)((nq + kern::kTileQueries - 1) / kern::kTileQueries);
+  if (use_tile)
+    launch(s, "fused_tile", [&] { return kern::launch_tile(fa, false, s); });
+  else if (use_deep)
     launch(s, "fused_deep", [&] { return kern::launch_deep(fa, kf16, deep_rs, s); });
   else if (use_stream)
     launch(s, "stream_f32", [&] { return kern::launch_stream(fa, s); });

@@ -109,9 +109,9 @@ struct SplitRowsArgs {
   float* norm;              // [n] or null
   int half_neg;
   float* seed;              // [n] or null
-  uint16_t* hi;             // [n, out_ld]
-  uint16_t* lo;             // [n, out_ld]
-  int out_ld;               // a multiple of 8
+  uint16_t* hi;             // [n, out_ld]; lo null: [n, 2 out_ld], kTilePieceRun hi
+  uint16_t* lo;             // pieces, then their lo pieces, and so on
+  int out_ld;               // a multiple of 8 (lo null: of kTilePieceRun)
   int query;                // the rows are the queries
   SplitState* st;
 };
@@ -209,6 +209,20 @@ constexpr int kDeepRows = 128;
 hipError_t launch_deep(const FusedArgs& a, bool f16, bool row_split, hipStream_t s);
 bool deep_supported(int ld, int T, bool f16);
 int deep_blocks_per_cu(int T, bool f16);
+// Deep rows in larger batches (knn_tile.hip): tiles of kTileKernelRows rows x
+// kTileQueries queries, a K loop over 128-byte chunks; the arguments of the
+// fused kernels (nqb = ceil(nq / kTileQueries)), with tile_segments(T)
+// segments per split (T 10 or 16).  pieces: base / queries are the interleaved
+// pieces of float32 rows (SplitRowsArgs with lo null, ld a multiple of
+// kTilePieceRun), on every route but the float32 one; else binary16 rows, ld a
+// multiple of 2 kTilePieceRun.
+constexpr int kTileKernelRows = 256;
+constexpr int kTileQueries = 256;
+constexpr int kTilePieceRun = 32;  // values in a run of one piece
+hipError_t launch_tile(const FusedArgs& a, bool pieces, hipStream_t s);
+bool tile_supported(int ld, int T, bool pieces);
+int tile_blocks_per_cu(int T, bool pieces);
+int tile_segments(int T);
 // The same arguments, segments and output over bit codes (knn_hamming.hip):
 // base / queries packed little-endian words, ld = packed row length in bytes
 // (bits_row_bytes: 16, 32, 64, 128 or 256, zero padded), bnorm the rows'

@@ -194,8 +194,14 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs a) {
         if (fabsf(rest - (float)lv) > fabsf(xs) * 0x1p-23f || (xs == 0.0f && x[u] != 0.0f)) ++lost;
       }
       lossy[j] += lost;
-      *(u32x4*)(a.hi + row * a.out_ld + c0 + c) = __builtin_bit_cast(u32x4, hi);
-      *(u32x4*)(a.lo + row * a.out_ld + c0 + c) = __builtin_bit_cast(u32x4, lo);
+      // (interleaved: a run of hi pieces, then their lo pieces)
+      constexpr int R = kTilePieceRun;
+      const int cc = c0 + c;
+      uint16_t* dh = a.lo ? a.hi + row * a.out_ld + cc
+                          : a.hi + row * 2 * a.out_ld + cc / R * (2 * R) + cc % R;
+      uint16_t* dl = a.lo ? a.lo + row * a.out_ld + cc : dh + R;
+      *(u32x4*)dh = __builtin_bit_cast(u32x4, hi);
+      *(u32x4*)dl = __builtin_bit_cast(u32x4, lo);
     }
     __syncthreads();
   }
@@ -238,7 +244,7 @@ hipError_t launch_split_init(const SplitInitArgs& a, hipStream_t s) {
 
 hipError_t launch_split_rows(const SplitRowsArgs& a, hipStream_t s) {
   if (a.n <= 0) return hipSuccess;
-  if (a.out_ld % 8 != 0 || a.out_ld < a.d) return hipErrorInvalidValue;
+  if (a.out_ld % (a.lo ? 8 : kTilePieceRun) != 0 || a.out_ld < a.d) return hipErrorInvalidValue;
   const dim3 grid((unsigned)((a.n + 255) / 256));
   const int esize = a.f16 ? 2 : 4;
   const bool vec = (uintptr_t)a.x % 16 == 0 && ((int64_t)a.ld * esize) % 16 == 0 &&

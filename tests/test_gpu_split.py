@@ -22,6 +22,11 @@ N, NQ = 66_001, 4_003  # n nq max(d, 32) past the route's least work, ragged til
 SAMPLE = 40            # queries checked: the first, the last and some between
 
 
+def size_of(d):
+    """Fewer rows and queries for long rows (the same matrix work)."""
+    return (N, NQ) if d <= 256 else (30_011, 2_003)
+
+
 def rows_of(kind, n, d, r):
     if kind == "bytes":        # 8-bit integers: the hi pieces alone
         return r.integers(0, 256, (n, d)).astype(np.float32)
@@ -41,17 +46,20 @@ def rows_of(kind, n, d, r):
     return x
 
 
-def sample(nq):
-    return np.unique(np.concatenate([[0, 1, 127, 128, nq - 1, nq - 2],
-                                     np.linspace(0, nq - 1, SAMPLE).astype(int)]))
+def sample(nq, count=SAMPLE):
+    edges = np.array([0, 1, 31, 32, 63, 64, 127, 128, nq - 1, nq - 2])
+    return np.unique(np.concatenate([edges[edges < nq],
+                                     np.linspace(0, nq - 1, count).astype(int)]))
 
 
-def check(engine, oracle, base, q, k, metric, exact, **filt):
+def check(engine, oracle, base, q, k, metric, exact, count=SAMPLE, **filt):
     if filt:
         ids, dist = engine.brute_force_knn_filtered(base, q, k, metric, **filt)
     else:
         ids, dist = engine.brute_force_knn(base, q, k, metric)
-    pick = sample(len(q))
+    pick = sample(len(q), count)
+    if base.dtype == np.float16:
+        base, q = oracle.f16_to_f32(base), oracle.f16_to_f32(q)
     if filt:
         oi, od = oracle.knn_filtered(base, q[pick], k, metric, **filt)
     else:
@@ -60,15 +68,18 @@ def check(engine, oracle, base, q, k, metric, exact, **filt):
         assert np.array_equal(ids[pick], oi)
         assert np.array_equal(dist[pick], od)
         return
-    b64, q64 = base.astype(np.float64), q[pick].astype(np.float64)
-    bn, qn = np.linalg.norm(b64, axis=1), np.linalg.norm(q64, axis=1)
+    q64 = q[pick].astype(np.float64)
+    bn = np.sqrt(np.einsum("ij,ij->i", base, base, dtype=np.float64))
+    qn = np.linalg.norm(q64, axis=1)
+    dots = np.concatenate([base[i:i + 20_000].astype(np.float64) @ q64.T
+                           for i in range(0, len(base), 20_000)])
     u = (base.shape[1] + 4) * 2.0 ** -24
     for i in range(len(pick)):
         got, g = ids[pick][i], dist[pick][i].astype(np.float64)
-        s = b64 @ q64[i]
+        s = dots[:, i]
         mag = qn[i] * bn
         if metric == "l2":
-            s = ((b64 - q64[i]) ** 2).sum(1)
+            s = bn * bn + qn[i] * qn[i] - 2 * s
             err = u * (qn[i] + bn) ** 2
         elif metric == "cosine":
             s, err = s / mag, np.full(len(bn), 2 * u)
@@ -104,18 +115,59 @@ def check(engine, oracle, base, q, k, metric, exact, **filt):
     ("outlier", "cosine", 128, 20, False),
     ("tiny row", "inner_product", 99, 10, False),
     ("tiny row", "l2", 36, 40, False),
+    # the tile kernel: rows too long to hold a query's pieces in registers
+    ("bytes", "l2", 130, 10, True),
+    ("bytes", "inner_product", 200, 16, True),
+    ("wide ints", "l2", 137, 10, True),
+    ("wide ints", "l2", 300, 33, True),
+    ("float", "l2", 129, 10, False),
+    ("float", "inner_product", 256, 3, False),
+    ("float", "cosine", 255, 40, False),
+    ("float", "l2", 257, 40, False),
+    ("float", "cosine", 384, 10, False),
+    ("float", "cosine", 301, 40, False),
+    ("float", "l2", 768, 16, False),
+    ("outlier", "l2", 144, 10, False),
+    ("outlier", "l2", 320, 16, False),
+    ("outlier", "cosine", 384, 10, False),
+    ("outlier", "cosine", 299, 10, False),
+    ("outlier", "cosine", 299, 40, False),
+    ("tiny row", "inner_product", 290, 40, False),
 ])
 def test_every_kind_of_values(engine, oracle, kind, metric, d, k, exact):
     r = np.random.default_rng(d + k)
-    base, q = rows_of(kind, N, d, r), rows_of(kind, NQ, d, r)
+    n, nq = size_of(d)
+    base, q = rows_of(kind, n, d, r), rows_of(kind, nq, d, r)
     check(engine, oracle, base, q, k, metric, exact)
 
 
-@pytest.mark.parametrize("kind", ["bytes", "float", "outlier"])
-def test_prefilter(engine, oracle, kind):
+@pytest.mark.parametrize("kind,d", [("bytes", 96), ("float", 96), ("outlier", 96),
+                                    ("bytes", 131), ("float", 272), ("outlier", 272)])
+def test_prefilter(engine, oracle, kind, d):
     r = np.random.default_rng(7)
-    base, q = rows_of(kind, N, 96, r), rows_of(kind, NQ, 96, r)
-    check(engine, oracle, base, q, 12, "l2", kind == "bytes", bitset=r.random(N) < 0.3)
+    n, nq = size_of(d)
+    base, q = rows_of(kind, n, d, r), rows_of(kind, nq, d, r)
+    check(engine, oracle, base, q, 12, "l2", kind == "bytes", bitset=r.random(n) < 0.3)
+
+
+@pytest.mark.parametrize("n,nq,d,k,metric", [
+    (200_003, 513, 1536, 10, "inner_product"), (300_001, 2_003, 257, 10, "l2"),
+    (150_037, 1_281, 800, 16, "inner_product"), (260_011, 1_500, 400, 40, "l2"),
+    (2_999, 60_000, 860, 10, "l2"),
+])
+def test_binary16_deep_batches(engine, oracle, n, nq, d, k, metric):
+    """The tile kernel on binary16 rows: its edges in rows, queries and dims."""
+    r = np.random.default_rng(n + d)
+    base = r.standard_normal((n, d), dtype=np.float32).astype(np.float16)
+    q = r.standard_normal((nq, d), dtype=np.float32).astype(np.float16)
+    check(engine, oracle, base, q, k, metric, False, count=8)
+
+
+def test_binary16_deep_prefilter(engine, oracle):
+    r = np.random.default_rng(8)
+    base = r.standard_normal((240_001, 320), dtype=np.float32).astype(np.float16)
+    q = r.standard_normal((2_001, 320), dtype=np.float32).astype(np.float16)
+    check(engine, oracle, base, q, 20, "l2", False, count=8, bitset=r.random(len(base)) < 0.4)
 
 
 def test_mixed_sides_and_ties(engine, oracle):
