@@ -1621,20 +1621,34 @@ void brute_force_knn_filtered_device(const Rows& base, const Rows& queries, int 
 }
 
 namespace {
-// Rows of at most 128 columns: the split-parallel scan over rows zero-padded
-// to 32, 64 or 128 columns (each split's exact best k), then the rank merge
-// of each query's lists; wider rows (whose scan would spill registers): a
-// query per workgroup over all rows (launch_pairwise).
+// Rows of at most 128 columns: for batches a query per lane
+// (launch_pairwise_lanes) and the stream-list merges; else the split-parallel
+// scan over rows zero-padded to 32, 64 or 128 columns (each split's exact best
+// k), then the rank merge of each query's lists.  Wider rows (whose scan would
+// spill registers): a query per workgroup over all rows (launch_pairwise).
+constexpr int64_t kLanesMinQueries = 64;
 void pairwise_search(Session& ss, kern::PairwiseArgs pa) {
   Arena& ar = ss.arena();
   hipStream_t s = ss.stream();
   const int d = pa.d;
-  const int ld = d <= 32 ? 32 : d <= 64 ? 64 : d <= 128 ? 128 : 0;
+  const int64_t n = pa.n, nq = pa.nq;
+  const int T = pa.k <= 10 ? 10 : 16;
+  const int lld = round_up(d, 32);
+  SplitPlan lanes;
+  if (nq >= kLanesMinQueries && nq < (int64_t(1) << 31) &&
+      kern::pairwise_lanes_supported(pa.metric, lld)) {
+    // workgroups of up to four groups of 64 queries, two a CU
+    const int64_t groups = (nq + 63) / 64, waves = std::min<int64_t>(4, groups);
+    lanes = plan_splits(n, (groups + waves - 1) / waves, pa.k, T, 1, 1,
+                        device_slots((int)(8 / waves)), false, max_merge_segments(pa.k, T));
+    if (lanes.ok && (lanes.rows_per_split + 8) * lld * 4 >= (int64_t(1) << 31)) lanes.ok = false;
+  }
+  const int ld = lanes.ok ? lld : d <= 32 ? 32 : d <= 64 ? 64 : d <= 128 ? 128 : 0;
   if (ld == 0) {
     launch(s, "pairwise", [&] { return kern::launch_pairwise(pa, s); });
     return;
   }
-  const int64_t n = pa.n, nq = pa.nq;
+  const kern::PairwiseArgs unpadded = pa;
   if (ld != d || (uintptr_t)pa.base % 16 != 0 || (uintptr_t)pa.queries % 16 != 0) {
     float* pb = ar.take<float>((size_t)n * ld);
     float* pq = ar.take<float>((size_t)nq * ld);
@@ -1644,6 +1658,31 @@ void pairwise_search(Session& ss, kern::PairwiseArgs pa) {
     launch(s, "prep", [&] { return kern::launch_transform(tq, s); });
     pa.base = pb;
     pa.queries = pq;
+  }
+  if (lanes.ok) {
+    pa.ld = ld;
+    pa.rows_per_split = lanes.rows_per_split;
+    pa.nsplit = lanes.nsplit;
+    pa.part = ar.take<uint64_t>((size_t)nq * lanes.nsplit * T);
+    const int slots = kern::bound_slots_for(T);
+    // (short splits end before a shared bound pays for its reads and atomics:
+    // 100k x 128, 200 queries in 512 splits 0.47 ms with it)
+    const BoundPlan bp = lanes.rows_per_split < 384 ? BoundPlan{}
+                                                    : shared_bound(pa.k, T, slots, lanes.nsplit);
+    pa.gkey = ar.take<uint32_t>((size_t)nq * slots);
+    pa.mslots = bp.m;
+    pa.pubj = bp.pubj;
+    launch(s, "prep", [&] { return kern::launch_bounds_init(pa.gkey, nq, slots, bp.m, s); });
+    launch(s, "pairwise", [&] { return kern::launch_pairwise_lanes(pa, T, s); });
+    int* flags = T < pa.k ? ar.take<int>((size_t)nq) : nullptr;
+    merge_lists(ar, s, pa.part, lanes.nsplit, T, pa.k, nq, kern::kInnerProduct, nullptr, 1, pa.ids,
+                pa.dists, flags);
+    if (flags) {
+      kern::PairwiseArgs redo = unpadded;
+      redo.flags = flags;
+      launch(s, "redo", [&] { return kern::launch_pairwise(redo, s); });
+    }
+    return;
   }
   // about four workgroups per CU slot in all, splits of whole 4,096-row
   // chunks when there are enough rows

@@ -591,8 +591,20 @@ struct PairwiseArgs {
   int64_t rows_per_split;
   int nsplit;               // a multiple of 8
   uint64_t* part;           // [nq][nsplit][k] out
+  // launch_pairwise: only the queries with flags[q] != 0 (null: all)
+  const int* flags;
+  // launch_pairwise_lanes: shared bounds (FusedArgs), slots of list length T
+  uint32_t* gkey;
+  int mslots;
+  int pubj;
 };
 hipError_t launch_pairwise(const PairwiseArgs& a, hipStream_t s);
+// Batches (a query per lane, knn_pairwise.hip): rows and queries [.][ld]
+// fp32, 16-byte aligned, zero past d, ld 32, 64, 96 or 128; stream lists of T
+// (10 or 16) ranks of -distance per split into part [nq][nsplit][T], for the
+// stream-list merges (k > T: with their flags, redone by launch_pairwise).
+hipError_t launch_pairwise_lanes(const PairwiseArgs& a, int T, hipStream_t s);
+bool pairwise_lanes_supported(int metric, int ld);
 // The same distances for rows of at most 128 columns, split-parallel:
 // workgroup (split, query) scores its split's rows -- eight lanes a row,
 // 16-byte loads, the lanes' partial sums met by DPP moves -- and selects

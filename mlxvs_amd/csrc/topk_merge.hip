@@ -937,6 +937,7 @@ __global__ __launch_bounds__(256) void pairwise_knn_kernel(PairwiseArgs a) {
   sc.inv_p = a.inv_p;
   sc.qs = sc.qss = 0.0f;
   for (int64_t q = blockIdx.x; q < a.nq; q += gridDim.x) {
+    if (a.flags && !a.flags[q]) continue;
     sc.query = a.queries + q * a.d;
     sc.allow = a.allow ? a.allow + q * a.allow_stride : nullptr;
     if constexpr (MET == kPwCorrelation) {

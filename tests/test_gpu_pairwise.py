@@ -136,3 +136,42 @@ def test_pairwise_wide_rows_float(engine, oracle, metric):
     tol = 2e-4 if metric in ("minkowski", "jensenshannon", "kl_divergence") else 1e-4
     ids, dist = engine.pairwise_knn(b, q, 10, metric, p)
     recall_check(oracle, ids, dist, b, q, 10, metric, p, tol)
+
+
+@pytest.mark.parametrize("metric", ["cityblock", "chebyshev", "hamming", "russellrao"])
+@pytest.mark.parametrize("nq,d,k", [(64, 5, 1), (65, 32, 10), (257, 33, 11), (300, 96, 16),
+                                    (130, 100, 40), (64, 128, 256)])
+def test_pairwise_batches_integer_bit_exact(engine, oracle, metric, nq, d, k):
+    # 64 queries and more: a query per lane (widths padded to 32, 64, 96 or
+    # 128), lists of 10 and 16, k past the lists; ties go to the lowest id
+    rng = np.random.default_rng(nq + d)
+    hi = 2 if metric == "russellrao" else 5
+    b = rng.integers(0, hi, (7_003, d)).astype(np.float32)
+    q = rng.integers(0, hi, (nq, d)).astype(np.float32)
+    ids, dist = engine.pairwise_knn(b, q, k, metric)
+    oid, odist = oracle.pairwise_knn(q, b, k, metric)
+    assert np.array_equal(ids, oid)
+    assert np.array_equal(dist, odist.astype(np.float32))
+
+
+@pytest.mark.parametrize("metric", ["correlation", "hellinger", "braycurtis"])
+def test_pairwise_batches_float(engine, oracle, metric):
+    b, q = data_for(metric, 5_000, 150, 77, 3)
+    ids, dist = engine.pairwise_knn(b, q, 12, metric)
+    recall_check(oracle, ids, dist, b, q, 12, metric)
+
+
+def test_pairwise_batches_neighbours_side_by_side(engine, oracle):
+    # a query's 60 nearest rows lie next to each other: more than a list of a
+    # split holds, so the query is flagged and redone over all rows
+    rng = np.random.default_rng(4)
+    b = (rng.random((40_000, 16)) * 100 + 50).astype(np.float32)
+    q = np.zeros((70, 16), np.float32)
+    for i in range(70):
+        q[i] = 10 * i
+        b[500 * i:500 * i + 60] = q[i] + rng.random((60, 16)).astype(np.float32)
+    ids, dist = engine.pairwise_knn(b, q, 60, "cityblock")
+    recall_check(oracle, ids, dist, b, q, 60, "cityblock")
+    bm = rng.random((70, 40_000)) < 0.3
+    ids, dist = engine.pairwise_knn(b, q, 10, "cityblock", bitmap=bm)
+    recall_check(oracle, ids, dist, b, q, 10, "cityblock", allowed=bm)
