@@ -652,8 +652,7 @@ bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, cons
     uqn = ar.take<float>((size_t)nq);
     kern::PrepArgs pb{in.base, n, d, d, f16, ubn, nullptr, nullptr, 0, 0};
     kern::PrepArgs pq{in.queries, nq, d, d, f16, uqn, nullptr, nullptr, 0, 0};
-    launch(s, "prep", [&] { return kern::launch_norms(pb, s); });
-    launch(s, "prep", [&] { return kern::launch_norms(pq, s); });
+    launch(s, "prep", [&] { return kern::launch_norms_pair(pb, pq, {}, s); });
   }
   if (l2) {
     bnorm = ar.take<float>((size_t)n);
@@ -662,8 +661,12 @@ bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, cons
   }
   kern::SplitRowsArgs sb{in.base, n, d, d, f16, ubn, bnorm, 1, seed, bhi, blo, sld, 0, st};
   kern::SplitRowsArgs sq{in.queries, nq, d, d, f16, uqn, qnorm, 0, nullptr, qhi, qlo, sld, 1, st};
-  launch(s, "prep", [&] { return kern::launch_split_rows(sb, s); });
-  launch(s, "prep", [&] { return kern::launch_split_rows(sq, s); });
+  const int nseg = lanes * plan.nsplit;
+  const int slots = kern::bound_slots_for(T);
+  const BoundPlan bp = shared_bound(k, T, slots, nseg);
+  uint32_t* gkey = ar.take<uint32_t>((size_t)nq * slots);
+  const kern::BoundsInit bi{gkey, nq * slots, slots, bp.m};
+  launch(s, "prep", [&] { return kern::launch_split_rows(sb, sq, bi, s); });
   if (!in_place) {
     float* pb = ar.take<float>((size_t)n * ld32);
     float* pq = ar.take<float>((size_t)nq * ld32);
@@ -679,12 +682,7 @@ bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, cons
     kq = pq;
   }
 
-  const int nseg = lanes * plan.nsplit;
   uint64_t* part = ar.take<uint64_t>((size_t)nq * nseg * T);
-  const int slots = kern::bound_slots_for(T);
-  const BoundPlan bp = shared_bound(k, T, slots, nseg);
-  uint32_t* gkey = ar.take<uint32_t>((size_t)nq * slots);
-  launch(s, "prep", [&] { return kern::launch_bounds_init(gkey, nq, slots, bp.m, s); });
   // one launch per route: all but the one that the rows take return at once
   kern::FusedArgs fa{bhi, qhi, seed, n, (int)nq, sld, cosine ? kern::kInnerProduct : metric,
                      plan.rows_per_split, plan.nsplit, T, k, part, gkey, bp.m, bp.pubj,
@@ -808,8 +806,7 @@ void float_knn(Session& ss, const FloatInputs& in, int k, int metric, int32_t* i
     float* uq = ar.take<float>((size_t)nq * kld);
     kern::PrepArgs pb{in.base, n, d, d, f16, nb, nullptr, nullptr, 0, 0};
     kern::PrepArgs pq{in.queries, nq, d, d, f16, nqv, nullptr, nullptr, 0, 0};
-    launch(s, "prep", [&] { return kern::launch_norms(pb, s); });
-    launch(s, "prep", [&] { return kern::launch_norms(pq, s); });
+    launch(s, "prep", [&] { return kern::launch_norms_pair(pb, pq, {}, s); });
     kern::PrepArgs tb{in.base, n, d, d, f16, nullptr, nb, ub, kld, 0};
     kern::PrepArgs tq{in.queries, nq, d, d, f16, nullptr, nqv, uq, kld, 0};
     launch(s, "prep", [&] { return kern::launch_transform(tb, s); });
@@ -817,21 +814,14 @@ void float_knn(Session& ss, const FloatInputs& in, int k, int metric, int32_t* i
     kbase = ub;
     kq = uq;
   } else {
+    // (the norms are launched once the kernel is chosen, with its bounds)
     if (cos_factors) {
       cnb = ar.take<float>((size_t)n);
       cnq = ar.take<float>((size_t)nq);
-      kern::PrepArgs pb{in.base, n, d, d, f16, cnb, nullptr, nullptr, 0, 0};
-      kern::PrepArgs pq{in.queries, nq, d, d, f16, cnq, nullptr, nullptr, 0, 0};
-      launch(s, "prep", [&] { return kern::launch_norms(pb, s); });
-      launch(s, "prep", [&] { return kern::launch_norms(pq, s); });
     }
     if (l2 && !use_scan) {
-      // the base norms are launched once the kernel is chosen (the streamed
-      // small-batch scan sums them itself)
       bnorm = ar.take<float>((size_t)n);
       qnorm = ar.take<float>((size_t)nq);
-      kern::PrepArgs pq{in.queries, nq, d, d, f16, qnorm, nullptr, nullptr, 0, 0};
-      launch(s, "prep", [&] { return kern::launch_norms(pq, s); });
     }
     const bool aligned = ((uintptr_t)in.base % 16 == 0) && ((uintptr_t)in.queries % 16 == 0);
     if (!aligned || d % vmul != 0) {
@@ -867,8 +857,6 @@ void float_knn(Session& ss, const FloatInputs& in, int k, int metric, int32_t* i
     // (not taken after all: the norms the other kernels read)
     bnorm = ar.take<float>((size_t)n);
     qnorm = ar.take<float>((size_t)nq);
-    kern::PrepArgs pq{in.queries, nq, d, d, f16, qnorm, nullptr, nullptr, 0, 0};
-    launch(s, "prep", [&] { return kern::launch_norms(pq, s); });
   }
   // lists of 16 with a prefilter (its kernel instances; exact for every k)
   const int T = use_tile ? tile_T : allow ? 16 : list_len_float(k);
@@ -901,9 +889,20 @@ void float_knn(Session& ss, const FloatInputs& in, int k, int metric, int32_t* i
       plan.ok = false;
   }
 
-  if (l2 && !(use_stream && plan.ok)) {
-    kern::PrepArgs pb{in.base, n, d, d, f16, bnorm, nullptr, nullptr, 0, 0, 1};
-    launch(s, "prep", [&] { return kern::launch_norms(pb, s); });
+  // the norms -- the streamed small-batch scan sums the rows' itself -- and
+  // the shared bounds
+  const int nseg = lanes * plan.nsplit;
+  const int slots = kern::bound_slots_for(T);
+  const BoundPlan bp = deep_rs || !plan.ok ? BoundPlan{} : shared_bound(k, T, slots, nseg);
+  uint32_t* gkey = plan.ok ? ar.take<uint32_t>((size_t)nq * slots) : nullptr;
+  {
+    kern::PrepArgs pb{in.base, l2 || cos_factors ? n : 0, d, d, f16, l2 ? bnorm : cnb, nullptr,
+                      nullptr, 0, 0, l2 ? 1 : 0};
+    kern::PrepArgs pq{in.queries, l2 || cos_factors ? nq : 0, d, d, f16, l2 ? qnorm : cnq, nullptr,
+                      nullptr, 0, 0};
+    if (use_stream && plan.ok) pb.n = 0;
+    const kern::BoundsInit bi{bp.m > 0 ? gkey : nullptr, nq * slots, slots, bp.m};
+    launch(s, "prep", [&] { return kern::launch_norms_pair(pb, pq, bi, s); });
   }
 
   // fp32 rows for the exhaustive path (only when it runs)
@@ -942,12 +941,7 @@ void float_knn(Session& ss, const FloatInputs& in, int k, int metric, int32_t* i
     return;
   }
 
-  const int nseg = lanes * plan.nsplit;
   uint64_t* part = ar.take<uint64_t>((size_t)nq * nseg * T);
-  const int slots = kern::bound_slots_for(T);
-  const BoundPlan bp = deep_rs ? BoundPlan{} : shared_bound(k, T, slots, nseg);
-  uint32_t* gkey = ar.take<uint32_t>((size_t)nq * slots);
-  launch(s, "prep", [&] { return kern::launch_bounds_init(gkey, nq, slots, bp.m, s); });
   // XCD order: the register-resident kernels share only the row tiles
   // (split-major); the deep kernel streams query chunks too (split-minor)
   kern::FusedArgs fa{kbase, kq, cos_factors ? cnb : bnorm, n, (int)nq, kld,

@@ -55,13 +55,22 @@ __device__ __forceinline__ float load_elem(const void* x, int f16, int64_t i) {
 // restatement's.  VEC: 16-byte aligned rows whose length is a multiple of 16
 // bytes, fetched with coalesced 16-byte loads (8 threads per 128-byte fp32
 // row slab); otherwise element loads.
+// One launch for two row sets and the shared bounds: workgroups [0, na) take
+// a's rows, [na, na + nb) b's, the rest the bounds.
 template <bool F16, bool VEC>
-__global__ __launch_bounds__(256) void row_norms_kernel(PrepArgs a) {
+__global__ __launch_bounds__(256) void row_norms_kernel(PrepArgs aa, PrepArgs ab, BoundsInit bi,
+                                                        uint32_t na, uint32_t nb) {
   constexpr int SS = 36;  // LDS row stride (floats): 16-byte rows, 8 rows hit distinct bank quads
   __shared__ __align__(16) float sh[256 * SS];
-  if (a.need && !a.need[blockIdx.x]) return;
+  if (blockIdx.x >= na + nb) {
+    init_bounds(bi, blockIdx.x - na - nb);
+    return;
+  }
+  const PrepArgs& a = blockIdx.x < na ? aa : ab;
+  const uint32_t blk = blockIdx.x < na ? blockIdx.x : blockIdx.x - na;
+  if (a.need && !a.need[blk]) return;
   const int tid = threadIdx.x;
-  const int64_t row0 = (int64_t)blockIdx.x * 256;
+  const int64_t row0 = (int64_t)blk * 256;
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   // VEC: the next slab's vectors are loaded into registers before the
   // current slab is summed, so its memory latency overlaps that work
@@ -1571,10 +1580,7 @@ __global__ __launch_bounds__(256) void select_kernel(SelectArgs a) {
   emit_topk<256>(sel, work, a.k, orow, a.metric, qn, a.dist_mode, a.ids, a.dists);
 }
 
-__global__ void bounds_init_kernel(uint32_t* p, int64_t count, int S, int m) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < count) p[i] = (int)(i % S) < m ? 0u : 0xffffffffu;
-}
+__global__ void bounds_init_kernel(BoundsInit bi) { init_bounds(bi, blockIdx.x); }
 
 // IVF-Flat candidate scores for any ld (the VALU route for rows longer
 // than the fused kernel takes): one workgroup per item, one (query, row)
@@ -2144,19 +2150,30 @@ hipError_t launch_fused_split(const FusedArgs& a, hipStream_t s) {
   return a.ld <= 64 ? split_t<32>(a, s) : split_t<64>(a, s);
 }
 
-hipError_t launch_norms(const PrepArgs& a, hipStream_t s) {
-  if (a.n <= 0) return hipSuccess;
-  const dim3 grid((unsigned)((a.n + 255) / 256));
-  const int esize = a.f16 ? 2 : 4;
-  const bool vec = (uintptr_t)a.x % 16 == 0 && ((int64_t)a.ld * esize) % 16 == 0;
-  if (a.f16) {
-    if (vec) hipLaunchKernelGGL((row_norms_kernel<true, true>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((row_norms_kernel<true, false>), grid, dim3(256), 0, s, a);
+hipError_t launch_norms_pair(const PrepArgs& a, const PrepArgs& b, const BoundsInit& bi,
+                             hipStream_t s) {
+  const unsigned na = (unsigned)((std::max<int64_t>(a.n, 0) + 255) / 256);
+  const unsigned nb = (unsigned)((std::max<int64_t>(b.n, 0) + 255) / 256);
+  const dim3 grid(na + nb + bounds_blocks(bi));
+  if (grid.x == 0) return hipSuccess;
+  if (na && nb && a.f16 != b.f16) return hipErrorInvalidValue;
+  const int f16 = na ? a.f16 : b.f16;
+  auto vec_ok = [](const PrepArgs& x) {
+    return x.n <= 0 || ((uintptr_t)x.x % 16 == 0 && ((int64_t)x.ld * (x.f16 ? 2 : 4)) % 16 == 0);
+  };
+  const bool vec = vec_ok(a) && vec_ok(b);
+  if (f16) {
+    if (vec) hipLaunchKernelGGL((row_norms_kernel<true, true>), grid, dim3(256), 0, s, a, b, bi, na, nb);
+    else hipLaunchKernelGGL((row_norms_kernel<true, false>), grid, dim3(256), 0, s, a, b, bi, na, nb);
   } else {
-    if (vec) hipLaunchKernelGGL((row_norms_kernel<false, true>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((row_norms_kernel<false, false>), grid, dim3(256), 0, s, a);
+    if (vec) hipLaunchKernelGGL((row_norms_kernel<false, true>), grid, dim3(256), 0, s, a, b, bi, na, nb);
+    else hipLaunchKernelGGL((row_norms_kernel<false, false>), grid, dim3(256), 0, s, a, b, bi, na, nb);
   }
   return hipGetLastError();
+}
+
+hipError_t launch_norms(const PrepArgs& a, hipStream_t s) {
+  return launch_norms_pair(a, PrepArgs{}, BoundsInit{}, s);
 }
 
 hipError_t launch_transform(const PrepArgs& a, hipStream_t s) {
@@ -2408,8 +2425,8 @@ int bound_slots_for(int T) {
 hipError_t launch_bounds_init(uint32_t* gkey, int64_t nq, int S, int m, hipStream_t s) {
   const int64_t count = nq * S;
   if (count <= 0) return hipSuccess;
-  hipLaunchKernelGGL(bounds_init_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0,
-                     s, gkey, count, S, m);
+  const BoundsInit bi{gkey, count, S, m};
+  hipLaunchKernelGGL(bounds_init_kernel, dim3(bounds_blocks(bi)), dim3(256), 0, s, bi);
   return hipGetLastError();
 }
 

@@ -46,6 +46,17 @@ struct PrepArgs {
 };
 hipError_t launch_norms(const PrepArgs& a, hipStream_t s);
 hipError_t launch_transform(const PrepArgs& a, hipStream_t s);
+// Shared per-query bounds at their initial state (launch_bounds_init), as a
+// part of another preparation launch: p null: none.
+struct BoundsInit {
+  uint32_t* p;
+  int64_t count;  // words: queries x slots
+  int S, m;       // slots a query, slots in use
+};
+// launch_norms of two row sets (b.n 0: of one) and the bounds in one launch:
+// a small call is a chain of short kernels, and each costs about 5 us.
+hipError_t launch_norms_pair(const PrepArgs& a, const PrepArgs& b, const BoundsInit& bi,
+                             hipStream_t s);
 
 // Float32 rows as two binary16 pieces: x 2^s = hi + lo, hi the nearest
 // binary16 and lo the nearest to the rest (13 bits at most: lo drops a last
@@ -115,7 +126,10 @@ struct SplitRowsArgs {
   int query;                // the rows are the queries
   SplitState* st;
 };
-hipError_t launch_split_rows(const SplitRowsArgs& a, hipStream_t s);
+// (the base rows, the queries and the bounds in one launch, as
+// launch_norms_pair)
+hipError_t launch_split_rows(const SplitRowsArgs& base, const SplitRowsArgs& queries,
+                             const BoundsInit& bi, hipStream_t s);
 
 // Fused distance + per-lane top-T selection.
 //   grid nsplit * nqb (nqb = ceil(nq / 128)); workgroup 256 threads.

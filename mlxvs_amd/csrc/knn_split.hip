@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include "knn_kernels.h"
+#include "topk_common.h"
 
 namespace mlxvs::kern {
 namespace {
@@ -82,12 +83,20 @@ __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArg
 // row in the order of row_norms_kernel (the norms are those), and turned into
 // pieces eight values a thread, 64 contiguous bytes a row and piece.  HBM
 // bound: each row is read once and written once (4 bytes a value both ways).
+// Workgroups [0, na) take the base rows, [na, na + nb) the queries, the rest
+// the shared bounds.
 template <bool F16, bool VEC>
-__global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs a) {
+__global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, SplitRowsArgs aq,
+                                                         BoundsInit bi, uint32_t na, uint32_t nb) {
   constexpr int SS = 36;  // LDS row stride (floats), as row_norms_kernel
   __shared__ __align__(16) float sh[256 * SS];
+  if (blockIdx.x >= na + nb) {
+    init_bounds(bi, blockIdx.x - na - nb);
+    return;
+  }
+  const SplitRowsArgs& a = blockIdx.x < na ? ab : aq;
   const int tid = threadIdx.x;
-  const int64_t row0 = (int64_t)blockIdx.x * 256;
+  const int64_t row0 = (int64_t)(blockIdx.x < na ? blockIdx.x : blockIdx.x - na) * 256;
   const float scale = a.query ? a.st->squery : a.st->sbase;
   const float seed_scale = a.st->sbase * a.st->squery;
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -242,19 +251,24 @@ hipError_t launch_split_init(const SplitInitArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_split_rows(const SplitRowsArgs& a, hipStream_t s) {
-  if (a.n <= 0) return hipSuccess;
-  if (a.out_ld % (a.lo ? 8 : kTilePieceRun) != 0 || a.out_ld < a.d) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)((a.n + 255) / 256));
-  const int esize = a.f16 ? 2 : 4;
-  const bool vec = (uintptr_t)a.x % 16 == 0 && ((int64_t)a.ld * esize) % 16 == 0 &&
-                   (a.d * esize) % 16 == 0;
-  if (a.f16) {
-    if (vec) hipLaunchKernelGGL((split_rows_kernel<true, true>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((split_rows_kernel<true, false>), grid, dim3(256), 0, s, a);
+hipError_t launch_split_rows(const SplitRowsArgs& base, const SplitRowsArgs& queries,
+                             const BoundsInit& bi, hipStream_t s) {
+  if (base.n < 1 || queries.n < 1 || base.f16 != queries.f16) return hipErrorInvalidValue;
+  bool vec = true;
+  for (const SplitRowsArgs* a : {&base, &queries}) {
+    if (a->out_ld % (a->lo ? 8 : kTilePieceRun) != 0 || a->out_ld < a->d) return hipErrorInvalidValue;
+    const int esize = a->f16 ? 2 : 4;
+    vec = vec && (uintptr_t)a->x % 16 == 0 && ((int64_t)a->ld * esize) % 16 == 0 &&
+          (a->d * esize) % 16 == 0;
+  }
+  const unsigned na = (unsigned)((base.n + 255) / 256), nb = (unsigned)((queries.n + 255) / 256);
+  const dim3 grid(na + nb + bounds_blocks(bi));
+  if (base.f16) {
+    if (vec) hipLaunchKernelGGL((split_rows_kernel<true, true>), grid, dim3(256), 0, s, base, queries, bi, na, nb);
+    else hipLaunchKernelGGL((split_rows_kernel<true, false>), grid, dim3(256), 0, s, base, queries, bi, na, nb);
   } else {
-    if (vec) hipLaunchKernelGGL((split_rows_kernel<false, true>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((split_rows_kernel<false, false>), grid, dim3(256), 0, s, a);
+    if (vec) hipLaunchKernelGGL((split_rows_kernel<false, true>), grid, dim3(256), 0, s, base, queries, bi, na, nb);
+    else hipLaunchKernelGGL((split_rows_kernel<false, false>), grid, dim3(256), 0, s, base, queries, bi, na, nb);
   }
   return hipGetLastError();
 }

@@ -12,6 +12,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "knn_kernels.h"
+
 namespace mlxvs::kern {
 
 // One count per lane with `on` into the LDS histogram hist[dig].  The
@@ -417,6 +419,19 @@ __device__ __forceinline__ void tile_of_workgroup(int id, int nsplit, int nqb, i
 // every few tiles.
 template <int T>
 constexpr int bound_slots() { return 8; }
+
+// The slots' initial state, 1,024 words a workgroup: zero in the m in use,
+// all ones in the others.
+constexpr int kBoundsPerBlock = 1024;
+__device__ __forceinline__ void init_bounds(const BoundsInit& b, uint32_t blk) {
+  for (int i = threadIdx.x; i < kBoundsPerBlock; i += 256) {
+    const int64_t j = (int64_t)blk * kBoundsPerBlock + i;
+    if (j < b.count) b.p[j] = (int)(j % b.S) < b.m ? 0u : 0xffffffffu;
+  }
+}
+inline unsigned bounds_blocks(const BoundsInit& b) {
+  return b.p ? (unsigned)((b.count + kBoundsPerBlock - 1) / kBoundsPerBlock) : 0u;
+}
 
 template <int S>
 struct SharedBound {
