@@ -714,7 +714,7 @@ bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, cons
   fa.nsplit = plan.nsplit * (lanes / 2);
   fa.rows_per_split = plan.rows_per_split / (lanes / 2);
   if (deep32)
-    launch(s, "fused_deep", [&] { return kern::launch_deep(fa, false, false, s); });
+    launch(s, "fused_deep", [&] { return kern::launch_deep(fa, false, s); });
   else
     launch(s, "fused_f32", [&] { return kern::launch_fused_f32(fa, s); });
   int* flags = T < k ? ar.take<int>((size_t)nq) : nullptr;
@@ -889,8 +889,8 @@ void float_knn(Session& ss, const FloatInputs& in, int k, int metric, int32_t* i
       plan.ok = false;
   }
 
-  // the norms -- the streamed small-batch scan sums the rows' itself -- and
-  // the shared bounds
+  // the norms -- the small-batch kernels sum the rows' themselves -- and the
+  // shared bounds
   const int nseg = lanes * plan.nsplit;
   const int slots = kern::bound_slots_for(T);
   const BoundPlan bp = deep_rs || !plan.ok ? BoundPlan{} : shared_bound(k, T, slots, nseg);
@@ -900,7 +900,7 @@ void float_knn(Session& ss, const FloatInputs& in, int k, int metric, int32_t* i
                       nullptr, 0, 0, l2 ? 1 : 0};
     kern::PrepArgs pq{in.queries, l2 || cos_factors ? nq : 0, d, d, f16, l2 ? qnorm : cnq, nullptr,
                       nullptr, 0, 0};
-    if (use_stream && plan.ok) pb.n = 0;
+    if ((use_stream || deep_rs) && plan.ok) pb.n = 0;
     const kern::BoundsInit bi{bp.m > 0 ? gkey : nullptr, nq * slots, slots, bp.m};
     launch(s, "prep", [&] { return kern::launch_norms_pair(pb, pq, bi, s); });
   }
@@ -951,11 +951,14 @@ void float_knn(Session& ss, const FloatInputs& in, int k, int metric, int32_t* i
   fa.allow = allow;
   fa.allow_stride = allow_stride;
   fa.qnorm = cnq;
+  if (deep_rs && T < k) fa.norm_out = bnorm;  // (the redo reads them)
   if (use_tile) fa.nqb = (int)((nq + kern::kTileQueries - 1) / kern::kTileQueries);
   if (use_tile)
     launch(s, "fused_tile", [&] { return kern::launch_tile(fa, false, s); });
   else if (use_deep)
-    launch(s, "fused_deep", [&] { return kern::launch_deep(fa, kf16, deep_rs, s); });
+    launch(s, "fused_deep", [&] {
+      return deep_rs ? kern::launch_deep_rs(fa, kf16, s) : kern::launch_deep(fa, kf16, s);
+    });
   else if (use_stream)
     launch(s, "stream_f32", [&] { return kern::launch_stream(fa, s); });
   else

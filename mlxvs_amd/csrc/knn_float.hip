@@ -628,13 +628,6 @@ __global__ __launch_bounds__(256, (fused_min_blocks<F16, DH>())) void fused_kern
 // ld >= 512 it is a few percent of the tile.  Lane (h, col) of row block rb
 // holds rows 32 rb + 8 (i / 4) + 4 h + i % 4: tile position bit 2 is h, so
 // the segments are those of fused_kernel (2 split + h).
-//
-// RS (row split, at most 32 queries): the four wavefronts take the four row
-// blocks of each tile against the same 32 queries, instead of all four
-// blocks against their own 32, so a small batch does a quarter of the MFMA
-// work per row and streams the rows at HBM speed.  Wavefront w's lanes then
-// hold rows 32 w + 8 (i / 4) + 4 h + i % 4: segments 8 split + 2 w + h
-// (part [nq][8 nsplit][T]), no shared bound.
 
 constexpr int kDeepChunkBytes = 128;           // bytes of a row per LDS stage (8 vectors)
 constexpr int kDeepChunkDwords = kDeepChunkBytes / 4;
@@ -648,7 +641,7 @@ constexpr int kDeepRB = kDeepRows / 32;        // MFMA row blocks per wavefront
 // FILT: with a prefilter (FusedArgs::allow), lists of 16.  COS: cosine by
 // factors (FusedArgs::qnorm), the tile's norm slots hold the rows' inverse
 // norms.
-template <int T, bool L2, bool F16, bool RS, bool FILT = false, bool COS = false>
+template <int T, bool L2, bool F16, bool FILT = false, bool COS = false>
 __global__ __launch_bounds__(256, 2) void deep_kernel(FusedArgs a) {
   if (!F16 && a.split && split_route(a.split->flags) != a.route) return;
   constexpr int esize = F16 ? 2 : 4;
@@ -672,14 +665,12 @@ __global__ __launch_bounds__(256, 2) void deep_kernel(FusedArgs a) {
     tile_of_workgroup(id, a.nsplit, a.nqb, a.xcd_major, split, qb);
   }
   const int qb0 = qb * kQueriesPerBlock;
-  // the wavefront's queries (its block of 32, or the block's first 32)
-  const int qw = RS ? 0 : wave * 32;
+  // the wavefront's queries
+  const int qw = wave * 32;
   const int q = qb0 + qw + col;
   const bool wave_on = qb0 + qw < a.nq;
   const bool qvalid = q < a.nq;
-  // row blocks of a tile per wavefront, and the first
-  constexpr int NB = RS ? 1 : kDeepRB;
-  const int rb0 = RS ? wave : 0;
+  constexpr int NB = kDeepRB;  // row blocks of a tile
   const int ld = a.ld;
   const int NC = ld / CH;
 
@@ -766,7 +757,7 @@ __global__ __launch_bounds__(256, 2) void deep_kernel(FusedArgs a) {
   const bool share = a.mslots > 0;
   uint32_t* gk = a.gkey + (int64_t)(qvalid ? q : 0) * S;
   // the lane's segment
-  const int seg = RS ? 8 * split + 2 * wave + h : 2 * split + h;
+  const int seg = 2 * split + h;
   const int myslot = share ? seg % a.mslots : 0;
   // Prefilter: the lane's query's filter words (word j: global rows 32 j ..
   // 32 j + 31; the split's first row is a multiple of 128)
@@ -805,7 +796,7 @@ __global__ __launch_bounds__(256, 2) void deep_kernel(FusedArgs a) {
       if constexpr (filt) {
 #pragma unroll
         for (int r = 0; r < NB; ++r) {
-          const int64_t rr = r0 + (int64_t)t * kDeepRows + 32 * (rb0 + r);
+          const int64_t rr = r0 + (int64_t)t * kDeepRows + 32 * r;
           if (qvalid && rr < r1) fwd[r] = fw[rr >> 5];
         }
       }
@@ -818,7 +809,7 @@ __global__ __launch_bounds__(256, 2) void deep_kernel(FusedArgs a) {
       // the lane's vectors of its rows at their swizzled slots (rows col +
       // 32 r share the swizzle of col)
       const uint32_t* qrow = cQ + (qw + col) * kDeepChunkDwords;
-      const uint32_t* arow = cA + (32 * rb0 + col) * kDeepChunkDwords;
+      const uint32_t* arow = cA + col * kDeepChunkDwords;
       const int sw = (col & 7) ^ ((col >> 3) & 1);
       // the fragments of vector step v + 1 are read before the MFMAs of
       // step v (a scheduling barrier keeps them there), so each step's
@@ -866,11 +857,11 @@ __global__ __launch_bounds__(256, 2) void deep_kernel(FusedArgs a) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             if constexpr (COS) {
-              const floatx4 hn = *(const floatx4*)&tnorm[t & 1][32 * (rb0 + r) + 8 * j + 4 * h];
+              const floatx4 hn = *(const floatx4*)&tnorm[t & 1][32 * r + 8 * j + 4 * h];
 #pragma unroll
               for (int u = 0; u < 4; ++u) sc[4 * j + u] = (acc[r][4 * j + u] * hn[u]) * qinv;
             } else if constexpr (L2) {
-              const floatx4 hn = *(const floatx4*)&tnorm[t & 1][32 * (rb0 + r) + 8 * j + 4 * h];
+              const floatx4 hn = *(const floatx4*)&tnorm[t & 1][32 * r + 8 * j + 4 * h];
 #pragma unroll
               for (int u = 0; u < 4; ++u) sc[4 * j + u] = acc[r][4 * j + u] + hn[u];
             } else {
@@ -878,8 +869,8 @@ __global__ __launch_bounds__(256, 2) void deep_kernel(FusedArgs a) {
               for (int u = 0; u < 4; ++u) sc[4 * j + u] = acc[r][4 * j + u];
             }
           }
-          inserted |= select_block<T, L2>(K, I, thr, sc, h, id0 + 32 * (rb0 + r),
-                                          lim0 - 32 * (rb0 + r),
+          inserted |= select_block<T, L2>(K, I, thr, sc, h, id0 + 32 * r,
+                                          lim0 - 32 * r,
                                           filt ? allowed_positions(fwd[r], h) : 0xffffffffu);
         }
         if (share && qvalid && inserted) {
@@ -909,7 +900,7 @@ __global__ __launch_bounds__(256, 2) void deep_kernel(FusedArgs a) {
   }
 
   if (qvalid) {
-    uint64_t* dst = a.part + ((int64_t)q * ((RS ? 8 : 2) * a.nsplit) + seg) * T;
+    uint64_t* dst = a.part + ((int64_t)q * (2 * a.nsplit) + seg) * T;
 #pragma unroll
     for (int i = 0; i < T; ++i) dst[i] = stream_rank(K[i], I[i]);
   }
@@ -2049,23 +2040,23 @@ template <int T>
 int deep_occupancy(bool f16) {
   int blocks = 0;
   const hipError_t e =
-      f16 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, deep_kernel<T, true, true, false>,
+      f16 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, deep_kernel<T, true, true>,
                                                          256, 0)
-          : hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, deep_kernel<T, true, false, false>,
+          : hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, deep_kernel<T, true, false>,
                                                          256, 0);
   return e == hipSuccess && blocks > 0 ? blocks : 1;
 }
 
-template <int T, bool F16, bool RS>
+template <int T, bool F16>
 hipError_t deep_inst(const FusedArgs& a, hipStream_t s) {
   const dim3 grid(a.nsplit * a.nqb);
   if constexpr (T == 16) {
     // a prefilter: its own instances (lists of 16 only)
     if (a.allow) {
       if (a.metric == kL2)
-        hipLaunchKernelGGL((deep_kernel<T, true, F16, RS, true>), grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((deep_kernel<T, true, F16, true>), grid, dim3(256), 0, s, a);
       else
-        hipLaunchKernelGGL((deep_kernel<T, false, F16, RS, true>), grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((deep_kernel<T, false, F16, true>), grid, dim3(256), 0, s, a);
       return hipGetLastError();
     }
   }
@@ -2076,21 +2067,20 @@ hipError_t deep_inst(const FusedArgs& a, hipStream_t s) {
       return hipErrorInvalidValue;
     } else {
       if (!a.bnorm || !a.qnorm) return hipErrorInvalidValue;
-      hipLaunchKernelGGL((deep_kernel<T, false, F16, RS, false, true>), grid, dim3(256), 0, s, a);
+      hipLaunchKernelGGL((deep_kernel<T, false, F16, false, true>), grid, dim3(256), 0, s, a);
       return hipGetLastError();
     }
   }
   if (a.metric == kL2)
-    hipLaunchKernelGGL((deep_kernel<T, true, F16, RS>), grid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL((deep_kernel<T, true, F16>), grid, dim3(256), 0, s, a);
   else
-    hipLaunchKernelGGL((deep_kernel<T, false, F16, RS>), grid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL((deep_kernel<T, false, F16>), grid, dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
 template <int T>
-hipError_t deep_t(const FusedArgs& a, bool f16, bool rs, hipStream_t s) {
-  if (f16) return rs ? deep_inst<T, true, true>(a, s) : deep_inst<T, true, false>(a, s);
-  return rs ? deep_inst<T, false, true>(a, s) : deep_inst<T, false, false>(a, s);
+hipError_t deep_t(const FusedArgs& a, bool f16, hipStream_t s) {
+  return f16 ? deep_inst<T, true>(a, s) : deep_inst<T, false>(a, s);
 }
 
 }  // namespace
@@ -2109,15 +2099,13 @@ int deep_blocks_per_cu(int T, bool f16) {
   return 1;
 }
 
-hipError_t launch_deep(const FusedArgs& a, bool f16, bool row_split, hipStream_t s) {
+hipError_t launch_deep(const FusedArgs& a, bool f16, hipStream_t s) {
   if (!deep_supported(a.ld, a.T, f16)) return hipErrorInvalidValue;
-  // row split: one block of at most 32 queries, no shared bound
-  if (row_split && (a.nq > 32 || a.nqb != 1 || a.mslots != 0)) return hipErrorInvalidValue;
   switch (a.T) {
-    case 4: return deep_t<4>(a, f16, row_split, s);
-    case 8: return deep_t<8>(a, f16, row_split, s);
-    case 10: return deep_t<10>(a, f16, row_split, s);
-    case 16: return deep_t<16>(a, f16, row_split, s);
+    case 4: return deep_t<4>(a, f16, s);
+    case 8: return deep_t<8>(a, f16, s);
+    case 10: return deep_t<10>(a, f16, s);
+    case 16: return deep_t<16>(a, f16, s);
   }
   return hipErrorInvalidValue;
 }

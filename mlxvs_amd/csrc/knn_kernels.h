@@ -189,6 +189,7 @@ struct FusedArgs {
   // rows' dot product times 1 / max(|b|, 1e-30) and 1 / max(|q|, 1e-30), the
   // factors the reference's unit rows divide by (src/knn.cpp:30-33)
   const float* qnorm;
+  float* norm_out;  // launch_deep_rs, L2: [n] -|b|^2 / 2 of the rows, or null
 };
 hipError_t launch_fused_f32(const FusedArgs& a, hipStream_t s);
 hipError_t launch_fused_f16(const FusedArgs& a, hipStream_t s);
@@ -217,10 +218,11 @@ int stream_blocks_per_cu(int ld);
 // fused kernels, with kDeepRows rows per tile and a K loop over 128-byte
 // chunks of the rows (32 or 64 dims) staged in LDS.
 constexpr int kDeepRows = 128;
-// row_split: at most 32 queries (nqb 1, mslots 0); the four wavefronts take
-// the four row blocks of each tile, segments 8 split + 2 w + h (part
-// [nq][8 nsplit][T]).
-hipError_t launch_deep(const FusedArgs& a, bool f16, bool row_split, hipStream_t s);
+hipError_t launch_deep(const FusedArgs& a, bool f16, hipStream_t s);
+// At most 32 queries (nqb 1, mslots 0; knn_deep_rs.hip): the four wavefronts
+// take the four row blocks of each tile, segments 8 split + 2 w + h (part
+// [nq][8 nsplit][T]).  The kernel sums the rows' norms itself (bnorm unused).
+hipError_t launch_deep_rs(const FusedArgs& a, bool f16, hipStream_t s);
 bool deep_supported(int ld, int T, bool f16);
 int deep_blocks_per_cu(int T, bool f16);
 // Deep rows in larger batches (knn_tile.hip): tiles of kTileKernelRows rows x

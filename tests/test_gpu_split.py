@@ -195,3 +195,22 @@ def test_infinite_values_take_the_float32_route(engine, oracle, value):
         assert (ids[:, 0] == 123).all() and np.isposinf(dist[:, 0]).all()
     else:
         assert not (ids == 123).any()
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("n,nq,d,k,metric", [
+    (130, 5, 320, 10, "l2"), (20_003, 32, 257, 10, "cosine"), (5_001, 1, 1536, 16, "l2"),
+    (9_999, 31, 500, 60, "l2"), (127, 8, 300, 3, "inner_product"), (12_345, 17, 640, 10, "cosine"),
+])
+def test_deep_rows_few_queries(engine, oracle, f16, n, nq, d, k, metric):
+    """The row-split kernel: norms summed beside the products, partial tiles, a
+    redo (k past the lists) that reads the norms it wrote, a zero row."""
+    r = np.random.default_rng(n + d)
+    base = r.standard_normal((n, d)).astype(np.float16 if f16 else np.float32)
+    q = r.standard_normal((nq, d)).astype(base.dtype)
+    base[n // 2] = 0
+    if k > 16:  # more neighbours side by side than a list holds
+        base[64:64 + k] = q[0] + (r.standard_normal((k, d)) * 0.1).astype(base.dtype)
+    if metric == "cosine":
+        base[n // 2] = base[n // 2 - 1]  # (the bound divides by the row's norm)
+    check(engine, oracle, base, q, k, metric, False)
