@@ -357,14 +357,15 @@ def main() -> int:
         tbytes = (float(nq) * n * 4 + nq * k * 8) / (cnt / args.steps)
         roof = {"bound": "hbm", "achieved": round(tbytes / per / 1e9, 1), "peak": PEAK_HBM,
                 "unit": "GB/s"}
-    elif w["kind"] == "ivf" and kname == "ivf_scan":
+    elif w["kind"] == "ivf" and kname in ("ivf_scan", "ivf_scan_hi", "ivf_scan_split"):
         # 2 d flops per (query, candidate row) of the probed lists
         c, data, ind, off = w["index"]
         probes = mlxvs_amd.kmeans_predict(q, c, w["n_probes"])
         cands = float(np.diff(off)[probes].sum())
         flops = 2.0 * d * cands / (cnt / args.steps)
         roof = {"bound": "mfma", "achieved": round(flops / per / 1e12, 2),
-                "peak": PEAK_FP32_MFMA, "unit": "TFLOP/s", "candidates_per_query": round(cands / nq, 1)}
+                "peak": PEAK_FP32_MFMA if kname == "ivf_scan" else PEAK_FP16_MFMA,
+                "unit": "TFLOP/s", "candidates_per_query": round(cands / nq, 1)}
     elif w["kind"] == "hamming" and kname == "scan_bits":
         # a few queries: the codes read once (the queries of a split share
         # the rows in L2)

@@ -1209,6 +1209,8 @@ V* to_device(Arena& ar, hipStream_t s, const std::vector<V>& v) {
   return p;
 }
 
+constexpr double kIvfSplitUses = 48;
+
 // One search on device pointers.  `off` is the host copy of the offsets
 // when the caller has one (the host-array entry), else null: the work is
 // then planned from the device offsets alone, and the call enqueues it
@@ -1328,7 +1330,17 @@ void ivf_search(Session& ss, const float* centers, int64_t lists, const float* d
     kern::IvfPlanArgs pa{probes, nq, P, offsets, order, (int)lists, cnt, pos,
                          dslots, ditems, dpairs, nitems, need, nblk};
     launch(s, "ivf_plan", [&] { return kern::launch_ivf_plan(pa, s); });
-    base_norms(need);
+    // rows scanned often enough that their binary16 pieces (SplitState) pay
+    // for themselves: 1M x 128 integer (real) rows, 1,024 lists, 20 probes,
+    // float32 against pieces: 10,000 queries 1.02 / 0.67 (0.77) ms a call,
+    // 5,000 0.77 / 0.62 (0.69); 2,500 would not gain
+    const int sld = round_up(d, 8);
+    const size_t piece_bytes = (size_t)(n + nq) * sld * 4 + (64u << 10);
+    const bool split = !ar.fixed() && n > 0 && kern::fused_split_supported(sld, T) &&
+                       npairs >= kIvfSplitUses * (double)lists &&
+                       npairs * (double)avg_rows * std::max(d, 32) >= kSplitMinWork &&
+                       piece_bytes <= kSplitMaxBytes && ar.reserve(piece_bytes);
+    if (!split) base_norms(need);
     const int nseg = 2 * P * rs;
     // every (query, probe) pair is in one item, so every segment is written
     uint64_t* part = ar.take<uint64_t>((size_t)nq * nseg * T);
@@ -1337,13 +1349,43 @@ void ivf_search(Session& ss, const float* centers, int64_t lists, const float* d
     // more slots costs more than the tighter bound saves
     const BoundPlan bp = shared_bound(k, T, 1, nseg);
     uint32_t* gkey = ar.take<uint32_t>((size_t)nq * slots_n);
-    launch(s, "prep", [&] { return kern::launch_bounds_init(gkey, nq, slots_n, bp.m, s); });
     kern::FusedArgs fa{kd, kq, bnorm, n, (int)nq, ld, km, 0, rs, T, k, part, gkey, bp.m, bp.pubj,
                        0, 0, ditems, dpairs, offsets, dslots, P, (int)max_items, nullptr, 0, 0,
                        nitems};
+    kern::SplitState* st = nullptr;
+    if (split) {
+      st = ar.take<kern::SplitState>(1);
+      uint16_t* bhi = ar.take<uint16_t>((size_t)n * sld);
+      uint16_t* blo = ar.take<uint16_t>((size_t)n * sld);
+      uint16_t* qhi = ar.take<uint16_t>((size_t)nq * sld);
+      uint16_t* qlo = ar.take<uint16_t>((size_t)nq * sld);
+      float* seed = l2 ? ar.take<float>((size_t)n) : nullptr;
+      const kern::SplitInitArgs si{kd, kq, n, nq, ld, ld, 0, st};
+      launch(s, "prep", [&] { return kern::launch_split_init(si, s); });
+      const kern::SplitRowsArgs sb{kd, n, ld, ld, 0, nullptr, bnorm, 1, seed, bhi, blo, sld, 0, st};
+      const kern::SplitRowsArgs sq{kq, nq, ld, ld, 0, nullptr, nullptr, 0, nullptr, qhi, qlo, sld,
+                                   1, st};
+      const kern::BoundsInit bi{gkey, nq * slots_n, slots_n, bp.m};
+      launch(s, "prep", [&] { return kern::launch_split_rows(sb, sq, bi, s); });
+      kern::FusedArgs fp = fa;
+      fp.base = bhi;
+      fp.queries = qhi;
+      fp.base_lo = blo;
+      fp.queries_lo = qlo;
+      fp.bnorm = seed;
+      fp.ld = sld;
+      fp.split = st;
+      for (fp.route = 1; fp.route <= 2; ++fp.route)
+        launch(s, fp.route == 1 ? "ivf_scan_hi" : "ivf_scan_split",
+               [&] { return kern::launch_ivf_select_pieces(fp, s); });
+      fa.split = st;
+      fa.route = 0;
+    } else {
+      launch(s, "prep", [&] { return kern::launch_bounds_init(gkey, nq, slots_n, bp.m, s); });
+    }
     launch(s, "ivf_scan", [&] { return kern::launch_ivf_select(fa, s); });
     int* flags = k > T ? ar.take<int>((size_t)nq) : nullptr;
-    merge_lists(ar, s, part, nseg, T, k, nq, metric, qnorm, 0, ids, dists, flags);
+    merge_lists(ar, s, part, nseg, T, k, nq, metric, qnorm, 0, ids, dists, flags, st);
     if (flags) {
       // the flagged queries again, over their probed lists' rows (columns out)
       kern::RedoArgs ra{kd, kq, l2 ? bnorm : nullptr, qnorm, flags, lists, (int)nq, ld, ld, 0, 0,

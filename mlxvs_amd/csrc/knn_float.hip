@@ -224,9 +224,9 @@ constexpr int fused_rb() {
 // values instead of one per value.
 template <bool F16, int DH, int T, bool L2, int MODE = 0, bool FILT = false, int NP = 1>
 __global__ __launch_bounds__(256, (fused_min_blocks<F16, DH>())) void fused_kernel(FusedArgs a) {
-  static_assert(NP == 1 || (F16 && MODE == 0), "pieces are binary16");
+  static_assert(NP == 1 || (F16 && MODE != 2), "pieces are binary16");
   uint32_t sflags = 0;
-  if constexpr (MODE == 0) {
+  if constexpr (MODE != 2) {
     if (a.split) {
       sflags = a.split->flags;
       if (split_route(sflags) != a.route) return;
@@ -1952,6 +1952,26 @@ hipError_t ivf_inst(const FusedArgs& a, hipStream_t s, int mode) {
   return hipGetLastError();
 }
 
+// The scan over binary16 pieces of the index's rows (routes 1 and 2).
+template <int DH, int T, int NP>
+hipError_t ivf_pieces_inst(const FusedArgs& a, dim3 grid, hipStream_t s) {
+  if (a.metric == kL2)
+    hipLaunchKernelGGL((fused_kernel<true, DH, T, true, 1, false, NP>), grid, dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((fused_kernel<true, DH, T, false, 1, false, NP>), grid, dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+template <int DH, int NP>
+hipError_t ivf_pieces_t(const FusedArgs& a, dim3 grid, hipStream_t s) {
+  switch (a.T) {
+    case 4: return ivf_pieces_inst<DH, 4, NP>(a, grid, s);
+    case 8: return ivf_pieces_inst<DH, 8, NP>(a, grid, s);
+    case 10: return ivf_pieces_inst<DH, 10, NP>(a, grid, s);
+    case 16: return ivf_pieces_inst<DH, 16, NP>(a, grid, s);
+  }
+  return hipErrorInvalidValue;
+}
+
 template <int DH>
 hipError_t ivf_dispatch_t(const FusedArgs& a, hipStream_t s, int mode) {
   if (mode == 2) return ivf_inst<DH, 4>(a, s, mode);
@@ -2239,6 +2259,15 @@ hipError_t launch_fused_f16(const FusedArgs& a, hipStream_t s) {
 }
 
 hipError_t launch_ivf_select(const FusedArgs& a, hipStream_t s) { return ivf_launch(a, s, 1); }
+
+hipError_t launch_ivf_select_pieces(const FusedArgs& a, hipStream_t s) {
+  if (!fused_split_supported(a.ld, a.T) || !a.split || (a.route == 2 && (!a.base_lo || !a.queries_lo)))
+    return hipErrorInvalidValue;
+  if (a.n_items <= 0) return hipSuccess;
+  const dim3 grid((unsigned)((int64_t)a.n_items * (a.nsplit > 1 ? a.nsplit : 1)));
+  if (a.route == 1) return a.ld <= 64 ? ivf_pieces_t<32, 1>(a, grid, s) : ivf_pieces_t<64, 1>(a, grid, s);
+  return a.ld <= 64 ? ivf_pieces_t<32, 2>(a, grid, s) : ivf_pieces_t<64, 2>(a, grid, s);
+}
 
 hipError_t launch_ivf_scores(const FusedArgs& a, hipStream_t s) { return ivf_launch(a, s, 2); }
 

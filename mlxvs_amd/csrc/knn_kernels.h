@@ -266,6 +266,9 @@ int bits_row_bytes(int nbytes);
 // 2 q.b - |b|^2) of queries q0 .. into scores [.][width] (other entries are
 // left as they are).  fp32, ld a multiple of 4 up to 256.
 hipError_t launch_ivf_select(const FusedArgs& a, hipStream_t s);
+// launch_ivf_select over the rows' binary16 pieces (route 1: base / queries
+// the hi pieces; route 2: with base_lo / queries_lo; bnorm the seeds).
+hipError_t launch_ivf_select_pieces(const FusedArgs& a, hipStream_t s);
 hipError_t launch_ivf_scores(const FusedArgs& a, hipStream_t s);
 // The same scores for any ld, on the VALU (rows of deep indexes).
 hipError_t launch_ivf_scores_any(const FusedArgs& a, hipStream_t s);

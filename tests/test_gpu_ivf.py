@@ -228,3 +228,38 @@ def test_lists_of_16_repeated_calls(oracle):
             ids, dist = mlxvs_amd.ivf_flat_search(c, data, ind, off, "l2", q, k, n_probes=12)
             assert np.array_equal(ids, wi), (k, rep)
             assert np.array_equal(dist, wd), (k, rep)
+
+
+@pytest.mark.parametrize("kind,metric,k", [("int", "l2", 10), ("int", "l2", 40), ("float", "l2", 10),
+                                           ("float", "inner_product", 16),
+                                           ("outlier", "l2", 10), ("float", "cosine", 4)])
+def test_large_batches_scan_binary16_pieces(engine, oracle, kind, metric, k):
+    # enough (query, probe) pairs per list that the scan multiplies the rows'
+    # binary16 pieces: hi alone (integers), both, or the float32 kernel (a value
+    # past binary16's range), the same answers as the restatement's
+    rng = np.random.default_rng(k)
+    n, nq, lists, P, d = 160_000, 6_003, 96, 12, 67
+    x = rng.integers(0, 256, (n, d)).astype(np.float32)
+    q = rng.integers(0, 256, (nq, d)).astype(np.float32)
+    if kind != "int":
+        x, q = x + rng.random(x.shape, np.float32), q + rng.random(q.shape, np.float32)
+    if kind == "outlier":
+        x[77, 3] = 4.0e7
+    if metric == "cosine":
+        x /= np.linalg.norm(x, axis=1, keepdims=True)
+    centers = np.ascontiguousarray(x[rng.choice(n, lists, replace=False)])
+    label = engine.kmeans_predict(x, centers)[:, 0]
+    order = np.argsort(label, kind="stable")
+    off = np.concatenate([[0], np.cumsum(np.bincount(label, minlength=lists))]).astype(np.int32)
+    data, ind = np.ascontiguousarray(x[order]), order.astype(np.int32)
+    ids, dist = engine.ivf_flat_search(centers, data, ind, off, metric, q, k, n_probes=P)
+    pick = np.unique(np.concatenate([[0, 127, 128, nq - 1], np.linspace(0, nq - 1, 40).astype(int)]))
+    oi, od = oracle.ivf_flat(centers, data, ind, off, q[pick], k, P, metric)
+    if kind == "int":
+        assert np.array_equal(ids[pick], oi) and np.array_equal(dist[pick], od)
+        return
+    assert (ids[pick] == oi).mean() > 0.99
+    # float32 sums over 67 values of either route: (d + 4) 2^-24 of the
+    # magnitudes that meet, |q|^2 + |b|^2 at most 2 * 67 * 256^2 (4e7 aside)
+    tol = 71 * 2.0 ** -24 * (1.0 if metric == "cosine" else 4 * 67 * 256.0 ** 2)
+    assert np.abs(dist[pick] - od).max() <= tol
