@@ -618,8 +618,13 @@ bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, cons
   if (tile) {
     plan = plan_tile(n, nq, k, T, sld, true);
   } else if (kern::fused_split_supported(sld, T)) {
-    plan = plan_splits(n, qblocks, k, T, 2, 2 * kern::kTileRows,
-                       device_slots(kern::fused_split_blocks_per_cu(sld, T)), true,
+    // rounds of the hi kernel's workgroups (three a CU, the two-piece kernel's
+    // two): 1M x 128, 3,000 queries, integers 1.20 -> 1.05 ms, real values 2.44
+    // -> 2.37; batches that take the bounded merge lose more to the extra
+    // lists (1,000 queries 0.97 -> 0.99)
+    const int bpc = nq > kern::kBoundMergeQueries ? kern::fused_blocks_per_cu(sld, T, true)
+                                                  : kern::fused_split_blocks_per_cu(sld, T);
+    plan = plan_splits(n, qblocks, k, T, 2, 2 * kern::kTileRows, device_slots(bpc), true,
                        max_merge_segments(k, T));
   }
   if (!plan.ok || (plan.rows_per_split + 2 * kern::kTileKernelRows) * std::max(ld32, sld) * 4 >=
