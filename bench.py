@@ -3,12 +3,12 @@
 
     python bench.py [--gpus 1] [--steps 10] [--warmup 2] [--workload c2]
 
-Default workload (BASELINE.json metric): configuration c2, exact L2 k-NN,
+Default workload (the headline metric): configuration c2, exact L2 k-NN,
 k = 10, 1,000,000 x 128 float32 base rows (1,024-component mixture, integer
 values in [0, 255]) and 10,000 queries.  Inputs are generated with
 mlxvs_amd.synth, copied to HBM before timing, and one step is one
-mlxvs_brute_force_knn_device call over all 10,000 queries (norms, fused
-MFMA distance + top-k, merge).  W warm-up steps, then exactly K timed steps
+mlxvs_brute_force_knn_device call over all 10,000 queries (norms and
+binary16 pieces, fused MFMA distance + top-k, merge).  W warm-up steps, then exactly K timed steps
 between two device synchronisations; value = queries answered per second.
 The same K steps then run again with the engine's HIP events around every
 launch (ms_per_step_profiled): the kernel times below come from them.
@@ -18,7 +18,9 @@ The same JSON line carries:
                 recorded around each of its launches in the second K steps
                 (2 nq n d flops per launch over its mean duration; for Hamming
                 2 nq n bits ops on the FP4 MFMA), against MI355X's dense peak
-                of that type (FP32 157.3, FP16 2516.6, FP4 10066.4 TFLOP/s),
+                of that type (FP32 157.3, FP16 2516.6, FP4 10066.4 TFLOP/s;
+                fp32 rows multiplied as binary16 pieces count against FP16,
+                2 nq n d flops whatever the number of products),
                 or, below the ridge point (small batches), the rows' bytes per
                 launch against HBM's 8 TB/s;
                 traffic = HBM bytes per launch from the committed rocprofv3
@@ -33,7 +35,7 @@ The same JSON line carries:
                 against the float64 golden fixture.
 
 Other workloads (c1, c2h, c3, c3cos, c3h, c4, c5, ivf, topk) are for measurement runs; the
-driver's line is the default.  --workload copy times a 1 GiB device copy, the
+headline line is the default.  --workload copy times a 1 GiB device copy, the
 reference reading for scaling HBM byte counters.
 """
 
