@@ -615,19 +615,34 @@ bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, cons
   const int64_t qblocks = (nq + kQueriesPerBlock - 1) / kQueriesPerBlock;
   const int lanes = tile ? kern::tile_segments(T) : 2;
   SplitPlan plan;
+  int64_t rows2 = 0;  // rows_per_split of routes 2 and 0 (not tile)
   if (tile) {
     plan = plan_tile(n, nq, k, T, sld, true);
   } else if (kern::fused_split_supported(sld, T)) {
-    // rounds of the hi kernel's workgroups (three a CU, the two-piece kernel's
-    // two): 1M x 128, 3,000 queries, integers 1.20 -> 1.05 ms, real values 2.44
-    // -> 2.37; batches that take the bounded merge lose more to the extra
+    // rounds of each kernel's workgroups: three a CU of the hi kernel, two of
+    // the two-piece and the float32 kernel.  They share the segments, and one
+    // whose rounds take fewer splits leaves the last ones empty.  1M x 128,
+    // 3,000 queries, integers 1.20 -> 1.05 ms with the hi kernel's own rounds;
+    // with its splits for the others as well 200k x 100, 2,000 queries, took
+    // 479 us (two pieces) and 1,217 us (float32), with their own 445 and
+    // 1,016.  Batches that take the bounded merge lose more to the extra
     // lists (1,000 queries 0.97 -> 0.99)
-    const int bpc = nq > kern::kBoundMergeQueries ? kern::fused_blocks_per_cu(sld, T, true)
-                                                  : kern::fused_split_blocks_per_cu(sld, T);
-    plan = plan_splits(n, qblocks, k, T, 2, 2 * kern::kTileRows, device_slots(bpc), true,
-                       max_merge_segments(k, T));
+    auto planned = [&](int bpc) {
+      return plan_splits(n, qblocks, k, T, 2, 2 * kern::kTileRows, device_slots(bpc), true,
+                         max_merge_segments(k, T));
+    };
+    plan = planned(kern::fused_split_blocks_per_cu(sld, T));
+    rows2 = plan.rows_per_split;
+    if (nq > kern::kBoundMergeQueries) {
+      const SplitPlan hi = planned(kern::fused_blocks_per_cu(sld, T, true));
+      if (hi.ok && plan.ok && hi.xcd == plan.xcd) {
+        plan.nsplit = std::max(plan.nsplit, hi.nsplit);
+        plan.rows_per_split = hi.rows_per_split;
+      }
+    }
   }
-  if (!plan.ok || (plan.rows_per_split + 2 * kern::kTileKernelRows) * std::max(ld32, sld) * 4 >=
+  if (!plan.ok || (std::max(plan.rows_per_split, rows2) + 2 * kern::kTileKernelRows) *
+                          std::max(ld32, sld) * 4 >=
                       (int64_t(1) << 31))
     return false;
   // the float32 route's operands: the rows in place, or a padded copy, and
@@ -705,6 +720,7 @@ bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, cons
     fa.route = 1;
     launch(s, "fused_hi", [&] { return kern::launch_fused_f16(fa, s); });
     fa.route = 2;
+    fa.rows_per_split = rows2;
     launch(s, "fused_split", [&] { return kern::launch_fused_split(fa, s); });
   }
   // (its two segments a split: the same lists over finer splits)
@@ -717,7 +733,7 @@ bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, cons
   if (cos_factors) fa.metric = kern::kCosine;
   fa.ld = ld32;
   fa.nsplit = plan.nsplit * (lanes / 2);
-  fa.rows_per_split = plan.rows_per_split / (lanes / 2);
+  fa.rows_per_split = tile ? plan.rows_per_split / (lanes / 2) : rows2;
   if (deep32)
     launch(s, "fused_deep", [&] { return kern::launch_deep(fa, false, s); });
   else

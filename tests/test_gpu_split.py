@@ -214,3 +214,13 @@ def test_deep_rows_few_queries(engine, oracle, f16, n, nq, d, k, metric):
     if metric == "cosine":
         base[n // 2] = base[n // 2 - 1]  # (the bound divides by the row's norm)
     check(engine, oracle, base, q, k, metric, False)
+
+
+@pytest.mark.parametrize("kind", ["bytes", "normal", "outlier"])
+@pytest.mark.parametrize("nq,k", [(1_025, 10), (2_000, 16)])
+def test_routes_with_their_own_rounds(engine, oracle, kind, nq, k):
+    """More queries than the bounded merge takes: the hi kernel's splits are
+    finer than the other two routes', whose last segments stay empty."""
+    r = np.random.default_rng(nq)
+    base, q = rows_of(kind, N, 128, r), rows_of(kind, nq, 128, r)
+    check(engine, oracle, base, q, k, "l2", kind == "bytes")
