@@ -20,6 +20,11 @@ constexpr int kSamplePer = 8;
 // 2^-13 is 2^-24, so a value down to 1/4096 of the largest keeps 24 bits and
 // smaller ones an error of 2^-36 of the largest.
 constexpr int kSampleExp = 11;
+// Samples whose largest value lies outside 2^-40 .. 2^40 take the float32
+// route: with both scales in 2^-28 .. 2^52 their product and its inverse, and
+// the seeds -|b|^2 / 2 sbase squery (below d 2^112, as sbase |b| < 2^16 sqrt(d)
+// and squery / sbase <= 2^80), stay inside float32.
+constexpr int kMaxSampleExp = 40;
 // Unit rows: their values are at most 1 (and a rounding), scaled to 2^15.
 constexpr float kUnitScale = 32768.0f;
 
@@ -62,17 +67,20 @@ __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArg
   __syncthreads();
   if (tid != 0) return;
   float sc[2];
+  uint32_t flags = 0;
   for (int side = 0; side < 2; ++side) {
     float x = 0.0f;
     for (int w = 0; w < kSampleThreads / 64; ++w) x = fmaxf(x, wmax[side][w]);
-    // (a sample of zeros, or one past 2^80 either way: any scale will do,
-    // the pass over all rows decides whether it did)
-    int e = 0;
-    const bool usable = x > 0x1p-80f && x < 0x1p80f;
-    if (usable) (void)frexpf(x, &e);  // x = f 2^e, f in [1/2, 1)
-    sc[side] = a.unit ? kUnitScale : usable ? ldexpf(1.0f, kSampleExp + 1 - e) : 1.0f;
+    sc[side] = a.unit ? kUnitScale : 1.0f;
+    if (a.unit || x == 0.0f) continue;  // (a sample of zeros: the pass over all rows decides)
+    int e = kMaxSampleExp + 1;
+    if (x < INFINITY) (void)frexpf(x, &e);  // x = f 2^e, f in [1/2, 1)
+    if (e < -kMaxSampleExp || e > kMaxSampleExp)
+      flags = kSplitRows32;
+    else
+      sc[side] = ldexpf(1.0f, kSampleExp + 1 - e);
   }
-  a.st->flags = 0;
+  a.st->flags = flags;
   a.st->sbase = sc[0];
   a.st->squery = sc[1];
   a.st->inv = 1.0f / (sc[0] * sc[1]);  // powers of two: exact

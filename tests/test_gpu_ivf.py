@@ -232,7 +232,8 @@ def test_lists_of_16_repeated_calls(oracle):
 
 @pytest.mark.parametrize("kind,metric,k", [("int", "l2", 10), ("int", "l2", 40), ("float", "l2", 10),
                                            ("float", "inner_product", 16),
-                                           ("outlier", "l2", 10), ("float", "cosine", 4)])
+                                           ("outlier", "l2", 10), ("float", "cosine", 4),
+                                           ("small", "inner_product", 10), ("small", "l2", 10)])
 def test_large_batches_scan_binary16_pieces(engine, oracle, kind, metric, k):
     # enough (query, probe) pairs per list that the scan multiplies the rows'
     # binary16 pieces: hi alone (integers), both, or the float32 kernel (a value
@@ -247,6 +248,8 @@ def test_large_batches_scan_binary16_pieces(engine, oracle, kind, metric, k):
         x[77, 3] = 4.0e7
     if metric == "cosine":
         x /= np.linalg.norm(x, axis=1, keepdims=True)
+    if kind == "small":  # (the two sides' scales multiply past float32's range)
+        x, q = x * np.float32(2.0 ** -60), q * np.float32(2.0 ** -60)
     centers = np.ascontiguousarray(x[rng.choice(n, lists, replace=False)])
     label = engine.kmeans_predict(x, centers)[:, 0]
     order = np.argsort(label, kind="stable")
@@ -262,4 +265,6 @@ def test_large_batches_scan_binary16_pieces(engine, oracle, kind, metric, k):
     # float32 sums over 67 values of either route: (d + 4) 2^-24 of the
     # magnitudes that meet, |q|^2 + |b|^2 at most 2 * 67 * 256^2 (4e7 aside)
     tol = 71 * 2.0 ** -24 * (1.0 if metric == "cosine" else 4 * 67 * 256.0 ** 2)
+    if kind == "small":
+        tol *= 2.0 ** -120
     assert np.abs(dist[pick] - od).max() <= tol

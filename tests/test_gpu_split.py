@@ -141,6 +141,28 @@ def test_every_kind_of_values(engine, oracle, kind, metric, d, k, exact):
     check(engine, oracle, base, q, k, metric, exact)
 
 
+@pytest.mark.parametrize("metric,d,eb,eq", [
+    ("inner_product", 128, -54, -54), ("inner_product", 100, -70, -46), ("inner_product", 300, -60, -60),
+    ("l2", 128, -54, -54), ("l2", 1536, -54.6, -54.6), ("l2", 1536, 44.5, -55), ("inner_product", 64, 30, -90),
+    # (the last scales that take the pieces)
+    ("l2", 96, -42, -42), ("l2", 96, 36, -42), ("inner_product", 96, -42, 36),
+])
+def test_scales_far_from_one(engine, oracle, metric, d, eb, eq):
+    """Values whose two scales multiply to (or whose seeds are) past float32's
+    range: sums that float32 holds, so the answers are ordinary ones.  A zero
+    row, and one whose squares underflow."""
+    r = np.random.default_rng(d)
+    n, nq = size_of(d)
+    base, q = rows_of("float", n, d, r), rows_of("float", nq, d, r)
+    base *= np.float32(2.0 ** eb)
+    q *= np.float32(2.0 ** eq)
+    if metric == "l2" and eb < 0:
+        base[7] = 0
+        if eb == -54:
+            base[8] *= np.float32(2.0 ** -20)
+    check(engine, oracle, base, q, 10, metric, False)
+
+
 @pytest.mark.parametrize("kind,d", [("bytes", 96), ("float", 96), ("outlier", 96),
                                     ("bytes", 131), ("float", 272), ("outlier", 272)])
 def test_prefilter(engine, oracle, kind, d):
