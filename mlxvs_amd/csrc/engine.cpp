@@ -679,8 +679,8 @@ bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, cons
     seed = ar.take<float>((size_t)n);
     qnorm = ar.take<float>((size_t)nq);
   }
-  kern::SplitRowsArgs sb{in.base, n, d, d, f16, ubn, bnorm, 1, seed, bhi, blo, sld, 0, st};
-  kern::SplitRowsArgs sq{in.queries, nq, d, d, f16, uqn, qnorm, 0, nullptr, qhi, qlo, sld, 1, st};
+  kern::SplitRowsArgs sb{in.base, n, d, d, f16, ubn, bnorm, 1, seed, bhi, blo, sld, 0, l2, st};
+  kern::SplitRowsArgs sq{in.queries, nq, d, d, f16, uqn, qnorm, 0, nullptr, qhi, qlo, sld, 1, l2, st};
   const int nseg = lanes * plan.nsplit;
   const int slots = kern::bound_slots_for(T);
   const BoundPlan bp = shared_bound(k, T, slots, nseg);
@@ -1381,11 +1381,11 @@ void ivf_search(Session& ss, const float* centers, int64_t lists, const float* d
       uint16_t* qhi = ar.take<uint16_t>((size_t)nq * sld);
       uint16_t* qlo = ar.take<uint16_t>((size_t)nq * sld);
       float* seed = l2 ? ar.take<float>((size_t)n) : nullptr;
-      const kern::SplitInitArgs si{kd, kq, n, nq, ld, ld, 0, st};
+      const kern::SplitInitArgs si{kd, kq, n, nq, d, ld, 0, st};
       launch(s, "prep", [&] { return kern::launch_split_init(si, s); });
-      const kern::SplitRowsArgs sb{kd, n, ld, ld, 0, nullptr, bnorm, 1, seed, bhi, blo, sld, 0, st};
+      const kern::SplitRowsArgs sb{kd, n, ld, ld, 0, nullptr, bnorm, 1, seed, bhi, blo, sld, 0, l2, st};
       const kern::SplitRowsArgs sq{kq, nq, ld, ld, 0, nullptr, nullptr, 0, nullptr, qhi, qlo, sld,
-                                   1, st};
+                                   1, l2, st};
       const kern::BoundsInit bi{gkey, nq * slots_n, slots_n, bp.m};
       launch(s, "prep", [&] { return kern::launch_split_rows(sb, sq, bi, s); });
       kern::FusedArgs fp = fa;

@@ -147,7 +147,7 @@ __global__ __launch_bounds__(256) void row_norms_kernel(PrepArgs aa, PrepArgs ab
 // fp32 rows, which are padded to 736, 0.57 -> 0.44 ms a call).
 template <typename Int>
 __global__ __launch_bounds__(256) void rows_transform_kernel(PrepArgs a, Int total) {
-  if (a.split && split_route(a.split->flags) != 0) return;
+  if (a.split && split_route(*a.split) != 0) return;
   const uint32_t lv = (uint32_t)a.out_ld / 4;
   // (the host keeps the grid's last step below Int's range)
   for (Int e = (Int)blockIdx.x * 256 + threadIdx.x; e < total; e += (Int)gridDim.x * 256) {
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256, (fused_min_blocks<F16, DH>())) void fused_kern
   if constexpr (MODE != 2) {
     if (a.split) {
       sflags = a.split->flags;
-      if (split_route(sflags) != a.route) return;
+      if (split_route(*a.split) != a.route) return;
     }
   }
   using E = typename std::conditional<F16, _Float16, float>::type;
@@ -643,7 +643,7 @@ constexpr int kDeepRB = kDeepRows / 32;        // MFMA row blocks per wavefront
 // norms.
 template <int T, bool L2, bool F16, bool FILT = false, bool COS = false>
 __global__ __launch_bounds__(256, 2) void deep_kernel(FusedArgs a) {
-  if (!F16 && a.split && split_route(a.split->flags) != a.route) return;
+  if (!F16 && a.split && split_route(*a.split) != a.route) return;
   constexpr int esize = F16 ? 2 : 4;
   constexpr int CH = kDeepChunkBytes / esize;  // dims per stage
   // chunks of the tile's rows and of the block's queries, loaded straight

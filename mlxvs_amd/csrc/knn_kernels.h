@@ -59,11 +59,11 @@ hipError_t launch_norms_pair(const PrepArgs& a, const PrepArgs& b, const BoundsI
                              hipStream_t s);
 
 // Float32 rows as two binary16 pieces: x 2^s = hi + lo, hi the nearest
-// binary16 and lo the nearest to the rest (13 bits at most: lo drops a last
-// bit of 24 at most), so that the products run on the fp16 MFMA, which sums
-// exact products of halves in float32.  One power of two scales all base
-// rows and one all queries (launch_split_init, from a sample); what a call's
-// rows turn out to need is collected on the device in SplitState::flags
+// binary16 and lo the nearest to the rest (12 bits and a sign: lo may drop the
+// last of a value's 24 bits, 2^-23 of it), so that the products run on the
+// fp16 MFMA, which sums exact products of halves in float32.  One power of two
+// scales all base rows and one all queries (launch_split_init, from a sample);
+// what a call's rows turn out to need is collected on the device in SplitState
 // (launch_split_rows), and every kernel of the call that serves one route
 // returns at once on another's.
 enum SplitFlags : uint32_t {
@@ -72,30 +72,48 @@ enum SplitFlags : uint32_t {
   kSplitBaseLong = 4,   // some base value has more than 16 significant bits
   kSplitQueryLong = 8,  // some query value has
   kSplitRows32 = 16,    // the pieces cannot stand for the rows: a value past
-                        // binary16's range or not finite, or a row most of
-                        // whose values lie below its precision
+                        // binary16's range or not finite, or (L2) a row that
+                        // they miss by more than 2^-25 of its length
 };
+// Values below 2^-2 in the pieces' scale lose more than their last bit: up to
+// 2^-25, whatever their size.  Under L2 that error meets |q| and stays below
+// the rounding of |q|^2 and |b|^2, so it is judged row by row (kSplitRows32).
+// An inner product can consist of such values alone (a query that is zero
+// where its rows are large), so it is held against what every pair's products
+// amount to: with caps, min(|q|, C) and min(|b|, C) of a column multiply to at
+// least C (min(|q|, C) + min(|b|, C) - C), so
+//   sum |q_i b_i| >= C (least[query] + least[base] - d C),
+// least the smallest sum of a nonzero row's capped values; and the error is at
+// most lost[base] top[query] + lost[query] top[base], lost the largest sum of a
+// row's errors past rounding.  Dense rows keep most of d C on both sides; sparse
+// or masked ones do not, and take the float32 route if they have such values.
+constexpr float kSplitCap = 48.0f;  // about 1/64 of the sample's largest value
 struct SplitState {
   uint32_t flags;
   float sbase, squery;  // 2^s of the base rows and of the queries
   float inv;            // scores from the pieces times inv are the rows' scores
+  float room;           // d C
+  // [base, queries]; not negative, so their bits order as they do
+  float lost[2], top[2], least[2];
 };
 // Which kernel a call's rows take: 0 the float32 MFMA, 1 the hi pieces alone
 // (no value has a lo piece: integers, rows that were binary16), 2 both.
-__host__ __device__ inline int split_route(uint32_t flags) {
-  return flags & kSplitRows32 ? 0 : flags & (kSplitBaseLow | kSplitQueryLow) ? 2 : 1;
+__device__ inline int split_route(const SplitState& s) {
+  if (s.flags & kSplitRows32) return 0;
+  const float error = s.lost[0] * s.top[1] + s.lost[1] * s.top[0];
+  if (error > 0.0f && !(error <= 0x1p-24f * kSplitCap * (s.least[0] + s.least[1] - s.room))) return 0;
+  return s.flags & (kSplitBaseLow | kSplitQueryLow) ? 2 : 1;
 }
-// The lo x lo products are at most 2^-24 of a value's product, below half a
-// unit of the float32 sum they would join; they are formed when both sides
-// have lo pieces and one side has short values only (at most 16 bits), whose
-// float32 sums can be exact.
-__host__ __device__ inline bool split_low_low(uint32_t flags) {
+// The lo x lo products are at most 2^-22 of a value's product, 2^-25 of it on
+// average; they are formed when both sides have lo pieces and one side has
+// short values only (at most 16 bits), whose float32 sums can be exact.
+__device__ inline bool split_low_low(uint32_t flags) {
   const uint32_t low = kSplitBaseLow | kSplitQueryLow, lng = kSplitBaseLong | kSplitQueryLong;
   return (flags & low) == low && (flags & lng) != lng;
 }
 // The factor that takes a call's list scores to the rows' scores.
-__host__ __device__ inline float list_score_scale(const SplitState* st) {
-  return st && split_route(st->flags) != 0 ? st->inv : 1.0f;
+__device__ inline float list_score_scale(const SplitState* st) {
+  return st && split_route(*st) != 0 ? st->inv : 1.0f;
 }
 // Sets st: no flags, the scales from a sample of the rows (unit: rows of
 // length at most 1).
@@ -124,6 +142,7 @@ struct SplitRowsArgs {
   uint16_t* lo;             // pieces, then their lo pieces, and so on
   int out_ld;               // a multiple of 8 (lo null: of kTilePieceRun)
   int query;                // the rows are the queries
+  int l2;                   // errors judged row by row (see SplitState)
   SplitState* st;
 };
 // (the base rows, the queries and the bounds in one launch, as

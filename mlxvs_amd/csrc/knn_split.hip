@@ -17,8 +17,8 @@ constexpr int kSampleThreads = 1024;
 constexpr int kSamplePer = 8;
 // The sample's largest value is scaled to [2^11, 2^12): binary16 ends at
 // 2^16, so values up to 16 times larger still fit, and its spacing below
-// 2^-13 is 2^-24, so a value down to 1/4096 of the largest keeps 24 bits and
-// smaller ones an error of 2^-36 of the largest.
+// 2^-13 is 2^-24, so a value down to 2^-2 keeps 23 bits and smaller ones have an
+// error of up to 2^-25 (split_route: where that is too much).
 constexpr int kSampleExp = 11;
 // Samples whose largest value lies outside 2^-40 .. 2^40 take the float32
 // route: with both scales in 2^-28 .. 2^52 their product and its inverse, and
@@ -84,6 +84,11 @@ __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArg
   a.st->sbase = sc[0];
   a.st->squery = sc[1];
   a.st->inv = 1.0f / (sc[0] * sc[1]);  // powers of two: exact
+  a.st->room = (float)a.d * kSplitCap;
+  for (int side = 0; side < 2; ++side) {
+    a.st->lost[side] = a.st->top[side] = 0.0f;
+    a.st->least[side] = INFINITY;
+  }
 }
 
 // 256 rows per workgroup, a 32-value slab at a time through LDS: fetched with
@@ -148,7 +153,9 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
     }
   };
   // pieces: thread t converts values 8 (t % 4) .. + 7 of rows t / 4 + 64 j
-  int lossy[4] = {0, 0, 0, 0};
+  // (rows' errors past rounding and what they are held against, SplitState;
+  // L2: both squared)
+  float lost[4] = {0, 0, 0, 0}, mass[4] = {0, 0, 0, 0}, top = 0.0f;
   uint32_t seen = 0;  // bit 0: a lo piece, 1: a long value, 2: out of range
   load_slab(0);
   for (int c0 = 0; c0 < a.out_ld; c0 += 32) {
@@ -194,23 +201,31 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
         for (int u = 0; u < 8; ++u) x[u] = x[u] / den;
       }
       halfx8 hi, lo;
-      int lost = 0;
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        const float xs = x[u] * scale;
+        const float xs = x[u] * scale, ax = fabsf(xs);
         const _Float16 hv = (_Float16)xs;
         const float rest = xs - (float)hv;  // exact
         const _Float16 lv = (_Float16)rest;
         hi[u] = hv;
         lo[u] = lv;
         const uint16_t lb = __builtin_bit_cast(uint16_t, lv);
-        if (!(fabsf(xs) <= 65504.0f)) seen |= 4u;
+        if (!(ax <= 65504.0f)) seen |= 4u;
         if (lb & 0x7fffu) seen |= 1u;
         if ((lb & 0x003fu) && (lb & 0x7c00u)) seen |= 2u;
-        // (rest - lo, exact; a value whose scaling underflowed is lost too)
-        if (fabsf(rest - (float)lv) > fabsf(xs) * 0x1p-23f || (xs == 0.0f && x[u] != 0.0f)) ++lost;
+        // (exact; a value whose scaling underflowed is lost too)
+        float err = fabsf(rest - (float)lv);
+        if (xs == 0.0f && x[u] != 0.0f) err = 0x1p-25f;
+        if (!(err > ax * 0x1p-23f)) err = 0.0f;
+        if (a.l2) {
+          lost[j] = __builtin_fmaf(err, err, lost[j]);
+          mass[j] = __builtin_fmaf(xs, xs, mass[j]);
+        } else {
+          lost[j] += err;
+          mass[j] += fminf(ax, kSplitCap);
+          top = fmaxf(top, ax);
+        }
       }
-      lossy[j] += lost;
       // (interleaved: a run of hi pieces, then their lo pieces)
       constexpr int R = kTilePieceRun;
       const int cc = c0 + c;
@@ -222,14 +237,21 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
     }
     __syncthreads();
   }
-  // a row most of whose values the pieces lose bits of (more than an eighth):
-  // its four threads' counts
+  // each row's four threads' sums (a row past the end: zeros)
+  float worst = 0.0f, least = INFINITY;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    int t = lossy[j];
-    t += __shfl_xor(t, 1);
-    t += __shfl_xor(t, 2);
-    if (8 * t > a.d) seen |= 4u;
+    float l = lost[j], m = mass[j];
+    l += __shfl_xor(l, 1);
+    m += __shfl_xor(m, 1);
+    l += __shfl_xor(l, 2);
+    m += __shfl_xor(m, 2);
+    if (a.l2) {
+      if (l > 0x1p-50f * m) seen |= 4u;
+    } else {
+      worst = fmaxf(worst, l);
+      if (m > 0.0f || l > 0.0f) least = fminf(least, m);
+    }
   }
   if ((a.norm || a.seed) && row0 + tid < a.n) {
     const float s01 = acc[0] + acc[1], s23 = acc[2] + acc[3];
@@ -241,6 +263,29 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
     const float half = nn > 0.0f ? -0.5f * nn : 0.0f;  // (+0, as row_norms_kernel)
     if (a.norm) a.norm[row0 + tid] = a.half_neg ? half : nn;
     if (a.seed) a.seed[row0 + tid] = half * seed_scale;
+  }
+  if (!a.l2) {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      worst = fmaxf(worst, __shfl_xor(worst, o));
+      least = fminf(least, __shfl_xor(least, o));
+      top = fmaxf(top, __shfl_xor(top, o));
+    }
+    if ((tid & 63) == 0) {
+      // (read first, as the flags below)
+      auto raise = [](float* p, float v) {
+        unsigned* w = (unsigned*)p;
+        const unsigned b = __float_as_uint(v);
+        if (b > __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+          __hip_atomic_fetch_max(w, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      };
+      raise(&a.st->lost[a.query], worst);
+      raise(&a.st->top[a.query], top);
+      unsigned* w = (unsigned*)&a.st->least[a.query];
+      const unsigned b = __float_as_uint(least);
+      if (b < __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        __hip_atomic_fetch_min(w, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
   }
   uint32_t any = (__builtin_amdgcn_ballot_w64(seen & 1u) ? (a.query ? kSplitQueryLow : kSplitBaseLow) : 0u) |
                  (__builtin_amdgcn_ballot_w64(seen & 2u) ? (a.query ? kSplitQueryLong : kSplitBaseLong) : 0u) |

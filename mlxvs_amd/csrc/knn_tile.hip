@@ -69,7 +69,7 @@ __global__ __launch_bounds__(kThreads, 1) void tile_kernel(FusedArgs a) {
   uint32_t sflags = 0;
   if (a.split) {
     sflags = a.split->flags;
-    if ((split_route(sflags) == 0) != (a.route == 0)) return;
+    if ((split_route(*a.split) == 0) != (a.route == 0)) return;
   }
   // separately named stages, so that loads into one are not taken to alias
   // the reads of another

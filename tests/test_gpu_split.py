@@ -6,11 +6,14 @@ the float32 kernels.  Every kind of values here must give what the float32
 route gives: integers bit for bit (their sums are exact either way), real
 values to float32 accuracy.
 
-The tolerance on real values: the pieces hold a value to 2^-24 of itself, the
-dropped lo x lo products are below 2^-24 of theirs, and the float32 sums have
-fewer roundings than the float32 kernels' (a multiply-add each: at most d
-2^-24 of the sum of magnitudes), so |error| <= (d + 4) 2^-24 sum |q_i b_i|,
-which Cauchy-Schwarz bounds by |q| |b|; L2 takes it twice and adds its norms'.
+The tolerance on real values is one of each sum's own terms, sum |q_i b_i| (not
+of the rows' lengths, which say nothing of a query that is zero where its rows
+are large).  In units of 2^-24 of it: the pieces hold each value to 2 (both
+sides: 4), the lo x lo products that may be left out are at most 4, a small
+value's loss at most 1 (inner products; L2: 2 of |q| |b|), and the float32 sums,
+on either unit, take at most one rounding a term: d + 9 in all.  L2 takes that
+twice and adds its norms' and last sums' roundings, d + 4 of |q|^2 + |b|^2 at
+most; cosine rounds each unit value, d / 8 + 6 a side.
 """
 
 import numpy as np
@@ -71,30 +74,31 @@ def check(engine, oracle, base, q, k, metric, exact, count=SAMPLE, **filt):
     q64 = q[pick].astype(np.float64)
     bn = np.sqrt(np.einsum("ij,ij->i", base, base, dtype=np.float64))
     qn = np.linalg.norm(q64, axis=1)
-    dots = np.concatenate([base[i:i + 20_000].astype(np.float64) @ q64.T
-                           for i in range(0, len(base), 20_000)])
-    u = (base.shape[1] + 4) * 2.0 ** -24
+
+    def products(f):
+        return np.concatenate([f(base[i:i + 20_000].astype(np.float64)) @ f(q64).T
+                               for i in range(0, len(base), 20_000)])
+
+    dots, terms = products(lambda x: x), products(np.abs)
+    d, u = base.shape[1], 2.0 ** -24
     for i in range(len(pick)):
         got, g = ids[pick][i], dist[pick][i].astype(np.float64)
-        s = dots[:, i]
-        mag = qn[i] * bn
+        s, err = dots[:, i], (d + 9) * u * terms[:, i]
         if metric == "l2":
             s = bn * bn + qn[i] * qn[i] - 2 * s
-            err = u * (qn[i] + bn) ** 2
+            err = 2 * err + (d + 4) * u * (qn[i] ** 2 + bn * bn) + 2 * u * qn[i] * bn
         elif metric == "cosine":
-            s, err = s / mag, np.full(len(bn), 2 * u)
-        else:
-            err = u * mag
+            mag = np.maximum(qn[i] * bn, 1e-300)
+            s, err = s / mag, (err + (d / 4 + 12) * u * terms[:, i]) / mag
         if "bitset" in filt:
             s = np.where(filt["bitset"], s, np.inf if metric == "l2" else -np.inf)
         assert len(set(got.tolist())) == k
-        assert (np.abs(g - s[got]) <= err[got]).all(), np.abs(g - s[got]).max()
-        # no row left out is better than the last kept by more than the errors
+        assert (np.abs(g - s[got]) <= err[got]).all(), (np.abs(g - s[got]) / err[got]).max()
+        # no row left out is better than one kept by more than their two errors
         order = s if metric == "l2" else -s
         left = np.ones(len(s), bool)
         left[got] = False
-        worst = (order[got] + 2 * err[got]).max()
-        assert ((order + 2 * err)[left] >= worst - 4 * err.max()).all()
+        assert (order + err)[left].min() >= (order - err)[got].max()
 
 
 @pytest.mark.parametrize("kind,metric,d,k,exact", [
@@ -139,6 +143,32 @@ def test_every_kind_of_values(engine, oracle, kind, metric, d, k, exact):
     n, nq = size_of(d)
     base, q = rows_of(kind, n, d, r), rows_of(kind, nq, d, r)
     check(engine, oracle, base, q, k, metric, exact)
+
+
+@pytest.mark.parametrize("metric", ["inner_product", "cosine", "l2"])
+@pytest.mark.parametrize("kind,d,scale", [
+    ("columns", 128, 1e-6), ("columns", 128, 1e-10), ("columns", 40, 1e-8), ("columns", 768, 1e-8),
+    ("rows", 128, 1e-6), ("rows", 300, 1e-8), ("rows", 64, 1e-3),
+])
+def test_small_values_decide(engine, oracle, metric, kind, d, scale):
+    """Scores that rest on values far below the rest of the data: columns of a
+    small scale under queries that are zero elsewhere, and sparse rows of small
+    values; neither has many values that the pieces lose bits of."""
+    r = np.random.default_rng(d)
+    n, nq = size_of(d)
+    base, q = rows_of("float", n, d, r), rows_of("float", nq, d, r)
+    some = r.choice(d, d // 16, replace=False)
+    if kind == "columns":
+        base[:, some] *= np.float32(scale)
+        keep = np.zeros(d, np.float32)
+        keep[some] = 1
+        q[::2] *= keep
+    else:
+        small = np.zeros((n // 8, d), np.float32)
+        small[:, some] = base[:n // 8, some] * np.float32(scale)
+        base[:n // 8] = small
+        check(engine, oracle, base, q, 10, metric, False, bitset=np.arange(n) < n // 8)
+    check(engine, oracle, base, q, 10, metric, False)
 
 
 @pytest.mark.parametrize("metric,d,eb,eq", [
