@@ -74,7 +74,14 @@ enum SplitFlags : uint32_t {
   kSplitRows32 = 16,    // the pieces cannot stand for the rows: a value past
                         // binary16's range or not finite, or (L2) a row that
                         // they miss by more than 2^-25 of its length
+  kSplitShort = 32,     // sums so short that the pieces' own error shows: only
+                        // rows without lo pieces take them
 };
+// Under L2 the lost 24th bits show in sums of few terms: rms error against 64
+// bits, pieces over float32 kernels, of near rows at 16 / 20 / 24 / 28 / 32
+// dims 1.13 / 1.09 / 1.01 / 0.99 / 0.94 (1.0 at 36 to 0.78 at 128); inner
+// products at 8 / 16 dims 1.09 / 0.80.
+constexpr int kSplitShortL2 = 32, kSplitShortDot = 16;
 // Values below 2^-2 in the pieces' scale lose more than their last bit: up to
 // 2^-25, whatever their size.  Under L2 that error meets |q| and stays below
 // the rounding of |q|^2 and |b|^2, so it is judged row by row (kSplitRows32).
@@ -102,11 +109,13 @@ __device__ inline int split_route(const SplitState& s) {
   if (s.flags & kSplitRows32) return 0;
   const float error = s.lost[0] * s.top[1] + s.lost[1] * s.top[0];
   if (error > 0.0f && !(error <= 0x1p-24f * kSplitCap * (s.least[0] + s.least[1] - s.room))) return 0;
-  return s.flags & (kSplitBaseLow | kSplitQueryLow) ? 2 : 1;
+  if (!(s.flags & (kSplitBaseLow | kSplitQueryLow))) return 1;
+  return s.flags & kSplitShort ? 0 : 2;
 }
 // The lo x lo products are at most 2^-22 of a value's product, 2^-25 of it on
 // average; they are formed when both sides have lo pieces and one side has
-// short values only (at most 16 bits), whose float32 sums can be exact.
+// short values only (at most 16 bits), whose float32 sums can be exact, and for
+// rows of at most 64 values, whose sums have few other roundings.
 __device__ inline bool split_low_low(uint32_t flags) {
   const uint32_t low = kSplitBaseLow | kSplitQueryLow, lng = kSplitBaseLong | kSplitQueryLong;
   return (flags & low) == low && (flags & lng) != lng;
@@ -115,14 +124,15 @@ __device__ inline bool split_low_low(uint32_t flags) {
 __device__ inline float list_score_scale(const SplitState* st) {
   return st && split_route(*st) != 0 ? st->inv : 1.0f;
 }
-// Sets st: no flags, the scales from a sample of the rows (unit: rows of
-// length at most 1).
+// Sets st: the scales from a sample of the rows (unit: rows of length at most
+// 1), no flags but kSplitShort.
 struct SplitInitArgs {
   const float* base;     // [n, ld], first d used
   const float* queries;  // [nq, ld]
   int64_t n, nq;
   int d, ld;
   int unit;
+  int l2;
   SplitState* st;
 };
 hipError_t launch_split_init(const SplitInitArgs& a, hipStream_t s);

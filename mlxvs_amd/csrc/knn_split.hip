@@ -67,7 +67,7 @@ __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArg
   __syncthreads();
   if (tid != 0) return;
   float sc[2];
-  uint32_t flags = 0;
+  uint32_t flags = a.d < (a.l2 ? kSplitShortL2 : kSplitShortDot) ? kSplitShort : 0u;
   for (int side = 0; side < 2; ++side) {
     float x = 0.0f;
     for (int w = 0; w < kSampleThreads / 64; ++w) x = fmaxf(x, wmax[side][w]);
@@ -76,7 +76,7 @@ __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArg
     int e = kMaxSampleExp + 1;
     if (x < INFINITY) (void)frexpf(x, &e);  // x = f 2^e, f in [1/2, 1)
     if (e < -kMaxSampleExp || e > kMaxSampleExp)
-      flags = kSplitRows32;
+      flags |= kSplitRows32;
     else
       sc[side] = ldexpf(1.0f, kSampleExp + 1 - e);
   }

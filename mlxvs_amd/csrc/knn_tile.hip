@@ -152,15 +152,10 @@ __global__ __launch_bounds__(kThreads, 1) void tile_kernel(FusedArgs a) {
   }
 
   floatx16 acc[NB][NC2];
-#pragma unroll
-  for (int b = 0; b < NB; ++b)
-#pragma unroll
-    for (int c = 0; c < NC2; ++c)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[b][c][i] = 0.0f;
 
   const bool blow = sflags & kSplitBaseLow, qlow = sflags & kSplitQueryLow;
   const bool lowlow = PIECES && split_low_low(sflags);
+  const bool seeds_first = a.ld <= kMaxFusedDimF32;
   int cc = 0, t = 0;
   auto step = [&](const uint32_t* cA, const uint32_t* cQ, uint32_t* nA, uint32_t* nQ) {
     // every wavefront's loads of this chunk have landed, and every wavefront
@@ -170,6 +165,25 @@ __global__ __launch_bounds__(kThreads, 1) void tile_kernel(FusedArgs a) {
     __builtin_amdgcn_sched_barrier(0);
     const bool last = cc + 1 == NC;
     if (wave_on) {
+      // L2: the sums start at the rows' -|b|^2 / 2 up to 256 values, where the
+      // float32 route's do too, and take it at their end above.  Whichever keeps
+      // them smaller on the way rounds less: values of one sign 0.53 units (rms,
+      // of 2^-24 of the sum of magnitudes) against 0.98 at 200 dims; values of
+      // both signs 1.40 against 0.56 at 384, and 3.0 against 0.73 at 1,536
+      if (cc == 0) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            floatx4 hn = {};
+            if (L2 && seeds_first)
+              hn = *(const floatx4*)&tnorm[kTR * (t & 1) + row_w + 32 * b + 8 * j + 4 * h];
+#pragma unroll
+            for (int c = 0; c < NC2; ++c)
+#pragma unroll
+              for (int u = 0; u < 4; ++u) acc[b][c][4 * j + u] = hn[u];
+          }
+      }
       const int sw = swz(col);
       const uint32_t* arow = cA + (row_w + col) * kChunkDwords;
       const uint32_t* qrow = cQ + (q_w + col) * kChunkDwords;
@@ -264,7 +278,7 @@ __global__ __launch_bounds__(kThreads, 1) void tile_kernel(FusedArgs a) {
             for (int j = 0; j < 4; ++j) {
               // L2 half scores q.b + (-|b|^2 / 2), one rounding (deep_kernel)
               floatx4 hn = {};
-              if constexpr (L2)
+              if (L2 && !seeds_first)
                 hn = *(const floatx4*)&tnorm[kTR * (t & 1) + row_w + 32 * b + 8 * j + 4 * h];
 #pragma unroll
               for (int u = 0; u < 4; ++u)
@@ -279,12 +293,6 @@ __global__ __launch_bounds__(kThreads, 1) void tile_kernel(FusedArgs a) {
               __hip_atomic_fetch_max(gk + myslot, kp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           }
         }
-#pragma unroll
-        for (int b = 0; b < NB; ++b)
-#pragma unroll
-          for (int c = 0; c < NC2; ++c)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[b][c][i] = 0.0f;
       }
     }
     __builtin_amdgcn_sched_barrier(0);

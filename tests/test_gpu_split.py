@@ -171,6 +171,36 @@ def test_small_values_decide(engine, oracle, metric, kind, d, scale):
     check(engine, oracle, base, q, 10, metric, False)
 
 
+@pytest.mark.parametrize("kind,metric,d", [
+    ("float", "l2", 16), ("float", "l2", 24), ("float", "l2", 40), ("float", "l2", 128),
+    ("positive", "l2", 200), ("float", "l2", 768), ("float", "inner_product", 9),
+    ("float", "inner_product", 33), ("positive", "inner_product", 300), ("float", "cosine", 96),
+    ("float", "cosine", 384),
+])
+def test_errors_no_larger_than_the_float32_kernels(engine, kind, metric, d):
+    """Errors against 64 bits of a batch and of its first 128 queries alone,
+    which the float32 kernels take.  128 x 50 distances: their rms is known to
+    1 / sqrt(2 x 6,400), under a percent, so 6% is past chance."""
+    r = np.random.default_rng(d)
+    n, nq = size_of(d)
+    make = (lambda *s: r.random(s, np.float32)) if kind == "positive" else (
+        lambda *s: r.standard_normal(s, np.float32))
+    base, q = make(n, d), make(nq, d)
+
+    def rms(batch):
+        ids, dist = engine.brute_force_knn(base, q[:batch], 50, metric)
+        b, x = base[ids[:128]].astype(np.float64), q[:128, None].astype(np.float64)
+        if metric == "l2":
+            want = ((b - x) ** 2).sum(2)
+        else:
+            want = (b * x).sum(2)
+            if metric == "cosine":
+                want /= np.linalg.norm(b, axis=2) * np.linalg.norm(x, axis=2)
+        return np.sqrt(((dist[:128] - want) ** 2).mean())
+
+    assert rms(nq) <= 1.06 * rms(128)
+
+
 @pytest.mark.parametrize("metric,d,eb,eq", [
     ("inner_product", 128, -54, -54), ("inner_product", 100, -70, -46), ("inner_product", 300, -60, -60),
     ("l2", 128, -54, -54), ("l2", 1536, -54.6, -54.6), ("l2", 1536, 44.5, -55), ("inner_product", 64, 30, -90),
