@@ -76,6 +76,12 @@ enum SplitFlags : uint32_t {
                         // they miss by more than 2^-25 of its length
   kSplitShort = 32,     // sums so short that the pieces' own error shows: only
                         // rows without lo pieces take them
+  // Integers (below 2^24), whose float32 sums are exact as long as they stay
+  // below 2^24 themselves:
+  kSplitFrac = 64,      // some value is none
+  kSplitCut = 128,      // some value is not hi + lo (its 24th bit)
+  kSplitFactors = 256,  // the float32 route divides dot products of the rows
+                        // themselves by their lengths (cosine by factors)
 };
 // Under L2 the lost 24th bits show in sums of few terms: rms error against 64
 // bits, pieces over float32 kernels, of near rows at 16 / 20 / 24 / 28 / 32
@@ -107,31 +113,34 @@ struct SplitState {
 // (no value has a lo piece: integers, rows that were binary16), 2 both.
 __device__ inline int split_route(const SplitState& s) {
   if (s.flags & kSplitRows32) return 0;
+  if (!(s.flags & kSplitFrac) && (s.flags & (kSplitCut | kSplitFactors))) return 0;
   const float error = s.lost[0] * s.top[1] + s.lost[1] * s.top[0];
   if (error > 0.0f && !(error <= 0x1p-24f * kSplitCap * (s.least[0] + s.least[1] - s.room))) return 0;
   if (!(s.flags & (kSplitBaseLow | kSplitQueryLow))) return 1;
   return s.flags & kSplitShort ? 0 : 2;
 }
 // The lo x lo products are at most 2^-22 of a value's product, 2^-25 of it on
-// average; they are formed when both sides have lo pieces and one side has
-// short values only (at most 16 bits), whose float32 sums can be exact, and for
-// rows of at most 64 values, whose sums have few other roundings.
+// average; they are formed when both sides have lo pieces and either one side
+// has short values only (at most 16 bits) or all values are integers -- sums that
+// can be exact in float32 --, and for rows of at most 64 values, whose sums have
+// few other roundings.
 __device__ inline bool split_low_low(uint32_t flags) {
   const uint32_t low = kSplitBaseLow | kSplitQueryLow, lng = kSplitBaseLong | kSplitQueryLong;
-  return (flags & low) == low && (flags & lng) != lng;
+  return (flags & low) == low && ((flags & lng) != lng || !(flags & kSplitFrac));
 }
 // The factor that takes a call's list scores to the rows' scores.
 __device__ inline float list_score_scale(const SplitState* st) {
   return st && split_route(*st) != 0 ? st->inv : 1.0f;
 }
 // Sets st: the scales from a sample of the rows (unit: rows of length at most
-// 1), no flags but kSplitShort.
+// 1) and the flags that need no pass over them.
 struct SplitInitArgs {
   const float* base;     // [n, ld], first d used
   const float* queries;  // [nq, ld]
   int64_t n, nq;
   int d, ld;
   int unit;
+  int factors;  // kSplitFactors (unit)
   int l2;
   SplitState* st;
 };

@@ -68,6 +68,7 @@ __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArg
   if (tid != 0) return;
   float sc[2];
   uint32_t flags = a.d < (a.l2 ? kSplitShortL2 : kSplitShortDot) ? kSplitShort : 0u;
+  if (a.unit) flags |= a.factors ? kSplitFactors : kSplitFrac;
   for (int side = 0; side < 2; ++side) {
     float x = 0.0f;
     for (int w = 0; w < kSampleThreads / 64; ++w) x = fmaxf(x, wmax[side][w]);
@@ -156,7 +157,8 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
   // (rows' errors past rounding and what they are held against, SplitState;
   // L2: both squared)
   float lost[4] = {0, 0, 0, 0}, mass[4] = {0, 0, 0, 0}, top = 0.0f;
-  uint32_t seen = 0;  // bit 0: a lo piece, 1: a long value, 2: out of range
+  // bit 0: a lo piece, 1: a long value, 2: out of range, 3: no integer, 4: a bit cut
+  uint32_t seen = 0;
   load_slab(0);
   for (int c0 = 0; c0 < a.out_ld; c0 += 32) {
     if constexpr (VEC) {
@@ -194,8 +196,13 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
       float x[8];
       *(floatx4*)&x[0] = *(const floatx4*)&sh[r * SS + c];
       *(floatx4*)&x[4] = *(const floatx4*)&sh[r * SS + c + 4];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (x[u] != rintf(x[u]) || !(fabsf(x[u]) < 0x1p24f)) seen |= 8u;
       if (a.unit_norms) {
-        const float nrm = sqrtf(a.unit_norms[row]);
+        const float nn = a.unit_norms[row];
+        if (!(nn < 0x1p24f)) seen |= 8u;  // (the sums may pass 2^24)
+        const float nrm = sqrtf(nn);
         const float den = nrm > 1e-30f ? nrm : 1e-30f;
 #pragma unroll
         for (int u = 0; u < 8; ++u) x[u] = x[u] / den;
@@ -216,6 +223,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
         // (exact; a value whose scaling underflowed is lost too)
         float err = fabsf(rest - (float)lv);
         if (xs == 0.0f && x[u] != 0.0f) err = 0x1p-25f;
+        if (err != 0.0f) seen |= 16u;
         if (!(err > ax * 0x1p-23f)) err = 0.0f;
         if (a.l2) {
           lost[j] = __builtin_fmaf(err, err, lost[j]);
@@ -289,7 +297,9 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
   }
   uint32_t any = (__builtin_amdgcn_ballot_w64(seen & 1u) ? (a.query ? kSplitQueryLow : kSplitBaseLow) : 0u) |
                  (__builtin_amdgcn_ballot_w64(seen & 2u) ? (a.query ? kSplitQueryLong : kSplitBaseLong) : 0u) |
-                 (__builtin_amdgcn_ballot_w64(seen & 4u) ? kSplitRows32 : 0u);
+                 (__builtin_amdgcn_ballot_w64(seen & 4u) ? kSplitRows32 : 0u) |
+                 (__builtin_amdgcn_ballot_w64(seen & 8u) ? kSplitFrac : 0u) |
+                 (__builtin_amdgcn_ballot_w64(seen & 16u) ? kSplitCut : 0u);
   // (read first: thousands of wavefronts would serialise on one word)
   if ((tid & 63) == 0 && any &&
       (any & ~__hip_atomic_load(&a.st->flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))

@@ -171,7 +171,31 @@ def test_small_values_decide(engine, oracle, metric, kind, d, scale):
     check(engine, oracle, base, q, 10, metric, False)
 
 
+@pytest.mark.parametrize("d", [128, 48, 131, 300])
+def test_integers_beside_long_ones(engine, oracle, d):
+    """Sums of 12-bit integers are exact, also where other rows and other
+    queries hold integers of 21 bits (and their own sums are not)."""
+    r = np.random.default_rng(d)
+    n, nq = size_of(d)
+    base, q = rows_of("wide ints", n, d, r), rows_of("wide ints", nq, d, r)
+    base[::8] *= 1001
+    q[np.setdiff1d(np.arange(0, nq, 8), sample(nq))] *= 1001
+    check(engine, oracle, base, q, 10, "l2", True)
+
+
+@pytest.mark.parametrize("d", [128, 300])
+def test_integers_of_24_bits(engine, oracle, d):
+    """Inner products with unit vectors are the rows' own 24-bit integers."""
+    r = np.random.default_rng(d)
+    n, nq = size_of(d)
+    base = r.integers(-(1 << 24) + 1, 1 << 24, (n, d)).astype(np.float32)
+    q = np.zeros((nq, d), np.float32)
+    q[np.arange(nq), r.integers(0, d, nq)] = 1
+    check(engine, oracle, base, q, 10, "inner_product", True)
+
+
 @pytest.mark.parametrize("kind,metric,d", [
+    ("bytes", "cosine", 320),
     ("float", "l2", 16), ("float", "l2", 24), ("float", "l2", 40), ("float", "l2", 128),
     ("positive", "l2", 200), ("float", "l2", 768), ("float", "inner_product", 9),
     ("float", "inner_product", 33), ("positive", "inner_product", 300), ("float", "cosine", 96),
@@ -179,16 +203,17 @@ def test_small_values_decide(engine, oracle, metric, kind, d, scale):
 ])
 def test_errors_no_larger_than_the_float32_kernels(engine, kind, metric, d):
     """Errors against 64 bits of a batch and of its first 128 queries alone,
-    which the float32 kernels take.  128 x 50 distances: their rms is known to
-    1 / sqrt(2 x 6,400), under a percent, so 6% is past chance."""
+    which the float32 kernels take.  128 x 16 distances: their rms is known to
+    1 / sqrt(2 x 2,048), 1.6%, so 6% is past chance."""
     r = np.random.default_rng(d)
     n, nq = size_of(d)
-    make = (lambda *s: r.random(s, np.float32)) if kind == "positive" else (
-        lambda *s: r.standard_normal(s, np.float32))
+    make = {"positive": lambda *s: r.random(s, np.float32),
+            "bytes": lambda *s: r.integers(0, 256, s).astype(np.float32),
+            "float": lambda *s: r.standard_normal(s, np.float32)}[kind]
     base, q = make(n, d), make(nq, d)
 
     def rms(batch):
-        ids, dist = engine.brute_force_knn(base, q[:batch], 50, metric)
+        ids, dist = engine.brute_force_knn(base, q[:batch], 16, metric)
         b, x = base[ids[:128]].astype(np.float64), q[:128, None].astype(np.float64)
         if metric == "l2":
             want = ((b - x) ** 2).sum(2)
