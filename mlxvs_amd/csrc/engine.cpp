@@ -627,9 +627,12 @@ bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, cons
     // 479 us (two pieces) and 1,217 us (float32), with their own 445 and
     // 1,016.  Batches that take the bounded merge lose more to the extra
     // lists (1,000 queries 0.97 -> 0.99)
+    // With k <= T larger batches keep to the lists that one wavefront merges
+    // (1M x 16, 10,000 queries: merge 0.53 -> 0.08 ms).
+    const int seg =
+        nq > kern::kBoundMergeQueries && k <= T ? 1024 / T : max_merge_segments(k, T);
     auto planned = [&](int bpc) {
-      return plan_splits(n, qblocks, k, T, 2, 2 * kern::kTileRows, device_slots(bpc), true,
-                         max_merge_segments(k, T));
+      return plan_splits(n, qblocks, k, T, 2, 2 * kern::kTileRows, device_slots(bpc), true, seg);
     };
     plan = planned(kern::fused_split_blocks_per_cu(sld, T));
     rows2 = plan.rows_per_split;

@@ -76,8 +76,7 @@ enum SplitFlags : uint32_t {
                         // they miss by more than 2^-25 of its length
   kSplitShort = 32,     // sums so short that the pieces' own error shows: only
                         // rows without lo pieces take them
-  // Integers (below 2^24), whose float32 sums are exact as long as they stay
-  // below 2^24 themselves:
+  // Integers, whose float32 sums are exact as long as they stay below 2^24:
   kSplitFrac = 64,      // some value is none
   kSplitCut = 128,      // some value is not hi + lo (its 24th bit)
   kSplitFactors = 256,  // the float32 route divides dot products of the rows

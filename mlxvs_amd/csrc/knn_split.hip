@@ -34,8 +34,10 @@ constexpr float kUnitScale = 32768.0f;
 // flight together (values scattered one by one took it 50 us, not 5).
 __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArgs a) {
   __shared__ float wmax[2][kSampleThreads / 64];
+  __shared__ int wlow[kSampleThreads / 64];
   const int tid = threadIdx.x;
   float m[2] = {0.0f, 0.0f};
+  bool low = false;  // a value of more than binary16's 11 bits: it has a lo piece
   if (!a.unit) {
     float v[2][kSamplePer];
 #pragma unroll
@@ -53,35 +55,48 @@ __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArg
 #pragma unroll
     for (int side = 0; side < 2; ++side)
 #pragma unroll
-      for (int i = 0; i < kSamplePer; ++i) m[side] = fmaxf(m[side], fabsf(v[side][i]));
+      for (int i = 0; i < kSamplePer; ++i) {
+        m[side] = fmaxf(m[side], fabsf(v[side][i]));
+        low |= (__float_as_uint(v[side][i]) & 0x1fffu) != 0u;
+      }
   }
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
     m[0] = fmaxf(m[0], __shfl_xor(m[0], o));
     m[1] = fmaxf(m[1], __shfl_xor(m[1], o));
   }
+  const int any_low = __builtin_amdgcn_ballot_w64(low) != 0;
   if ((tid & 63) == 0) {
     wmax[0][tid >> 6] = m[0];
     wmax[1][tid >> 6] = m[1];
+    wlow[tid >> 6] = any_low;
   }
   __syncthreads();
   if (tid != 0) return;
   float sc[2];
   uint32_t flags = a.d < (a.l2 ? kSplitShortL2 : kSplitShortDot) ? kSplitShort : 0u;
   if (a.unit) flags |= a.factors ? kSplitFactors : kSplitFrac;
+  for (int w = 0; w < kSampleThreads / 64; ++w)
+    if ((flags & kSplitShort) && wlow[w]) flags |= kSplitRows32;  // (at once: no pieces made)
+  bool large = !a.unit;  // both sides past 2^26: every value an integer, no sum exact
   for (int side = 0; side < 2; ++side) {
     float x = 0.0f;
     for (int w = 0; w < kSampleThreads / 64; ++w) x = fmaxf(x, wmax[side][w]);
     sc[side] = a.unit ? kUnitScale : 1.0f;
-    if (a.unit || x == 0.0f) continue;  // (a sample of zeros: the pass over all rows decides)
+    if (a.unit) continue;
+    if (x == 0.0f) {  // (a sample of zeros: the pass over all rows decides)
+      large = false;
+      continue;
+    }
     int e = kMaxSampleExp + 1;
     if (x < INFINITY) (void)frexpf(x, &e);  // x = f 2^e, f in [1/2, 1)
+    if (x < 0x1p26f) large = false;
     if (e < -kMaxSampleExp || e > kMaxSampleExp)
       flags |= kSplitRows32;
     else
       sc[side] = ldexpf(1.0f, kSampleExp + 1 - e);
   }
-  a.st->flags = flags;
+  a.st->flags = large ? flags | kSplitFrac : flags;
   a.st->sbase = sc[0];
   a.st->squery = sc[1];
   a.st->inv = 1.0f / (sc[0] * sc[1]);  // powers of two: exact
@@ -111,6 +126,17 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
   const SplitRowsArgs& a = blockIdx.x < na ? ab : aq;
   const int tid = threadIdx.x;
   const int64_t row0 = (int64_t)(blockIdx.x < na ? blockIdx.x : blockIdx.x - na) * 256;
+  // Once the rows are known to take the float32 route their pieces are not
+  // made, and only the norms are left to do (an outlier halfway through
+  // 500k x 768 rows, 700 queries: 5.12 -> 4.91 ms a call).
+  // (one thread's view for the whole workgroup, behind the loop's first barrier)
+  __shared__ bool s_rows32;
+  if (threadIdx.x == 0) {
+    const uint32_t known =
+        __hip_atomic_load(&a.st->flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_rows32 = (known & kSplitRows32) ||
+               ((known & kSplitShort) && (known & (kSplitBaseLow | kSplitQueryLow)));
+  }
   const float scale = a.query ? a.st->squery : a.st->sbase;
   const float seed_scale = a.st->sbase * a.st->squery;
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -157,8 +183,14 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
   // (rows' errors past rounding and what they are held against, SplitState;
   // L2: both squared)
   float lost[4] = {0, 0, 0, 0}, mass[4] = {0, 0, 0, 0}, top = 0.0f;
-  // bit 0: a lo piece, 1: a long value, 2: out of range, 3: no integer, 4: a bit cut
-  uint32_t seen = 0;
+  // (what the flags need is gathered as ORs of bits, one operation a value:
+  // with compares and selects instead the pass was bound by them, 500k x 768
+  // cosine, 2,000 queries 5.25 ms a call against 5.10)
+  uint32_t lowbits = 0;   // of the lo pieces, two a word
+  uint32_t cutbits = 0;   // of what the pieces leave out: bit 30 (2 and above) only if
+                          // a value is past binary16's range or not finite
+  uint32_t fracbits = 0;  // of the values' fractions
+  bool rows32_seen = false;
   load_slab(0);
   for (int c0 = 0; c0 < a.out_ld; c0 += 32) {
     if constexpr (VEC) {
@@ -179,6 +211,8 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
     }
     if (c0 + 32 < a.out_ld) load_slab(c0 + 32);
     __syncthreads();
+    const bool rows32 = s_rows32;
+    if (rows32 && !a.norm && !a.seed) return;
     if (a.norm || a.seed) {
 #pragma unroll
       for (int j4 = 0; j4 < 32; j4 += 4) {
@@ -192,16 +226,15 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
     for (int j = 0; j < 4; ++j) {
       const int r = (tid >> 2) + 64 * j, c = 8 * (tid & 3);
       const int64_t row = row0 + r;
-      if (row >= a.n || c0 + c >= a.out_ld) continue;
+      if (rows32 || row >= a.n || c0 + c >= a.out_ld) continue;
       float x[8];
       *(floatx4*)&x[0] = *(const floatx4*)&sh[r * SS + c];
       *(floatx4*)&x[4] = *(const floatx4*)&sh[r * SS + c + 4];
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (x[u] != rintf(x[u]) || !(fabsf(x[u]) < 0x1p24f)) seen |= 8u;
+      for (int u = 0; u < 8; ++u) fracbits |= __float_as_uint(__builtin_amdgcn_fractf(x[u]));
       if (a.unit_norms) {
         const float nn = a.unit_norms[row];
-        if (!(nn < 0x1p24f)) seen |= 8u;  // (the sums may pass 2^24)
+        if (!(nn < 0x1p24f)) fracbits = 1u;  // (the sums may pass 2^24)
         const float nrm = sqrtf(nn);
         const float den = nrm > 1e-30f ? nrm : 1e-30f;
 #pragma unroll
@@ -216,15 +249,11 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
         const _Float16 lv = (_Float16)rest;
         hi[u] = hv;
         lo[u] = lv;
-        const uint16_t lb = __builtin_bit_cast(uint16_t, lv);
-        if (!(ax <= 65504.0f)) seen |= 4u;
-        if (lb & 0x7fffu) seen |= 1u;
-        if ((lb & 0x003fu) && (lb & 0x7c00u)) seen |= 2u;
-        // (exact; a value whose scaling underflowed is lost too)
-        float err = fabsf(rest - (float)lv);
-        if (xs == 0.0f && x[u] != 0.0f) err = 0x1p-25f;
-        if (err != 0.0f) seen |= 16u;
-        if (!(err > ax * 0x1p-23f)) err = 0.0f;
+        float err = fabsf(rest - (float)lv);  // exact
+        if (scale < 1.0f && xs == 0.0f && x[u] != 0.0f) err = 0x1p-25f;  // (underflow)
+        cutbits |= __float_as_uint(err);
+        // (from 2^-2 on at most a last bit)
+        if (!(ax < 0.25f)) err = 0.0f;
         if (a.l2) {
           lost[j] = __builtin_fmaf(err, err, lost[j]);
           mass[j] = __builtin_fmaf(xs, xs, mass[j]);
@@ -233,6 +262,10 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
           mass[j] += fminf(ax, kSplitCap);
           top = fmaxf(top, ax);
         }
+      }
+      {
+        const u32x4 lw = __builtin_bit_cast(u32x4, lo);
+        lowbits |= (lw[0] | lw[1]) | (lw[2] | lw[3]);
       }
       // (interleaved: a run of hi pieces, then their lo pieces)
       constexpr int R = kTilePieceRun;
@@ -255,7 +288,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
     l += __shfl_xor(l, 2);
     m += __shfl_xor(m, 2);
     if (a.l2) {
-      if (l > 0x1p-50f * m) seen |= 4u;
+      if (l > 0x1p-50f * m) rows32_seen = true;
     } else {
       worst = fmaxf(worst, l);
       if (m > 0.0f || l > 0.0f) least = fminf(least, m);
@@ -267,7 +300,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
     const float nn = (s01 + s23) + (s45 + s67);
     // (squared norms near the ends of float32: their sums are not the
     // scaled ones)
-    if (!(nn < 0x1p100f) || (nn > 0.0f && nn < 0x1p-100f)) seen |= 4u;
+    if (!(nn < 0x1p100f) || (nn > 0.0f && nn < 0x1p-100f)) rows32_seen = true;
     const float half = nn > 0.0f ? -0.5f * nn : 0.0f;  // (+0, as row_norms_kernel)
     if (a.norm) a.norm[row0 + tid] = a.half_neg ? half : nn;
     if (a.seed) a.seed[row0 + tid] = half * seed_scale;
@@ -295,11 +328,14 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
         __hip_atomic_fetch_min(w, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
-  uint32_t any = (__builtin_amdgcn_ballot_w64(seen & 1u) ? (a.query ? kSplitQueryLow : kSplitBaseLow) : 0u) |
-                 (__builtin_amdgcn_ballot_w64(seen & 2u) ? (a.query ? kSplitQueryLong : kSplitBaseLong) : 0u) |
-                 (__builtin_amdgcn_ballot_w64(seen & 4u) ? kSplitRows32 : 0u) |
-                 (__builtin_amdgcn_ballot_w64(seen & 8u) ? kSplitFrac : 0u) |
-                 (__builtin_amdgcn_ballot_w64(seen & 16u) ? kSplitCut : 0u);
+  // (a lo piece's sign does not count; more than five bits of one: a value of
+  // more than 16)
+  auto any_of = [](bool b) { return __builtin_amdgcn_ballot_w64(b) != 0; };
+  const uint32_t any =
+      (any_of(lowbits & 0x7fff7fffu) ? (a.query ? kSplitQueryLow : kSplitBaseLow) : 0u) |
+      (any_of(lowbits & 0x003f003fu) ? (a.query ? kSplitQueryLong : kSplitBaseLong) : 0u) |
+      (any_of(rows32_seen || (cutbits & 0x40000000u)) ? kSplitRows32 : 0u) |
+      (any_of(fracbits & 0x7fffffffu) ? kSplitFrac : 0u) | (any_of(cutbits) ? kSplitCut : 0u);
   // (read first: thousands of wavefronts would serialise on one word)
   if ((tid & 63) == 0 && any &&
       (any & ~__hip_atomic_load(&a.st->flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
