@@ -81,6 +81,9 @@ enum SplitFlags : uint32_t {
   kSplitCut = 128,      // some value is not hi + lo (its 24th bit)
   kSplitFactors = 256,  // the float32 route divides dot products of the rows
                         // themselves by their lengths (cosine by factors)
+  // Inner products and cosine: some row loses more than rounding
+  kSplitBaseLoss = 512,
+  kSplitQueryLoss = 1024,
 };
 // Under L2 the lost 24th bits show in sums of few terms: rms error against 64
 // bits, pieces over float32 kernels, of near rows at 16 / 20 / 24 / 28 / 32
@@ -99,22 +102,27 @@ constexpr int kSplitShortL2 = 32, kSplitShortDot = 16;
 // most lost[base] top[query] + lost[query] top[base], lost the largest sum of a
 // row's errors past rounding.  Dense rows keep most of d C on both sides; sparse
 // or masked ones do not, and take the float32 route if they have such values.
-constexpr float kSplitCap = 48.0f;  // about 1/64 of the sample's largest value
+// C at 1/128 to 1/64 of the sample's largest value takes rows whose largest
+// value is 60 times their rms; short rows, whose sums have less room, need a
+// larger one.
+__host__ __device__ constexpr float split_cap(int d) { return d < 64 ? 64.0f : 32.0f; }
 struct SplitState {
   uint32_t flags;
   float sbase, squery;  // 2^s of the base rows and of the queries
   float inv;            // scores from the pieces times inv are the rows' scores
-  float room;           // d C
-  // [base, queries]; not negative, so their bits order as they do
-  float lost[2], top[2], least[2];
+  float cap, room;      // C, d C
+  float lost[2], top[2], least[2];  // [base, queries]
 };
 // Which kernel a call's rows take: 0 the float32 MFMA, 1 the hi pieces alone
 // (no value has a lo piece: integers, rows that were binary16), 2 both.
 __device__ inline int split_route(const SplitState& s) {
   if (s.flags & kSplitRows32) return 0;
   if (!(s.flags & kSplitFrac) && (s.flags & (kSplitCut | kSplitFactors))) return 0;
-  const float error = s.lost[0] * s.top[1] + s.lost[1] * s.top[0];
-  if (error > 0.0f && !(error <= 0x1p-24f * kSplitCap * (s.least[0] + s.least[1] - s.room))) return 0;
+  if (s.flags & (kSplitBaseLoss | kSplitQueryLoss)) {
+    const float error = (s.flags & kSplitBaseLoss ? s.lost[0] * s.top[1] : 0.0f) +
+                        (s.flags & kSplitQueryLoss ? s.lost[1] * s.top[0] : 0.0f);
+    if (!(error <= 0x1p-24f * s.cap * (s.least[0] + s.least[1] - s.room))) return 0;
+  }
   if (!(s.flags & (kSplitBaseLow | kSplitQueryLow))) return 1;
   return s.flags & kSplitShort ? 0 : 2;
 }

@@ -34,10 +34,13 @@ constexpr float kUnitScale = 32768.0f;
 // flight together (values scattered one by one took it 50 us, not 5).
 __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArgs a) {
   __shared__ float wmax[2][kSampleThreads / 64];
-  __shared__ int wlow[kSampleThreads / 64];
+  __shared__ uint32_t wflags[kSampleThreads / 64];
   const int tid = threadIdx.x;
   float m[2] = {0.0f, 0.0f};
-  bool low = false;  // a value of more than binary16's 11 bits: it has a lo piece
+  // what the sample's bits show already (values of more than 11 and 16 bits,
+  // values that two pieces do not hold, fractions): set here, the workgroups of
+  // the pass need not all report it at once
+  uint32_t shown = 0;
   if (!a.unit) {
     float v[2][kSamplePer];
 #pragma unroll
@@ -56,8 +59,13 @@ __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArg
     for (int side = 0; side < 2; ++side)
 #pragma unroll
       for (int i = 0; i < kSamplePer; ++i) {
-        m[side] = fmaxf(m[side], fabsf(v[side][i]));
-        low |= (__float_as_uint(v[side][i]) & 0x1fffu) != 0u;
+        const float x = v[side][i], f = __builtin_amdgcn_frexp_mantf(x);  // (+-[1/2, 1))
+        m[side] = fmaxf(m[side], fabsf(x));
+        if (__float_as_uint(x) & 0x1fffu) shown |= side ? kSplitQueryLow : kSplitBaseLow;
+        if (__float_as_uint(x) & 0xffu) shown |= side ? kSplitQueryLong : kSplitBaseLong;
+        const float rest = f - (float)(_Float16)f;
+        if (rest - (float)(_Float16)rest != 0.0f) shown |= kSplitCut;
+        if (__float_as_uint(__builtin_amdgcn_fractf(x)) & 0x7fffffffu) shown |= kSplitFrac;
       }
   }
 #pragma unroll
@@ -65,19 +73,19 @@ __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArg
     m[0] = fmaxf(m[0], __shfl_xor(m[0], o));
     m[1] = fmaxf(m[1], __shfl_xor(m[1], o));
   }
-  const int any_low = __builtin_amdgcn_ballot_w64(low) != 0;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) shown |= __shfl_xor(shown, o);
   if ((tid & 63) == 0) {
     wmax[0][tid >> 6] = m[0];
     wmax[1][tid >> 6] = m[1];
-    wlow[tid >> 6] = any_low;
+    wflags[tid >> 6] = shown;
   }
   __syncthreads();
   if (tid != 0) return;
   float sc[2];
   uint32_t flags = a.d < (a.l2 ? kSplitShortL2 : kSplitShortDot) ? kSplitShort : 0u;
   if (a.unit) flags |= a.factors ? kSplitFactors : kSplitFrac;
-  for (int w = 0; w < kSampleThreads / 64; ++w)
-    if ((flags & kSplitShort) && wlow[w]) flags |= kSplitRows32;  // (at once: no pieces made)
+  for (int w = 0; w < kSampleThreads / 64; ++w) flags |= wflags[w];
   bool large = !a.unit;  // both sides past 2^26: every value an integer, no sum exact
   for (int side = 0; side < 2; ++side) {
     float x = 0.0f;
@@ -100,10 +108,15 @@ __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArg
   a.st->sbase = sc[0];
   a.st->squery = sc[1];
   a.st->inv = 1.0f / (sc[0] * sc[1]);  // powers of two: exact
-  a.st->room = (float)a.d * kSplitCap;
+  // (the largest values, sums and losses that dense rows reach: only rows past
+  // them are reported)
+  const float cap = split_cap(a.d);
+  a.st->cap = cap;
+  a.st->room = (float)a.d * cap;
   for (int side = 0; side < 2; ++side) {
-    a.st->lost[side] = a.st->top[side] = 0.0f;
-    a.st->least[side] = INFINITY;
+    a.st->lost[side] = 0x1p-25f;
+    a.st->top[side] = 0x1p12f;
+    a.st->least[side] = 0.75f * (float)a.d * cap;
   }
 }
 
@@ -128,7 +141,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
   const int64_t row0 = (int64_t)(blockIdx.x < na ? blockIdx.x : blockIdx.x - na) * 256;
   // Once the rows are known to take the float32 route their pieces are not
   // made, and only the norms are left to do (an outlier halfway through
-  // 500k x 768 rows, 700 queries: 5.12 -> 4.91 ms a call).
+  // 500k x 768 rows, 700 queries: 5.15 -> 5.09 ms a call, float32 alone 4.69).
   // (one thread's view for the whole workgroup, behind the loop's first barrier)
   __shared__ bool s_rows32;
   if (threadIdx.x == 0) {
@@ -139,6 +152,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
   }
   const float scale = a.query ? a.st->squery : a.st->sbase;
   const float seed_scale = a.st->sbase * a.st->squery;
+  const float cap = a.st->cap;
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   constexpr int EPV = F16 ? 8 : 4;
   constexpr int VPR = 32 / EPV;
@@ -259,7 +273,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
           mass[j] = __builtin_fmaf(xs, xs, mass[j]);
         } else {
           lost[j] += err;
-          mass[j] += fminf(ax, kSplitCap);
+          mass[j] += fminf(ax, cap);
           top = fmaxf(top, ax);
         }
       }
@@ -305,6 +319,20 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
     if (a.norm) a.norm[row0 + tid] = a.half_neg ? half : nn;
     if (a.seed) a.seed[row0 + tid] = half * seed_scale;
   }
+  // One report a workgroup, and only of what the state does not show yet: the
+  // workgroups of a small call end together, and their atomics on one line
+  // would serialise (a wavefront's own values each: 76,775 x 78 rows, inner
+  // product, 125 us of preparation against 64).  (A lo piece's sign does not
+  // count; more than five bits of one: a value of more than 16.)
+  auto any_of = [](bool b) { return __builtin_amdgcn_ballot_w64(b) != 0; };
+  const uint32_t any =
+      (any_of(lowbits & 0x7fff7fffu) ? (a.query ? kSplitQueryLow : kSplitBaseLow) : 0u) |
+      (any_of(lowbits & 0x003f003fu) ? (a.query ? kSplitQueryLong : kSplitBaseLong) : 0u) |
+      (any_of(rows32_seen || (cutbits & 0x40000000u)) ? kSplitRows32 : 0u) |
+      (any_of(fracbits & 0x7fffffffu) ? kSplitFrac : 0u) | (any_of(cutbits) ? kSplitCut : 0u) |
+      (any_of(worst > 0.0f) ? (a.query ? kSplitQueryLoss : kSplitBaseLoss) : 0u);
+  __shared__ uint32_t rflags[4];
+  __shared__ float red[3][4];
   if (!a.l2) {
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -312,34 +340,33 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
       least = fminf(least, __shfl_xor(least, o));
       top = fmaxf(top, __shfl_xor(top, o));
     }
-    if ((tid & 63) == 0) {
-      // (read first, as the flags below)
-      auto raise = [](float* p, float v) {
-        unsigned* w = (unsigned*)p;
-        const unsigned b = __float_as_uint(v);
-        if (b > __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-          __hip_atomic_fetch_max(w, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      };
-      raise(&a.st->lost[a.query], worst);
-      raise(&a.st->top[a.query], top);
-      unsigned* w = (unsigned*)&a.st->least[a.query];
-      const unsigned b = __float_as_uint(least);
-      if (b < __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        __hip_atomic_fetch_min(w, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
   }
-  // (a lo piece's sign does not count; more than five bits of one: a value of
-  // more than 16)
-  auto any_of = [](bool b) { return __builtin_amdgcn_ballot_w64(b) != 0; };
-  const uint32_t any =
-      (any_of(lowbits & 0x7fff7fffu) ? (a.query ? kSplitQueryLow : kSplitBaseLow) : 0u) |
-      (any_of(lowbits & 0x003f003fu) ? (a.query ? kSplitQueryLong : kSplitBaseLong) : 0u) |
-      (any_of(rows32_seen || (cutbits & 0x40000000u)) ? kSplitRows32 : 0u) |
-      (any_of(fracbits & 0x7fffffffu) ? kSplitFrac : 0u) | (any_of(cutbits) ? kSplitCut : 0u);
-  // (read first: thousands of wavefronts would serialise on one word)
-  if ((tid & 63) == 0 && any &&
-      (any & ~__hip_atomic_load(&a.st->flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
-    __hip_atomic_fetch_or(&a.st->flags, any, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if ((tid & 63) == 0) {
+    rflags[tid >> 6] = any;
+    red[0][tid >> 6] = worst;
+    red[1][tid >> 6] = top;
+    red[2][tid >> 6] = least;
+  }
+  __syncthreads();
+  if (tid != 0) return;
+  SplitState* st = a.st;
+  auto word = [](const void* p) {
+    return __hip_atomic_load((const unsigned*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  const uint32_t all = (rflags[0] | rflags[1]) | (rflags[2] | rflags[3]);
+  if (all & ~word(&st->flags))
+    __hip_atomic_fetch_or(&st->flags, all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (a.l2) return;
+  // (not negative: their bits order as they do)
+  const unsigned w = __float_as_uint(fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3])));
+  const unsigned t = __float_as_uint(fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3])));
+  const unsigned l = __float_as_uint(fminf(fminf(red[2][0], red[2][1]), fminf(red[2][2], red[2][3])));
+  if (w > word(&st->lost[a.query]))
+    __hip_atomic_fetch_max((unsigned*)&st->lost[a.query], w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (t > word(&st->top[a.query]))
+    __hip_atomic_fetch_max((unsigned*)&st->top[a.query], t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (l < word(&st->least[a.query]))
+    __hip_atomic_fetch_min((unsigned*)&st->least[a.query], l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 }  // namespace
