@@ -1685,10 +1685,11 @@ void brute_force_knn_filtered_device(const Rows& base, const Rows& queries, int 
 
 namespace {
 // Rows of at most 128 columns: for batches a query per lane
-// (launch_pairwise_lanes) and the stream-list merges; else the split-parallel
-// scan over rows zero-padded to 32, 64 or 128 columns (each split's exact best
-// k), then the rank merge of each query's lists.  Wider rows (whose scan would
-// spill registers): a query per workgroup over all rows (launch_pairwise).
+// (launch_pairwise_lanes) and the stream-list merges, the queries that those
+// flag searched again by the scan; else the split-parallel scan alone, over rows
+// zero-padded to 32, 64 or 128 columns (each split's exact best k), then the rank
+// merge of each query's lists.  Wider rows (whose scan would spill registers): a
+// query per workgroup over all rows (launch_pairwise).
 constexpr int64_t kLanesMinQueries = 64;
 void pairwise_search(Session& ss, kern::PairwiseArgs pa) {
   Arena& ar = ss.arena();
@@ -1698,16 +1699,27 @@ void pairwise_search(Session& ss, kern::PairwiseArgs pa) {
   const int T = pa.k <= 10 ? 10 : 16;
   const int lld = round_up(d, 32);
   SplitPlan lanes;
+  bool strided = false;
   if (nq >= kLanesMinQueries && nq < (int64_t(1) << 31) &&
       kern::pairwise_lanes_supported(pa.metric, lld)) {
     // workgroups of up to four groups of 64 queries, two a CU
     const int64_t groups = (nq + 63) / 64, waves = std::min<int64_t>(4, groups);
     lanes = plan_splits(n, (groups + waves - 1) / waves, pa.k, T, 1, 1,
                         device_slots((int)(8 / waves)), false, max_merge_segments(pa.k, T));
-    if (lanes.ok && (lanes.rows_per_split + 8) * lld * 4 >= (int64_t(1) << 31)) lanes.ok = false;
+    strided = lanes.ok && (n + 8 * (int64_t)lanes.nsplit) * lld * 4 < (int64_t(1) << 31);
+    if (!strided && (lanes.rows_per_split + 8) * lld * 4 >= (int64_t(1) << 31)) lanes.ok = false;
   }
   const int ld = lanes.ok ? lld : d <= 32 ? 32 : d <= 64 ? 64 : d <= 128 ? 128 : 0;
-  if (ld == 0) {
+  // the scan: about four workgroups per CU slot in all, splits of whole
+  // 4,096-row chunks when there are enough rows
+  const int64_t want = std::max<int64_t>(8, 4 * device_slots(1) / nq);
+  int64_t rps = std::max<int64_t>(256, (n + want - 1) / want);
+  if (rps > 2048) rps = (rps + 4095) / 4096 * 4096;
+  const int64_t nsplit = ((n + rps - 1) / rps + 7) / 8 * 8;
+  const int64_t m = nsplit * pa.k;
+  const bool scan_ok = ld != 0 && (rps + 4096) * 4 * ld < (int64_t(1) << 31) &&
+                       (m + 4096) * 8 < (int64_t(1) << 31) && nsplit * nq < (int64_t(1) << 31);
+  if (!lanes.ok && !scan_ok) {
     launch(s, "pairwise", [&] { return kern::launch_pairwise(pa, s); });
     return;
   }
@@ -1722,11 +1734,16 @@ void pairwise_search(Session& ss, kern::PairwiseArgs pa) {
     pa.base = pb;
     pa.queries = pq;
   }
+  pa.ld = ld;
+  const bool redo = lanes.ok && T < pa.k;
+  const bool scans = scan_ok && (!lanes.ok || redo);
+  // (the scan's lists of a redo where the lanes' were)
+  pa.part = ar.take<uint64_t>((size_t)std::max(lanes.ok ? nq * lanes.nsplit * T : 0, scans ? nq * m : 0));
+  int* flags = redo ? ar.take<int>((size_t)nq) : nullptr;
   if (lanes.ok) {
-    pa.ld = ld;
     pa.rows_per_split = lanes.rows_per_split;
     pa.nsplit = lanes.nsplit;
-    pa.part = ar.take<uint64_t>((size_t)nq * lanes.nsplit * T);
+    pa.strided = strided;
     const int slots = kern::bound_slots_for(T);
     // (short splits end before a shared bound pays for its reads and atomics:
     // 100k x 128, 200 queries in 512 splits 0.47 ms with it)
@@ -1737,36 +1754,23 @@ void pairwise_search(Session& ss, kern::PairwiseArgs pa) {
     pa.pubj = bp.pubj;
     launch(s, "prep", [&] { return kern::launch_bounds_init(pa.gkey, nq, slots, bp.m, s); });
     launch(s, "pairwise", [&] { return kern::launch_pairwise_lanes(pa, T, s); });
-    int* flags = T < pa.k ? ar.take<int>((size_t)nq) : nullptr;
     merge_lists(ar, s, pa.part, lanes.nsplit, T, pa.k, nq, kern::kInnerProduct, nullptr, 1, pa.ids,
                 pa.dists, flags);
-    if (flags) {
-      kern::PairwiseArgs redo = unpadded;
-      redo.flags = flags;
-      launch(s, "redo", [&] { return kern::launch_pairwise(redo, s); });
+    if (!redo) return;
+    if (!scans) {
+      kern::PairwiseArgs all = unpadded;
+      all.flags = flags;
+      launch(s, "redo", [&] { return kern::launch_pairwise(all, s); });
+      return;
     }
-    return;
   }
-  // about four workgroups per CU slot in all, splits of whole 4,096-row
-  // chunks when there are enough rows
-  const int64_t want = std::max<int64_t>(8, 4 * device_slots(1) / nq);
-  int64_t rps = std::max<int64_t>(256, (n + want - 1) / want);
-  if (rps > 2048) rps = (rps + 4095) / 4096 * 4096;
-  const int64_t nsplit = ((n + rps - 1) / rps + 7) / 8 * 8;
-  const int64_t m = nsplit * pa.k;
-  if ((rps + 4096) * 4 * ld >= (int64_t(1) << 31) || (m + 4096) * 8 >= (int64_t(1) << 31) ||
-      nsplit * nq >= (int64_t(1) << 31)) {
-    launch(s, "pairwise", [&] { return kern::launch_pairwise(pa, s); });
-    return;
-  }
-  pa.ld = ld;
+  pa.flags = flags;
   pa.rows_per_split = rps;
   pa.nsplit = (int)nsplit;
-  pa.part = ar.take<uint64_t>((size_t)(nq * m));
   uint64_t* lev = ar.take<uint64_t>((size_t)std::max<int64_t>(1, kern::merge_ranks_scratch(nq, m, pa.k)));
-  launch(s, "pairwise", [&] { return kern::launch_pairwise_scan(pa, s); });
-  launch(s, "merge", [&] {
-    return kern::launch_merge_ranks(pa.part, nq, m, pa.k, lev, pa.ids, pa.dists, s);
+  launch(s, redo ? "redo" : "pairwise", [&] { return kern::launch_pairwise_scan(pa, s); });
+  launch(s, redo ? "redo" : "merge", [&] {
+    return kern::launch_merge_ranks(pa.part, nq, m, pa.k, lev, pa.ids, pa.dists, s, flags);
   });
 }
 }  // namespace

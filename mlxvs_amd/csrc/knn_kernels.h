@@ -650,23 +650,25 @@ struct PairwiseArgs {
   int32_t* ids;             // [nq][k] out
   float* dists;             // [nq][k] out
   // launch_pairwise_scan only: rows and queries [.][ld] fp32, 16-byte
-  // aligned, zero past d, ld one of 32, 64, 128; the splits' lists
+  // aligned, zero past d, ld one of 32, 64, 96, 128; the splits' lists
   int ld;
   int64_t rows_per_split;
   int nsplit;               // a multiple of 8
   uint64_t* part;           // [nq][nsplit][k] out
-  // launch_pairwise: only the queries with flags[q] != 0 (null: all)
+  // launch_pairwise and launch_pairwise_scan: only the queries with flags[q] !=
+  // 0 (null: all)
   const int* flags;
   // launch_pairwise_lanes: shared bounds (FusedArgs), slots of list length T
   uint32_t* gkey;
   int mslots;
   int pubj;
+  int strided;  // split s takes the rows s, s + nsplit, .. (else neighbouring rows)
 };
 hipError_t launch_pairwise(const PairwiseArgs& a, hipStream_t s);
 // Batches (a query per lane, knn_pairwise.hip): rows and queries [.][ld]
 // fp32, 16-byte aligned, zero past d, ld 32, 64, 96 or 128; stream lists of T
 // (10 or 16) ranks of -distance per split into part [nq][nsplit][T], for the
-// stream-list merges (k > T: with their flags, redone by launch_pairwise).
+// stream-list merges (k > T: with their flags, redone by launch_pairwise_scan).
 hipError_t launch_pairwise_lanes(const PairwiseArgs& a, int T, hipStream_t s);
 bool pairwise_lanes_supported(int metric, int ld);
 // The same distances for rows of at most 128 columns, split-parallel:
@@ -740,10 +742,11 @@ hipError_t launch_scan_float(const ScanFloatArgs& a, hipStream_t s);
 // results: ids, distances -score.  Groups of 4,096 ranks are reduced to
 // their best k on a workgroup each, level by level, into `scratch`
 // (merge_ranks_scratch(nq, m, k) ranks), until one workgroup per query
-// finishes.
+// finishes.  flags: only the queries with flags[q] != 0 (null: all).
 int64_t merge_ranks_scratch(int64_t nq, int64_t m, int k);
 hipError_t launch_merge_ranks(const uint64_t* part, int64_t nq, int64_t m, int k, uint64_t* scratch,
-                              int32_t* ids, float* dists, hipStream_t s);
+                              int32_t* ids, float* dists, hipStream_t s,
+                              const int* flags = nullptr);
 
 // Device scratch of the no-allocation entry point (scratch.hip): a fixed
 // array of kScratchBytes per GPU, held until the process ends.  Returns its

@@ -11,11 +11,12 @@
 // else, no lane sums to meet, no LDS, no barrier; rows arrive four ahead.
 // (Rows through scalar loads instead: the compiler gathered them in front of
 // their use and waited for each.)  Bound: VALU, 0.65 ms of L1's two operations
-// a value for that case; measured 0.86 ms (2.97 before).
+// a value for that case; measured 0.80 ms (2.97 before).
 //
 // A lane keeps the best T rows of its query (a sorted stream list, as the
 // fused kernels), and all splits of a query share a bound on its k-th best
-// (SharedBound).  Segments: one per split (part [nq][nsplit][T]).
+// (SharedBound).  With k > T the queries whose lists may have been too short are
+// searched again by the scan (launch_pairwise_scan under the merge's flags).  Segments: one per split (part [nq][nsplit][T]).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -44,8 +45,8 @@ __device__ __forceinline__ void each(F&& f) {
   }
 }
 
-// The same terms, and the same sums -- eight of every eighth value, met in
-// pairs --, precision and finish as MetricChunkScorer's.
+// The same terms, precision and finish as MetricChunkScorer's; the sums are
+// eight partial ones met in pairs as there (here each of every eighth value).
 template <int MET>
 struct LaneMetric {
   static constexpr int NA = MET == kPwCorrelation ? 3 : MET == kPwBrayCurtis ? 2 : 1;
@@ -111,9 +112,15 @@ __global__ __launch_bounds__(256, 2) void pairwise_lanes_kernel(PairwiseArgs a) 
   const int split = blockIdx.x % a.nsplit;
   const int64_t q = ((int64_t)(blockIdx.x / a.nsplit) * waves + wv) * 64 + lane;
   const bool qvalid = q < a.nq;
-  const int64_t r0 = min(a.n, (int64_t)split * a.rows_per_split);
-  const int64_t r1 = min(a.n, r0 + a.rows_per_split);
-  const int nrows = (int)(r1 - r0);
+  // the split's rows r0, r0 + row_step, ..: every nsplit-th row, so that rows
+  // side by side -- a dataset in the order of its groups -- do not meet in one
+  // split's list (100k x 128 rows in groups of 200, 1,000 queries, k = 50: with
+  // splits of neighbouring rows every query was flagged and the call took 38.9
+  // ms); neighbouring rows past 2^31 bytes of them
+  const int64_t row_step = a.strided ? a.nsplit : 1;
+  const int64_t r0 = min(a.n, a.strided ? (int64_t)split : (int64_t)split * a.rows_per_split);
+  const int64_t span = a.strided ? a.n - r0 : min(a.n - r0, a.rows_per_split);  // rows to the last's end
+  const int nrows = (int)((span + row_step - 1) / row_step);
 
   float qv[DQ];
   {
@@ -155,12 +162,13 @@ __global__ __launch_bounds__(256, 2) void pairwise_lanes_kernel(PairwiseArgs a) 
   // lane n of 16 holds values 64 v + 4 n .. + 3 of a row (the last 32 of an odd
   // count: 64 v + 2 n, + 1); rows past the split read zero
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(a.base + r0 * DQ), (short)0, nrows * DQ * 4, 0x00020000);
+      (void*)(a.base + r0 * DQ), (short)0, (int)(span * DQ * 4), 0x00020000);
+  const uint32_t step = (uint32_t)row_step * (DQ * 4);
   constexpr int V4 = DQ / 64, V2 = DQ % 64 / 32;
   constexpr int AHEAD = 4;
   uint32_t x[AHEAD][PER];
   auto load = [&](int r, uint32_t (&y)[PER]) {
-    const uint32_t off = (uint32_t)r * (DQ * 4);
+    const uint32_t off = (uint32_t)r * step;
 #pragma unroll
     for (int v = 0; v < V4; ++v) {
       const u32x4 t = __builtin_bit_cast(
@@ -216,11 +224,10 @@ __global__ __launch_bounds__(256, 2) void pairwise_lanes_kernel(PairwiseArgs a) 
     uint32_t key[AHEAD];
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u) key[u] = row_key(r + u, x[u]);
-    const int64_t row = r0 + r;
     if (fw) {
 #pragma unroll
       for (int u = 0; u < AHEAD; ++u) {
-        const int64_t j = min(row + u, r1 - 1);
+        const int64_t j = r0 + min(r + u, nrows - 1) * row_step;
         if (!((fw[j >> 5] >> (j & 31)) & 1u)) key[u] = 0u;
       }
     }
@@ -242,7 +249,7 @@ __global__ __launch_bounds__(256, 2) void pairwise_lanes_kernel(PairwiseArgs a) 
       for (int u = 0; u < AHEAD; ++u) {
         const bool pass = key[u] >= need;
         if (__builtin_amdgcn_ballot_w64(pass) == 0) continue;
-        stream_insert<T>(K, I, pass ? key[u] : 0u, (uint32_t)(row + u));
+        stream_insert<T>(K, I, pass ? key[u] : 0u, (uint32_t)(r0 + (r + u) * row_step));
         // (a later row needs a larger key than the last: equal ones lose)
         need = max(need, qvalid && K[T - 1] ? K[T - 1] + 1u : need);
       }
@@ -293,7 +300,8 @@ hipError_t launch_pairwise_lanes(const PairwiseArgs& a, int T, hipStream_t s) {
   if (!pairwise_lanes_supported(a.metric, a.ld) || (T != 10 && T != 16) || a.nsplit < 1 ||
       a.rows_per_split < 1 || (int64_t)a.nsplit * a.rows_per_split < a.n || a.d > a.ld ||
       (uintptr_t)a.base % 16 != 0 || (uintptr_t)a.queries % 16 != 0 || !a.part || !a.gkey ||
-      (a.rows_per_split + 8) * a.ld * 4 >= (int64_t(1) << 31) ||
+      (a.strided ? a.n + 8 * (int64_t)a.nsplit : a.rows_per_split + 8) * a.ld * 4 >=
+          (int64_t(1) << 31) ||
       (a.allow && a.allow_stride != 0 && a.allow_stride < (a.n + 31) / 32))
     return hipErrorInvalidValue;
   const int64_t groups = (a.nq + 63) / 64;

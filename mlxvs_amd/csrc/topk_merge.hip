@@ -1898,10 +1898,12 @@ __global__ __launch_bounds__(256) void scan_float_kernel(ScanFloatArgs a) {
 // distances = -score; -1 / +inf past the ranks there are).
 __global__ __launch_bounds__(256) void merge_ranks_kernel(const uint64_t* part, int64_t m,
                                                           int64_t w, int k, uint64_t* out,
-                                                          int32_t* ids, float* dists) {
+                                                          int32_t* ids, float* dists,
+                                                          const int* flags) {
   constexpr int NT = 256;
   __shared__ RowSelect sm;
   const int q = blockIdx.x, g = blockIdx.y;
+  if (flags && !flags[q]) return;
   const int64_t c0 = (int64_t)g * w, c1 = min(m, c0 + w);
   RankSource src{__builtin_amdgcn_make_buffer_rsrc((void*)(part + (int64_t)q * m), (short)0,
                                                    (int)(m * 8), 0x00020000)};
@@ -1950,6 +1952,7 @@ __global__ __launch_bounds__(256) void pairwise_scan_kernel(PairwiseArgs a) {
   const int xcd = (int)(id & 7);
   const int split = (int)(local / a.nq) * 8 + xcd;
   const int64_t q = local % a.nq;
+  if (a.flags && !a.flags[q]) return;
   const int64_t r0 = min(a.n, (int64_t)split * a.rows_per_split);
   const int64_t r1 = min(a.n, r0 + a.rows_per_split);
   constexpr int rowb = 128 * NL;
@@ -2090,6 +2093,7 @@ hipError_t launch_pairwise_scan(const PairwiseArgs& a, hipStream_t s) {
   switch (a.ld) {
     case 32: MLXVS_PWS_NL(1) break;
     case 64: MLXVS_PWS_NL(2) break;
+    case 96: MLXVS_PWS_NL(3) break;
     case 128: MLXVS_PWS_NL(4) break;
     default: return hipErrorInvalidValue;
   }
@@ -2156,7 +2160,7 @@ int64_t merge_ranks_scratch(int64_t nq, int64_t m, int k) {
 }
 
 hipError_t launch_merge_ranks(const uint64_t* part, int64_t nq, int64_t m, int k, uint64_t* scratch,
-                              int32_t* ids, float* dists, hipStream_t s) {
+                              int32_t* ids, float* dists, hipStream_t s, const int* flags) {
   if (nq <= 0) return hipSuccess;
   // byte offsets of the ranks (and of the last chunk past them) in 32 bits
   if (k < 1 || k > kMaxK || m < 0 || (m + 4096) * 8 >= (int64_t(1) << 31) ||
@@ -2166,7 +2170,7 @@ hipError_t launch_merge_ranks(const uint64_t* part, int64_t nq, int64_t m, int k
   while (m > 4096) {
     const int64_t groups = (m + 4095) / 4096;
     hipLaunchKernelGGL(merge_ranks_kernel, dim3((unsigned)nq, (unsigned)groups), dim3(256), 0, s,
-                       part, m, (int64_t)4096, k, scratch, nullptr, nullptr);
+                       part, m, (int64_t)4096, k, scratch, nullptr, nullptr, flags);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     part = scratch;
@@ -2174,7 +2178,7 @@ hipError_t launch_merge_ranks(const uint64_t* part, int64_t nq, int64_t m, int k
     m = groups * k;
   }
   hipLaunchKernelGGL(merge_ranks_kernel, dim3((unsigned)nq, 1), dim3(256), 0, s, part, m, m, k,
-                     nullptr, ids, dists);
+                     nullptr, ids, dists, flags);
   return hipGetLastError();
 }
 

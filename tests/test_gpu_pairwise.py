@@ -162,8 +162,8 @@ def test_pairwise_batches_float(engine, oracle, metric):
 
 
 def test_pairwise_batches_neighbours_side_by_side(engine, oracle):
-    # a query's 60 nearest rows lie next to each other: more than a list of a
-    # split holds, so the query is flagged and redone over all rows
+    # a query's 60 nearest rows lie next to each other: more than a list of one
+    # split would hold if splits were neighbouring rows
     rng = np.random.default_rng(4)
     b = (rng.random((40_000, 16)) * 100 + 50).astype(np.float32)
     q = np.zeros((70, 16), np.float32)
@@ -175,3 +175,26 @@ def test_pairwise_batches_neighbours_side_by_side(engine, oracle):
     bm = rng.random((70, 40_000)) < 0.3
     ids, dist = engine.pairwise_knn(b, q, 10, "cityblock", bitmap=bm)
     recall_check(oracle, ids, dist, b, q, 10, "cityblock", allowed=bm)
+
+
+@pytest.mark.parametrize("d,metric", [(16, "cityblock"), (80, "chebyshev"), (128, "cityblock"), (40, "hamming")])
+def test_pairwise_batches_redo(engine, oracle, d, metric):
+    # neighbours at a stride, one per query: where it is the split count (or
+    # shares a large factor with it) they meet in few splits' lists of 16, and
+    # the query goes through the scan again; the others' results stay
+    rng = np.random.default_rng(d)
+    n, k = 40_000, 60
+    strides = list(range(480, 620)) + [250, 256, 500, 512, 625, 640, 750, 768, 800, 1000, 1024, 1250]
+    nq = len(strides)
+    b = rng.integers(50, 200, (n, d)).astype(np.float32)
+    q = np.zeros((nq, d), np.float32)
+    at = rng.permutation(d)[:2]
+    for i, st in enumerate(strides):
+        q[i, :] = 3 * i - 300
+        rows = np.arange(i, n, st)[:k + 5]
+        b[rows] = q[i] if metric == "hamming" else q[i] + rng.integers(0, 2, (len(rows), d))
+        b[np.ix_(rows, at)] += rng.integers(0, 4, (len(rows), 2))
+    ids, dist = engine.pairwise_knn(b, q, k, metric)
+    oid, odist = oracle.pairwise_knn(q, b, k, metric)
+    assert np.array_equal(ids, oid)
+    assert np.array_equal(dist, odist.astype(np.float32))
