@@ -66,6 +66,11 @@ std::map<std::string, std::pair<int64_t, double>> g_prof_totals;
 // no-allocation entry point).
 thread_local bool t_dry = false;
 thread_local bool t_noprof = false;
+struct DryRun {
+  const bool was = t_dry;
+  DryRun() { t_dry = true; }
+  ~DryRun() { t_dry = was; }
+};
 
 template <typename F>
 void launch(hipStream_t s, const char* stage, F&& f) {
@@ -134,6 +139,12 @@ class Arena {
     chunks_.push_back({base, size, 0});
   }
   ~Arena() = default;  // device memory is reclaimed at process exit
+  // Counts what a dry run takes and holds no memory.
+  static Arena counting() {
+    Arena a;
+    a.chunks_.push_back({(char*)(uintptr_t)4096, ~size_t(0) >> 1, 0});
+    return a;
+  }
 
   bool fixed() const { return fixed_; }
   size_t used() const { return chunks_.empty() ? 0 : chunks_[0].used; }
@@ -175,8 +186,8 @@ class Arena {
     return p;
   }
 
-  // Whether `bytes` more can be taken (in pieces of any size) without an
-  // allocation that fails: room is made now.  A fixed arena answers no.
+  // Whether `bytes` more (as used() counts them) can be taken without another
+  // allocation: room is made now.  A fixed arena answers no.
   bool reserve(size_t bytes) {
     if (fixed_) return false;
     for (const auto& c : chunks_)
@@ -196,11 +207,17 @@ class Arena {
     check_hip(hipEventRecord(done_, s), "hipEventRecord");
     if (chunks_.size() > 1) {
       check_hip(hipEventSynchronize(done_), "hipEventSynchronize");
-      size_t total = 0;
+      size_t total = 0, largest = 0, used = 0;
       for (auto& c : chunks_) {
         total += c.size;
+        largest = std::max(largest, c.size);
+        used += c.used;
         (void)hipFree(c.ptr);
       }
+      // (large arenas: what this call took and an eighth, not all that the
+      // chunks beside each other came to)
+      if (total > (size_t(256) << 20))
+        total = std::max(largest, std::min(total, used + used / 8));
       chunks_.clear();
       char* p = nullptr;
       check_hip(hipMalloc(&p, total), "hipMalloc (workspace)");
@@ -566,8 +583,9 @@ constexpr double kTileMinWork = 1.6e10;  // n nq d
 // queries 0.53 / 0.52; 1M x 1536 x 10,000 35.2 / 28.6.
 constexpr int64_t kTileF16MinQueries = 384;
 constexpr double kTileF16MinWork = 1.5e11;  // n nq d
-// Device memory for the pieces and the operands of the float32 route: as
-// much as the rows take, so large collections keep the float32 kernels.
+// The workspace of such a call, above all the pieces (as much as the rows take)
+// and the operands of the float32 route: large collections keep the float32
+// kernels.
 constexpr size_t kSplitMaxBytes = size_t(16) << 30;
 
 // The deep rows' tile kernel for nq queries: its list length and split plan
@@ -591,7 +609,6 @@ int list_len_tile(int k, bool allow) { return allow || k > 10 ? 16 : 10; }
 // `allow`: prefilter words as FusedArgs.
 bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, const uint32_t* allow,
                      int64_t allow_stride, int32_t* ids, float* dists) {
-  Arena& ar = ss.arena();
   hipStream_t s = ss.stream();
   const int64_t n = in.n, nq = in.nq;
   const int d = in.d;
@@ -601,7 +618,7 @@ bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, cons
   // values) or the deep kernel
   const bool tile = round_up(d, 8) > kern::kMaxSplitDim;
   const double work = (double)n * (double)nq * std::max(d, 32);
-  if (ar.fixed() || (in.f16 && !cosine) || nq >= (int64_t(1) << 31) ||
+  if (ss.arena().fixed() || (in.f16 && !cosine) || nq >= (int64_t(1) << 31) ||
       nq < (tile ? kTileMinQueries : kSplitMinQueries) ||
       work < (tile ? kTileMinWork : kSplitMinWork))
     return false;
@@ -653,102 +670,111 @@ bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, cons
   const bool cos_factors = cosine && !in.f16 && deep32 && k <= 16 && !allow;
   const bool in_place = (!cosine || cos_factors) && (uintptr_t)in.base % 16 == 0 &&
                         (uintptr_t)in.queries % 16 == 0 && d % vmul32 == 0;
-  const size_t rows_all = (size_t)(n + nq);
-  const size_t bytes = rows_all * ((size_t)sld * 4 + (in_place ? 0 : (size_t)ld32 * 4)) + (64u << 10);
-  if (bytes > kSplitMaxBytes || !ar.reserve(bytes)) return false;
 
-  // (interleaved pieces: the hi arrays hold both)
-  uint16_t* bhi = ar.take<uint16_t>((size_t)n * sld * (tile ? 2 : 1));
-  uint16_t* blo = tile ? nullptr : ar.take<uint16_t>((size_t)n * sld);
-  uint16_t* qhi = ar.take<uint16_t>((size_t)nq * sld * (tile ? 2 : 1));
-  uint16_t* qlo = tile ? nullptr : ar.take<uint16_t>((size_t)nq * sld);
-  auto* st = ar.take<kern::SplitState>(1);
-  const int f16 = in.f16 ? 1 : 0;
-  const void *kbase = in.base, *kq = in.queries;
-  float *bnorm = nullptr, *qnorm = nullptr, *seed = nullptr;
-  float *ubn = nullptr, *uqn = nullptr;  // cosine: |b|^2, |q|^2
-  kern::SplitInitArgs si{(const float*)in.base, (const float*)in.queries, n, nq, d, d,
-                         cosine ? 1 : 0, cos_factors ? 1 : 0, l2, st};
-  launch(s, "prep", [&] { return kern::launch_split_init(si, s); });
-  if (cosine) {
-    ubn = ar.take<float>((size_t)n);
-    uqn = ar.take<float>((size_t)nq);
-    kern::PrepArgs pb{in.base, n, d, d, f16, ubn, nullptr, nullptr, 0, 0};
-    kern::PrepArgs pq{in.queries, nq, d, d, f16, uqn, nullptr, nullptr, 0, 0};
-    launch(s, "prep", [&] { return kern::launch_norms_pair(pb, pq, {}, s); });
-  }
-  if (l2) {
-    bnorm = ar.take<float>((size_t)n);
-    seed = ar.take<float>((size_t)n);
-    qnorm = ar.take<float>((size_t)nq);
-  }
-  kern::SplitRowsArgs sb{in.base, n, d, d, f16, ubn, bnorm, 1, seed, bhi, blo, sld, 0, l2, st};
-  kern::SplitRowsArgs sq{in.queries, nq, d, d, f16, uqn, qnorm, 0, nullptr, qhi, qlo, sld, 1, l2, st};
-  const int nseg = lanes * plan.nsplit;
-  const int slots = kern::bound_slots_for(T);
-  const BoundPlan bp = shared_bound(k, T, slots, nseg);
-  uint32_t* gkey = ar.take<uint32_t>((size_t)nq * slots);
-  const kern::BoundsInit bi{gkey, nq * slots, slots, bp.m};
-  launch(s, "prep", [&] { return kern::launch_split_rows(sb, sq, bi, s); });
-  if (!in_place) {
-    float* pb = ar.take<float>((size_t)n * ld32);
-    float* pq = ar.take<float>((size_t)nq * ld32);
-    const float* un = cos_factors ? nullptr : ubn;
-    const float* uq = cos_factors ? nullptr : uqn;
-    kern::PrepArgs tb{in.base, n, d, d, f16, nullptr, un, pb, ld32, 0};
-    kern::PrepArgs tq{in.queries, nq, d, d, f16, nullptr, uq, pq, ld32, 0};
-    // (the redo of cosine queries reads the unit rows on every route)
-    if (!(cosine && k > T)) tb.split = tq.split = st;
-    launch(s, "prep", [&] { return kern::launch_transform(tb, s); });
-    launch(s, "prep", [&] { return kern::launch_transform(tq, s); });
-    kbase = pb;
-    kq = pq;
-  }
+  // The whole call, over the arena it is given: first counted, so that either
+  // all of it has room before anything is enqueued or the float32 kernels run
+  // in less.
+  auto run = [&](Arena& ar) {
+    // (interleaved pieces: the hi arrays hold both)
+    uint16_t* bhi = ar.take<uint16_t>((size_t)n * sld * (tile ? 2 : 1));
+    uint16_t* blo = tile ? nullptr : ar.take<uint16_t>((size_t)n * sld);
+    uint16_t* qhi = ar.take<uint16_t>((size_t)nq * sld * (tile ? 2 : 1));
+    uint16_t* qlo = tile ? nullptr : ar.take<uint16_t>((size_t)nq * sld);
+    auto* st = ar.take<kern::SplitState>(1);
+    const int f16 = in.f16 ? 1 : 0;
+    const void *kbase = in.base, *kq = in.queries;
+    float *bnorm = nullptr, *qnorm = nullptr, *seed = nullptr;
+    float *ubn = nullptr, *uqn = nullptr;  // cosine: |b|^2, |q|^2
+    kern::SplitInitArgs si{(const float*)in.base, (const float*)in.queries, n, nq, d, d,
+                           cosine ? 1 : 0, cos_factors ? 1 : 0, l2, st};
+    launch(s, "prep", [&] { return kern::launch_split_init(si, s); });
+    if (cosine) {
+      ubn = ar.take<float>((size_t)n);
+      uqn = ar.take<float>((size_t)nq);
+      kern::PrepArgs pb{in.base, n, d, d, f16, ubn, nullptr, nullptr, 0, 0};
+      kern::PrepArgs pq{in.queries, nq, d, d, f16, uqn, nullptr, nullptr, 0, 0};
+      launch(s, "prep", [&] { return kern::launch_norms_pair(pb, pq, {}, s); });
+    }
+    if (l2) {
+      bnorm = ar.take<float>((size_t)n);
+      seed = ar.take<float>((size_t)n);
+      qnorm = ar.take<float>((size_t)nq);
+    }
+    kern::SplitRowsArgs sb{in.base, n, d, d, f16, ubn, bnorm, 1, seed, bhi, blo, sld, 0, l2, st};
+    kern::SplitRowsArgs sq{in.queries, nq, d, d, f16, uqn, qnorm, 0, nullptr, qhi, qlo, sld, 1, l2, st};
+    const int nseg = lanes * plan.nsplit;
+    const int slots = kern::bound_slots_for(T);
+    const BoundPlan bp = shared_bound(k, T, slots, nseg);
+    uint32_t* gkey = ar.take<uint32_t>((size_t)nq * slots);
+    const kern::BoundsInit bi{gkey, nq * slots, slots, bp.m};
+    launch(s, "prep", [&] { return kern::launch_split_rows(sb, sq, bi, s); });
+    if (!in_place) {
+      float* pb = ar.take<float>((size_t)n * ld32);
+      float* pq = ar.take<float>((size_t)nq * ld32);
+      const float* un = cos_factors ? nullptr : ubn;
+      const float* uq = cos_factors ? nullptr : uqn;
+      kern::PrepArgs tb{in.base, n, d, d, f16, nullptr, un, pb, ld32, 0};
+      kern::PrepArgs tq{in.queries, nq, d, d, f16, nullptr, uq, pq, ld32, 0};
+      // (the redo of cosine queries reads the unit rows on every route)
+      if (!(cosine && k > T)) tb.split = tq.split = st;
+      launch(s, "prep", [&] { return kern::launch_transform(tb, s); });
+      launch(s, "prep", [&] { return kern::launch_transform(tq, s); });
+      kbase = pb;
+      kq = pq;
+    }
 
-  uint64_t* part = ar.take<uint64_t>((size_t)nq * nseg * T);
-  // one launch per route: all but the one that the rows take return at once
-  kern::FusedArgs fa{bhi, qhi, seed, n, (int)nq, sld, cosine ? kern::kInnerProduct : metric,
-                     plan.rows_per_split, plan.nsplit, T, k, part, gkey, bp.m, bp.pubj,
-                     (int)qblocks, plan.xcd ? (tile ? 2 : 1) : 0};
-  fa.allow = allow;
-  fa.allow_stride = allow_stride;
-  fa.split = st;
-  fa.base_lo = blo;
-  fa.queries_lo = qlo;
-  if (tile) {
-    fa.route = 1;  // (both piece routes)
-    fa.nqb = (int)((nq + kern::kTileQueries - 1) / kern::kTileQueries);
-    launch(s, "fused_tile", [&] { return kern::launch_tile(fa, true, s); });
-  } else {
-    fa.route = 1;
-    launch(s, "fused_hi", [&] { return kern::launch_fused_f16(fa, s); });
-    fa.route = 2;
-    fa.rows_per_split = rows2;
-    launch(s, "fused_split", [&] { return kern::launch_fused_split(fa, s); });
+    uint64_t* part = ar.take<uint64_t>((size_t)nq * nseg * T);
+    // one launch per route: all but the one that the rows take return at once
+    kern::FusedArgs fa{bhi, qhi, seed, n, (int)nq, sld, cosine ? kern::kInnerProduct : metric,
+                       plan.rows_per_split, plan.nsplit, T, k, part, gkey, bp.m, bp.pubj,
+                       (int)qblocks, plan.xcd ? (tile ? 2 : 1) : 0};
+    fa.allow = allow;
+    fa.allow_stride = allow_stride;
+    fa.split = st;
+    fa.base_lo = blo;
+    fa.queries_lo = qlo;
+    if (tile) {
+      fa.route = 1;  // (both piece routes)
+      fa.nqb = (int)((nq + kern::kTileQueries - 1) / kern::kTileQueries);
+      launch(s, "fused_tile", [&] { return kern::launch_tile(fa, true, s); });
+    } else {
+      fa.route = 1;
+      launch(s, "fused_hi", [&] { return kern::launch_fused_f16(fa, s); });
+      fa.route = 2;
+      fa.rows_per_split = rows2;
+      launch(s, "fused_split", [&] { return kern::launch_fused_split(fa, s); });
+    }
+    // (its two segments a split: the same lists over finer splits)
+    fa.route = 0;
+    fa.nqb = (int)qblocks;
+    fa.base = kbase;
+    fa.queries = kq;
+    fa.bnorm = cos_factors ? ubn : bnorm;
+    fa.qnorm = cos_factors ? uqn : nullptr;
+    if (cos_factors) fa.metric = kern::kCosine;
+    fa.ld = ld32;
+    fa.nsplit = plan.nsplit * (lanes / 2);
+    fa.rows_per_split = tile ? plan.rows_per_split / (lanes / 2) : rows2;
+    if (deep32)
+      launch(s, "fused_deep", [&] { return kern::launch_deep(fa, false, s); });
+    else
+      launch(s, "fused_f32", [&] { return kern::launch_fused_f32(fa, s); });
+    int* flags = T < k ? ar.take<int>((size_t)nq) : nullptr;
+    merge_lists(ar, s, part, nseg, T, k, nq, metric, qnorm, 0, ids, dists, flags, st);
+    if (T >= k) return;
+    kern::RedoArgs ra{cosine ? kbase : in.base, cosine ? kq : in.queries, bnorm, qnorm, flags, n,
+                      (int)nq, cosine ? ld32 : d, d, 0, 0, metric, 0, k, ids, dists};
+    ra.allow = allow;
+    ra.allow_stride = allow_stride;
+    launch(s, "redo", [&] { return kern::launch_redo(ra, s); });
+  };
+  Arena need = Arena::counting();
+  {
+    DryRun dry;
+    run(need);
   }
-  // (its two segments a split: the same lists over finer splits)
-  fa.route = 0;
-  fa.nqb = (int)qblocks;
-  fa.base = kbase;
-  fa.queries = kq;
-  fa.bnorm = cos_factors ? ubn : bnorm;
-  fa.qnorm = cos_factors ? uqn : nullptr;
-  if (cos_factors) fa.metric = kern::kCosine;
-  fa.ld = ld32;
-  fa.nsplit = plan.nsplit * (lanes / 2);
-  fa.rows_per_split = tile ? plan.rows_per_split / (lanes / 2) : rows2;
-  if (deep32)
-    launch(s, "fused_deep", [&] { return kern::launch_deep(fa, false, s); });
-  else
-    launch(s, "fused_f32", [&] { return kern::launch_fused_f32(fa, s); });
-  int* flags = T < k ? ar.take<int>((size_t)nq) : nullptr;
-  merge_lists(ar, s, part, nseg, T, k, nq, metric, qnorm, 0, ids, dists, flags, st);
-  if (T >= k) return true;
-  kern::RedoArgs ra{cosine ? kbase : in.base, cosine ? kq : in.queries, bnorm, qnorm, flags, n,
-                    (int)nq, cosine ? ld32 : d, d, 0, 0, metric, 0, k, ids, dists};
-  ra.allow = allow;
-  ra.allow_stride = allow_stride;
-  launch(s, "redo", [&] { return kern::launch_redo(ra, s); });
+  if (need.used() > kSplitMaxBytes || !ss.arena().reserve(need.used())) return false;
+  run(ss.arena());
   return true;
 }
 
@@ -1359,63 +1385,70 @@ void ivf_search(Session& ss, const float* centers, int64_t lists, const float* d
     // float32 against pieces: 10,000 queries 1.02 / 0.67 (0.77) ms a call,
     // 5,000 0.77 / 0.62 (0.69); 2,500 would not gain
     const int sld = round_up(d, 8);
-    const size_t piece_bytes = (size_t)(n + nq) * sld * 4 + (64u << 10);
-    const bool split = !ar.fixed() && n > 0 && kern::fused_split_supported(sld, T) &&
-                       npairs >= kIvfSplitUses * (double)lists &&
-                       npairs * (double)avg_rows * std::max(d, 32) >= kSplitMinWork &&
-                       piece_bytes <= kSplitMaxBytes && ar.reserve(piece_bytes);
-    if (!split) base_norms(need);
-    const int nseg = 2 * P * rs;
-    // every (query, probe) pair is in one item, so every segment is written
-    uint64_t* part = ar.take<uint64_t>((size_t)nq * nseg * T);
-    const int slots_n = kern::bound_slots_for(T);
-    // one slot: the items are short (a list's rows), and a tile's read of
-    // more slots costs more than the tighter bound saves
-    const BoundPlan bp = shared_bound(k, T, 1, nseg);
-    uint32_t* gkey = ar.take<uint32_t>((size_t)nq * slots_n);
-    kern::FusedArgs fa{kd, kq, bnorm, n, (int)nq, ld, km, 0, rs, T, k, part, gkey, bp.m, bp.pubj,
-                       0, 0, ditems, dpairs, offsets, dslots, P, (int)max_items, nullptr, 0, 0,
-                       nitems};
-    kern::SplitState* st = nullptr;
-    if (split) {
-      st = ar.take<kern::SplitState>(1);
-      uint16_t* bhi = ar.take<uint16_t>((size_t)n * sld);
-      uint16_t* blo = ar.take<uint16_t>((size_t)n * sld);
-      uint16_t* qhi = ar.take<uint16_t>((size_t)nq * sld);
-      uint16_t* qlo = ar.take<uint16_t>((size_t)nq * sld);
-      float* seed = l2 ? ar.take<float>((size_t)n) : nullptr;
-      const kern::SplitInitArgs si{kd, kq, n, nq, d, ld, 0, 0, l2, st};
-      launch(s, "prep", [&] { return kern::launch_split_init(si, s); });
-      const kern::SplitRowsArgs sb{kd, n, ld, ld, 0, nullptr, bnorm, 1, seed, bhi, blo, sld, 0, l2, st};
-      const kern::SplitRowsArgs sq{kq, nq, ld, ld, 0, nullptr, nullptr, 0, nullptr, qhi, qlo, sld,
-                                   1, l2, st};
-      const kern::BoundsInit bi{gkey, nq * slots_n, slots_n, bp.m};
-      launch(s, "prep", [&] { return kern::launch_split_rows(sb, sq, bi, s); });
-      kern::FusedArgs fp = fa;
-      fp.base = bhi;
-      fp.queries = qhi;
-      fp.base_lo = blo;
-      fp.queries_lo = qlo;
-      fp.bnorm = seed;
-      fp.ld = sld;
-      fp.split = st;
-      for (fp.route = 1; fp.route <= 2; ++fp.route)
-        launch(s, fp.route == 1 ? "ivf_scan_hi" : "ivf_scan_split",
-               [&] { return kern::launch_ivf_select_pieces(fp, s); });
-      fa.split = st;
-      fa.route = 0;
-    } else {
-      launch(s, "prep", [&] { return kern::launch_bounds_init(gkey, nq, slots_n, bp.m, s); });
+    const bool pays = !ar.fixed() && n > 0 && kern::fused_split_supported(sld, T) &&
+                      npairs >= kIvfSplitUses * (double)lists &&
+                      npairs * (double)avg_rows * std::max(d, 32) >= kSplitMinWork;
+    auto scan = [&](Arena& ar, bool split) {
+      if (!split) base_norms(need);
+      const int nseg = 2 * P * rs;
+      // every (query, probe) pair is in one item, so every segment is written
+      uint64_t* part = ar.take<uint64_t>((size_t)nq * nseg * T);
+      const int slots_n = kern::bound_slots_for(T);
+      // one slot: the items are short (a list's rows), and a tile's read of
+      // more slots costs more than the tighter bound saves
+      const BoundPlan bp = shared_bound(k, T, 1, nseg);
+      uint32_t* gkey = ar.take<uint32_t>((size_t)nq * slots_n);
+      kern::FusedArgs fa{kd, kq, bnorm, n, (int)nq, ld, km, 0, rs, T, k, part, gkey, bp.m, bp.pubj,
+                         0, 0, ditems, dpairs, offsets, dslots, P, (int)max_items, nullptr, 0, 0,
+                         nitems};
+      kern::SplitState* st = nullptr;
+      if (split) {
+        st = ar.take<kern::SplitState>(1);
+        uint16_t* bhi = ar.take<uint16_t>((size_t)n * sld);
+        uint16_t* blo = ar.take<uint16_t>((size_t)n * sld);
+        uint16_t* qhi = ar.take<uint16_t>((size_t)nq * sld);
+        uint16_t* qlo = ar.take<uint16_t>((size_t)nq * sld);
+        float* seed = l2 ? ar.take<float>((size_t)n) : nullptr;
+        const kern::SplitInitArgs si{kd, kq, n, nq, d, ld, 0, 0, l2, st};
+        launch(s, "prep", [&] { return kern::launch_split_init(si, s); });
+        const kern::SplitRowsArgs sb{kd, n, ld, ld, 0, nullptr, bnorm, 1, seed, bhi, blo, sld, 0, l2, st};
+        const kern::SplitRowsArgs sq{kq, nq, ld, ld, 0, nullptr, nullptr, 0, nullptr, qhi, qlo, sld,
+                                     1, l2, st};
+        const kern::BoundsInit bi{gkey, nq * slots_n, slots_n, bp.m};
+        launch(s, "prep", [&] { return kern::launch_split_rows(sb, sq, bi, s); });
+        kern::FusedArgs fp = fa;
+        fp.base = bhi;
+        fp.queries = qhi;
+        fp.base_lo = blo;
+        fp.queries_lo = qlo;
+        fp.bnorm = seed;
+        fp.ld = sld;
+        fp.split = st;
+        for (fp.route = 1; fp.route <= 2; ++fp.route)
+          launch(s, fp.route == 1 ? "ivf_scan_hi" : "ivf_scan_split",
+                 [&] { return kern::launch_ivf_select_pieces(fp, s); });
+        fa.split = st;
+        fa.route = 0;
+      } else {
+        launch(s, "prep", [&] { return kern::launch_bounds_init(gkey, nq, slots_n, bp.m, s); });
+      }
+      launch(s, "ivf_scan", [&] { return kern::launch_ivf_select(fa, s); });
+      int* flags = k > T ? ar.take<int>((size_t)nq) : nullptr;
+      merge_lists(ar, s, part, nseg, T, k, nq, metric, qnorm, 0, ids, dists, flags, st);
+      if (flags) {
+        // the flagged queries again, over their probed lists' rows (columns out)
+        kern::RedoArgs ra{kd, kq, l2 ? bnorm : nullptr, qnorm, flags, lists, (int)nq, ld, ld, 0, 0,
+                          metric, 0, k, ids, dists, probes, dslots, offsets, P};
+        launch(s, "redo", [&] { return kern::launch_redo(ra, s); });
+      }
+    };
+    // (its workspace counted first, as float_knn_split's)
+    Arena counted = Arena::counting();
+    if (pays) {
+      DryRun dry;
+      scan(counted, true);
     }
-    launch(s, "ivf_scan", [&] { return kern::launch_ivf_select(fa, s); });
-    int* flags = k > T ? ar.take<int>((size_t)nq) : nullptr;
-    merge_lists(ar, s, part, nseg, T, k, nq, metric, qnorm, 0, ids, dists, flags, st);
-    if (flags) {
-      // the flagged queries again, over their probed lists' rows (columns out)
-      kern::RedoArgs ra{kd, kq, l2 ? bnorm : nullptr, qnorm, flags, lists, (int)nq, ld, ld, 0, 0,
-                        metric, 0, k, ids, dists, probes, dslots, offsets, P};
-      launch(s, "redo", [&] { return kern::launch_redo(ra, s); });
-    }
+    scan(ar, pays && counted.used() <= kSplitMaxBytes && ar.reserve(counted.used()));
     kern::IvfMapArgs mp{ids, dists, (int)nq, k, nullptr, 0, probes, dslots, offsets, indices, P,
                         pad};
     launch(s, "ivf_map", [&] { return kern::launch_ivf_map(mp, s); });

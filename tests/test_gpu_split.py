@@ -331,3 +331,51 @@ def test_routes_with_their_own_rounds(engine, oracle, kind, nq, k):
     r = np.random.default_rng(nq)
     base, q = rows_of(kind, N, 128, r), rows_of(kind, nq, 128, r)
     check(engine, oracle, base, q, k, "l2", kind == "bytes")
+
+
+def held_after(engine, call):
+    """Device memory that the engine keeps after one call on an empty workspace."""
+    import ctypes
+
+    from mlxvs_amd import _hip
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        _hip.check(_hip.lib().hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)), "hipMemGetInfo")
+        return a.value
+
+    call()
+    _hip.synchronize()
+    engine.release_workspace()
+    _hip.DeviceBuffer(1 << 20)  # (the runtime returns freed memory by the next allocation)
+    before = free()
+    call()
+    _hip.synchronize()
+    return before - free()
+
+
+def test_workspace_is_what_the_call_takes(engine):
+    """The pieces are as large as the rows and everything else is small: the
+    call's room is made at once, for all of it, and not doubled on the way."""
+    from mlxvs_amd import _hip
+
+    n, nq, d, k = 1_000_000, 2_600, 128, 10
+    base, q = _hip.DeviceBuffer(n * d * 4), _hip.DeviceBuffer(nq * d * 4)
+    ids, dist = _hip.DeviceBuffer(nq * k * 4), _hip.DeviceBuffer(nq * k * 4)
+    r = np.random.default_rng(0)
+    x = r.standard_normal((n, d), np.float32)
+    base.upload(x)
+    q.upload(x[:nq])
+    pieces = (n + nq) * d * 4
+    held = held_after(engine, lambda: engine.brute_force_knn_device(
+        base.value, n, q.value, nq, d, k, "l2", ids.value, dist.value))
+    assert pieces <= held <= 1.25 * pieces
+    lists = 512
+    off = np.linspace(0, n, lists + 1).astype(np.int32)
+    cen, offs, ind = (_hip.DeviceBuffer.from_array(a) for a in
+                      (x[off[:-1]], off, np.arange(n, dtype=np.int32)))
+    held = held_after(engine, lambda: engine.ivf_flat_search_device(
+        cen.value, lists, base.value, n, ind.value, offs.value, d, "l2", q.value, nq, k,
+        ids.value, dist.value, n_probes=16))
+    assert pieces <= held <= 1.25 * pieces
+    engine.release_workspace()
