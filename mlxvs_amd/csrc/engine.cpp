@@ -1259,7 +1259,7 @@ V* to_device(Arena& ar, hipStream_t s, const std::vector<V>& v) {
   return p;
 }
 
-constexpr double kIvfSplitUses = 48;
+constexpr double kIvfSplitUses = 58;
 
 // One search on device pointers.  `off` is the host copy of the offsets
 // when the caller has one (the host-array entry), else null: the work is
@@ -1383,7 +1383,9 @@ void ivf_search(Session& ss, const float* centers, int64_t lists, const float* d
     // rows scanned often enough that their binary16 pieces (SplitState) pay
     // for themselves: 1M x 128 integer (real) rows, 1,024 lists, 20 probes,
     // float32 against pieces: 10,000 queries 1.02 / 0.67 (0.77) ms a call,
-    // 5,000 0.77 / 0.62 (0.69); 2,500 would not gain
+    // 5,000 0.77 / 0.62 (0.69), 4,000 0.70 / 0.60 (0.65), fewer not enough work;
+    // 4M x 128: 3,000 queries (58 uses a list) 1.73 / 1.53 (1.73), 2,500 1.63 /
+    // 1.52 (1.71)
     const int sld = round_up(d, 8);
     const bool pays = !ar.fixed() && n > 0 && kern::fused_split_supported(sld, T) &&
                       npairs >= kIvfSplitUses * (double)lists &&
