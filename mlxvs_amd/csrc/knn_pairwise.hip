@@ -16,7 +16,8 @@
 // A lane keeps the best T rows of its query (a sorted stream list, as the
 // fused kernels), and all splits of a query share a bound on its k-th best
 // (SharedBound).  With k > T the queries whose lists may have been too short are
-// searched again by the scan (launch_pairwise_scan under the merge's flags).  Segments: one per split (part [nq][nsplit][T]).
+// searched again by the scan (launch_pairwise_scan under the merge's flags).
+// Segments: one per split (part [nq][nsplit][T]).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>

@@ -15,9 +15,9 @@
 // With pieces a chunk's fragments feed lo x hi, hi x lo and hi x hi (three
 // products of a chunk that costs two to fetch and to read).
 //
-// What bounds it: at these rates the card lowers its clock (1.5 to 1.7 GHz of
-// 2.4 under every fp16 kernel here, with the MFMA busy half of the time), so
-// what counts is the work beside the products.  Tried at 1M x 1536 x 10,000,
+// What bounds it: at these rates the card lowers its clock (1.82 GHz of 2.4 with
+// pieces, 1.73 on binary16 rows), and the MFMA is busy 67% and 62% of the time,
+// so what counts is the work and the waits beside the products.  Tried at 1M x 1536 x 10,000,
 // binary16 / float32 rows: deep_kernel's 128 x 128 (five fragments for four
 // products) 35.2 / 227 ms (on the float32 MFMA); 256 x 128 with four
 // wavefronts, two workgroups a CU, 64-byte chunks and three stages 37.1 / 108;
