@@ -686,7 +686,7 @@ bool float_knn_split(Session& ss, const FloatInputs& in, int k, int metric, cons
     float *bnorm = nullptr, *qnorm = nullptr, *seed = nullptr;
     float *ubn = nullptr, *uqn = nullptr;  // cosine: |b|^2, |q|^2
     kern::SplitInitArgs si{(const float*)in.base, (const float*)in.queries, n, nq, d, d,
-                           cosine ? 1 : 0, cos_factors ? 1 : 0, l2, st};
+                           cosine ? 1 : 0, cos_factors ? 1 : 0, l2, f16, st};
     launch(s, "prep", [&] { return kern::launch_split_init(si, s); });
     if (cosine) {
       ubn = ar.take<float>((size_t)n);
@@ -1411,7 +1411,7 @@ void ivf_search(Session& ss, const float* centers, int64_t lists, const float* d
         uint16_t* qhi = ar.take<uint16_t>((size_t)nq * sld);
         uint16_t* qlo = ar.take<uint16_t>((size_t)nq * sld);
         float* seed = l2 ? ar.take<float>((size_t)n) : nullptr;
-        const kern::SplitInitArgs si{kd, kq, n, nq, d, ld, 0, 0, l2, st};
+        const kern::SplitInitArgs si{kd, kq, n, nq, d, ld, 0, 0, l2, 0, st};
         launch(s, "prep", [&] { return kern::launch_split_init(si, s); });
         const kern::SplitRowsArgs sb{kd, n, ld, ld, 0, nullptr, bnorm, 1, seed, bhi, blo, sld, 0, l2, st};
         const kern::SplitRowsArgs sq{kq, nq, ld, ld, 0, nullptr, nullptr, 0, nullptr, qhi, qlo, sld,

@@ -90,6 +90,25 @@ enum SplitFlags : uint32_t {
 // dims 1.13 / 1.09 / 1.01 / 0.99 / 0.94 (1.0 at 36 to 0.78 at 128); inner
 // products at 8 / 16 dims 1.09 / 0.80.
 constexpr int kSplitShortL2 = 32, kSplitShortDot = 16;
+// The same where long rows have few terms that count.  `terms`: dims times the
+// rows' spread, (sum |x|)^2 / (d sum x^2), on both sides, over that of normal
+// values (2 / pi each), so that normal rows have d; `held`: the share of pairs of
+// values with none zero (from a sample, 64 values of a row: long tails count for
+// more than they are, log-normal rows for d / 2).  Rms errors, pieces over float32
+// kernels, 100k rows, 3,000 queries, at 36 / 50 / 96 dims:
+//   L2: log-normal rows (terms d / 2) 1.16 / 1.07 / 0.93; 30% zeros (terms and
+//   held d / 2) 1.16 / 1.06 / 0.96; columns whose scales vary by e^3 (terms below
+//   1) 1.30 / 1.18 / 1.02, 1.07 / 1.03 at 160 / 256 and 0.84 at 300 (the tile
+//   kernel's sums with the norms last); half zeros (held 1/4) 1.27 / 1.23 / 1.14,
+//   1.13 at 512, and 80% zeros 1.57 to 1.02: the float32 sums round only where a
+//   product is not zero, a sum of eight nearly always;
+//   inner products: log-normal 1.28 / 1.10 / 0.91; cosine: small counts (terms
+//   d / 4) 1.16 / 1.00 / 0.92.
+constexpr float kSplitNormalSpread = 2.4674011f;  // (pi / 2)^2
+__host__ __device__ constexpr bool split_few_terms(int d, bool l2, float terms, float held) {
+  if (!l2) return d < 64 && terms < 26.0f && terms < 0.6f * (float)d;
+  return held < 0.3f || (d < 64 && terms < 30.0f) || (d <= 256 && terms < 4.0f);
+}
 // Values below 2^-2 in the pieces' scale lose more than their last bit: up to
 // 2^-25, whatever their size.  Under L2 that error meets |q| and stays below
 // the rounding of |q|^2 and |b|^2, so it is judged row by row (kSplitRows32).
@@ -149,6 +168,7 @@ struct SplitInitArgs {
   int unit;
   int factors;  // kSplitFactors (unit)
   int l2;
+  int f16;      // base, queries: binary16 (unit)
   SplitState* st;
 };
 hipError_t launch_split_init(const SplitInitArgs& a, hipStream_t s);

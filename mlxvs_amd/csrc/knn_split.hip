@@ -33,91 +33,158 @@ constexpr float kUnitScale = 32768.0f;
 // columns by a multiplicative hash).  One workgroup, 16 coalesced loads a lane in
 // flight together (values scattered one by one took it 50 us, not 5).
 __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArgs a) {
-  __shared__ float wmax[2][kSampleThreads / 64];
-  __shared__ uint32_t wflags[kSampleThreads / 64];
-  const int tid = threadIdx.x;
+  constexpr int W = kSampleThreads / 64;
+  __shared__ float wmax[2][W], wspread[2][W];
+  __shared__ int wzero[2][W];
+  __shared__ uint32_t wflags[W];
+  const int tid = threadIdx.x, wave = tid >> 6;
   float m[2] = {0.0f, 0.0f};
+  int zeros[2] = {0, 0};
   // what the sample's bits show already (values of more than 11 and 16 bits,
   // values that two pieces do not hold, fractions): set here, the workgroups of
   // the pass need not all report it at once
   uint32_t shown = 0;
-  if (!a.unit) {
-    float v[2][kSamplePer];
+  float v[2][kSamplePer];
+  // (one branch on the type around all loads, which stay in flight together)
+  auto fetch = [&](auto zero) {
+    using E = decltype(zero);
+    E raw[2][kSamplePer];
 #pragma unroll
     for (int side = 0; side < 2; ++side) {
-      const float* x = side ? a.queries : a.base;
+      const E* x = (const E*)(side ? a.queries : a.base);
       const int64_t n = side ? a.nq : a.n;
 #pragma unroll
       for (int i = 0; i < kSamplePer; ++i) {
-        const uint32_t j = (uint32_t)(i * (kSampleThreads / 64) + (tid >> 6));
-        const int64_t r = (int64_t)j * n / (kSamplePer * kSampleThreads / 64);
+        const uint32_t j = (uint32_t)(i * W + wave);
+        const int64_t r = (int64_t)j * n / (kSamplePer * W);
         const uint32_t c = ((j * 2654435761u >> 8) + (tid & 63)) % (uint32_t)a.d;
-        v[side][i] = x[r * a.ld + c];
+        raw[side][i] = x[r * a.ld + c];
       }
     }
 #pragma unroll
     for (int side = 0; side < 2; ++side)
 #pragma unroll
-      for (int i = 0; i < kSamplePer; ++i) {
-        const float x = v[side][i], f = __builtin_amdgcn_frexp_mantf(x);  // (+-[1/2, 1))
-        m[side] = fmaxf(m[side], fabsf(x));
-        if (__float_as_uint(x) & 0x1fffu) shown |= side ? kSplitQueryLow : kSplitBaseLow;
-        if (__float_as_uint(x) & 0xffu) shown |= side ? kSplitQueryLong : kSplitBaseLong;
-        const float rest = f - (float)(_Float16)f;
-        if (rest - (float)(_Float16)rest != 0.0f) shown |= kSplitCut;
-        if (__float_as_uint(__builtin_amdgcn_fractf(x)) & 0x7fffffffu) shown |= kSplitFrac;
-      }
+      for (int i = 0; i < kSamplePer; ++i) v[side][i] = (float)raw[side][i];
+  };
+  if (a.f16)
+    fetch((_Float16)0.0f);
+  else
+    fetch(0.0f);
+#pragma unroll
+  for (int side = 0; side < 2; ++side)
+#pragma unroll
+    for (int i = 0; i < kSamplePer; ++i) {
+      const float x = v[side][i];
+      const uint32_t bits = __float_as_uint(x);
+      m[side] = fmaxf(m[side], fabsf(x));
+      zeros[side] += __popcll(__builtin_amdgcn_ballot_w64(x == 0.0f));
+      if (a.unit) continue;
+      const float f = __builtin_amdgcn_frexp_mantf(x);  // (+-[1/2, 1))
+      if (bits & 0x1fffu) shown |= side ? kSplitQueryLow : kSplitBaseLow;
+      if (bits & 0xffu) shown |= side ? kSplitQueryLong : kSplitBaseLong;
+      const float rest = f - (float)(_Float16)f;
+      if (rest - (float)(_Float16)rest != 0.0f) shown |= kSplitCut;
+      if (__float_as_uint(__builtin_amdgcn_fractf(x)) & 0x7fffffffu) shown |= kSplitFrac;
+    }
+  // Each row's (sum |x|)^2 / (64 sum x^2): 16 rows' sums over the wavefront, lane
+  // l % 16 ending with row l % 16 (base rows, then queries)
+  float s1[2 * kSamplePer], s2[2 * kSamplePer];
+#pragma unroll
+  for (int i = 0; i < 2 * kSamplePer; ++i) {
+    s1[i] = fabsf(v[i / kSamplePer][i % kSamplePer]);
+    s2[i] = s1[i] * s1[i];
   }
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const bool up = tid >> b & 1;
+#pragma unroll
+    for (int i = 0; i < kSamplePer >> b; ++i) {
+      const float a1 = up ? s1[2 * i + 1] : s1[2 * i], b1 = up ? s1[2 * i] : s1[2 * i + 1];
+      const float a2 = up ? s2[2 * i + 1] : s2[2 * i], b2 = up ? s2[2 * i] : s2[2 * i + 1];
+      s1[i] = a1 + __shfl_xor(b1, 1 << b);
+      s2[i] = a2 + __shfl_xor(b2, 1 << b);
+    }
+  }
+#pragma unroll
+  for (int o = 16; o < 64; o <<= 1) {
+    s1[0] += __shfl_xor(s1[0], o);
+    s2[0] += __shfl_xor(s2[0], o);
+  }
+  // (squares past float32's ends: taken as spread evenly)
+  const float sq = s1[0] * s1[0];
+  float spread = s1[0] == 0.0f ? 0.0f : sq >= 0x1p-100f && sq < 0x1p120f ? sq / (64.0f * s2[0]) : 1.0f;
+#pragma unroll
+  for (int o = 1; o < kSamplePer; o <<= 1) spread += __shfl_xor(spread, o);
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
     m[0] = fmaxf(m[0], __shfl_xor(m[0], o));
     m[1] = fmaxf(m[1], __shfl_xor(m[1], o));
+    shown |= __shfl_xor(shown, o);
   }
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) shown |= __shfl_xor(shown, o);
+  static_assert(kSamplePer == 8, "lane 8: the first query row's");
+  if ((tid & 63) == 0 || (tid & 63) == 8) wspread[tid >> 3 & 1][wave] = spread;
   if ((tid & 63) == 0) {
-    wmax[0][tid >> 6] = m[0];
-    wmax[1][tid >> 6] = m[1];
-    wflags[tid >> 6] = shown;
+    for (int side = 0; side < 2; ++side) {
+      wmax[side][wave] = m[side];
+      wzero[side][wave] = zeros[side];
+    }
+    wflags[wave] = shown;
   }
   __syncthreads();
-  if (tid != 0) return;
-  float sc[2];
-  uint32_t flags = a.d < (a.l2 ? kSplitShortL2 : kSplitShortDot) ? kSplitShort : 0u;
-  if (a.unit) flags |= a.factors ? kSplitFactors : kSplitFrac;
-  for (int w = 0; w < kSampleThreads / 64; ++w) flags |= wflags[w];
-  bool large = !a.unit;  // both sides past 2^26: every value an integer, no sum exact
-  for (int side = 0; side < 2; ++side) {
-    float x = 0.0f;
-    for (int w = 0; w < kSampleThreads / 64; ++w) x = fmaxf(x, wmax[side][w]);
-    sc[side] = a.unit ? kUnitScale : 1.0f;
-    if (a.unit) continue;
-    if (x == 0.0f) {  // (a sample of zeros: the pass over all rows decides)
-      large = false;
-      continue;
-    }
+  // the first wavefront: lane 16 side + w takes wavefront w's of that side (lanes
+  // from 32 on repeat them), then lane 0 writes the state
+  if (tid >= 64) return;
+  static_assert(W == 16, "sixteen lanes a side");
+  const int side = tid >> 4 & 1, w = tid & 15;
+  float x = wmax[side][w], part = wspread[side][w];
+  int z = wzero[side][w];
+  uint32_t flags = wflags[w];
+#pragma unroll
+  for (int o = 1; o < 16; o <<= 1) {
+    x = fmaxf(x, __shfl_xor(x, o));
+    part += __shfl_xor(part, o);
+    z += __shfl_xor(z, o);
+    flags |= __shfl_xor(flags, o);
+  }
+  const float sp = part / (float)(kSamplePer * W);
+  const float held = 1.0f - (float)z / (float)(kSamplePer * kSampleThreads);
+  float sc = a.unit ? kUnitScale : 1.0f;
+  // both sides past 2^26: every value an integer, no sum exact
+  const uint32_t large = !a.unit && x >= 0x1p26f;
+  if (!a.unit && x != 0.0f) {  // (a sample of zeros: the pass over all rows decides)
     int e = kMaxSampleExp + 1;
     if (x < INFINITY) (void)frexpf(x, &e);  // x = f 2^e, f in [1/2, 1)
-    if (x < 0x1p26f) large = false;
     if (e < -kMaxSampleExp || e > kMaxSampleExp)
       flags |= kSplitRows32;
     else
-      sc[side] = ldexpf(1.0f, kSampleExp + 1 - e);
+      sc = ldexpf(1.0f, kSampleExp + 1 - e);
   }
-  a.st->flags = large ? flags | kSplitFrac : flags;
-  a.st->sbase = sc[0];
-  a.st->squery = sc[1];
-  a.st->inv = 1.0f / (sc[0] * sc[1]);  // powers of two: exact
+  flags |= __shfl_xor(flags, 16);
+  const float sp_q = __shfl_xor(sp, 16), held_q = __shfl_xor(held, 16);
+  const float sc_q = __shfl_xor(sc, 16);
+  const uint32_t large_q = __shfl_xor(large, 16);
+  if (tid != 0) return;
+  if (a.d < (a.l2 ? kSplitShortL2 : kSplitShortDot) ||
+      split_few_terms(a.d, a.l2, (float)a.d * sp * sp_q * kSplitNormalSpread, held * held_q))
+    flags |= kSplitShort;
+  if (a.unit) flags |= a.factors ? kSplitFactors : kSplitFrac;
+  if (large && large_q) flags |= kSplitFrac;
+  const float cap = split_cap(a.d);
+  SplitState st;
+  st.flags = flags;
+  st.sbase = sc;
+  st.squery = sc_q;
+  st.inv = 1.0f / (sc * sc_q);  // powers of two: exact
   // (the largest values, sums and losses that dense rows reach: only rows past
   // them are reported)
-  const float cap = split_cap(a.d);
-  a.st->cap = cap;
-  a.st->room = (float)a.d * cap;
-  for (int side = 0; side < 2; ++side) {
-    a.st->lost[side] = 0x1p-25f;
-    a.st->top[side] = 0x1p12f;
-    a.st->least[side] = 0.75f * (float)a.d * cap;
+  st.cap = cap;
+  st.room = (float)a.d * cap;
+  for (int i = 0; i < 2; ++i) {
+    st.lost[i] = 0x1p-25f;
+    st.top[i] = 0x1p12f;
+    st.least[i] = 0.75f * (float)a.d * cap;
   }
+  *a.st = st;
 }
 
 // 256 rows per workgroup, a 32-value slab at a time through LDS: fetched with

@@ -200,6 +200,10 @@ def test_integers_of_24_bits(engine, oracle, d):
     ("positive", "l2", 200), ("float", "l2", 768), ("float", "inner_product", 9),
     ("float", "inner_product", 33), ("positive", "inner_product", 300), ("float", "cosine", 96),
     ("float", "cosine", 384),
+    # few terms that count, in long rows too
+    ("half zeros", "l2", 40), ("half zeros", "l2", 128), ("half zeros", "l2", 300),
+    ("sparse", "l2", 96), ("sparse", "l2", 160), ("log-normal", "l2", 40),
+    ("log-normal", "inner_product", 36), ("counts", "cosine", 36),
 ])
 def test_errors_no_larger_than_the_float32_kernels(engine, kind, metric, d):
     """Errors against 64 bits of a batch and of its first 128 queries alone,
@@ -209,6 +213,10 @@ def test_errors_no_larger_than_the_float32_kernels(engine, kind, metric, d):
     n, nq = size_of(d)
     make = {"positive": lambda *s: r.random(s, np.float32),
             "bytes": lambda *s: r.integers(0, 256, s).astype(np.float32),
+            "half zeros": lambda *s: np.maximum(r.standard_normal(s, np.float32), 0),
+            "sparse": lambda *s: np.abs(r.standard_normal(s, np.float32)) * (r.random(s) < 0.05),
+            "log-normal": lambda *s: np.exp(r.standard_normal(s, np.float32)),
+            "counts": lambda *s: r.poisson(0.5, s).astype(np.float32),
             "float": lambda *s: r.standard_normal(s, np.float32)}[kind]
     base, q = make(n, d), make(nq, d)
 
@@ -220,7 +228,7 @@ def test_errors_no_larger_than_the_float32_kernels(engine, kind, metric, d):
         else:
             want = (b * x).sum(2)
             if metric == "cosine":
-                want /= np.linalg.norm(b, axis=2) * np.linalg.norm(x, axis=2)
+                want /= np.maximum(np.linalg.norm(b, axis=2) * np.linalg.norm(x, axis=2), 1e-30)
         return np.sqrt(((dist[:128] - want) ** 2).mean())
 
     assert rms(nq) <= 1.06 * rms(128)
