@@ -76,7 +76,8 @@ enum SplitFlags : uint32_t {
                         // they miss by more than 2^-25 of its length
   kSplitShort = 32,     // sums so short that the pieces' own error shows: only
                         // rows without lo pieces take them
-  // Integers, whose float32 sums are exact as long as they stay below 2^24:
+  // Integers, whose float32 sums are exact as long as they stay below 2^24
+  // (kSplitFactors: multiples of any power of two, alike):
   kSplitFrac = 64,      // some value is none
   kSplitCut = 128,      // some value is not hi + lo (its 24th bit)
   kSplitFactors = 256,  // the float32 route divides dot products of the rows
@@ -84,6 +85,7 @@ enum SplitFlags : uint32_t {
   // Inner products and cosine: some row loses more than rounding
   kSplitBaseLoss = 512,
   kSplitQueryLoss = 1024,
+  kSplitOver9 = 2048,   // (kSplitFactors) some value has more than 9 significant bits
 };
 // Under L2 the lost 24th bits show in sums of few terms: rms error against 64
 // bits, pieces over float32 kernels, of near rows at 16 / 20 / 24 / 28 / 32
@@ -131,12 +133,17 @@ struct SplitState {
   float inv;            // scores from the pieces times inv are the rows' scores
   float cap, room;      // C, d C
   float lost[2], top[2], least[2];  // [base, queries]
+  float fix[2];         // values times this are integers, as far as the sample shows
+                        // (kSplitFactors; else 1)
 };
 // Which kernel a call's rows take: 0 the float32 MFMA, 1 the hi pieces alone
 // (no value has a lo piece: integers, rows that were binary16), 2 both.
 __device__ inline int split_route(const SplitState& s) {
   if (s.flags & kSplitRows32) return 0;
   if (!(s.flags & kSplitFrac) && (s.flags & (kSplitCut | kSplitFactors))) return 0;
+  // (products of at most 18 bits: fewer roundings in float32 sums than in unit
+  // rows; values of 8 bits at 512 dims 1.13 times the float32 kernels' error)
+  if ((s.flags & kSplitFactors) && !(s.flags & kSplitOver9)) return 0;
   if (s.flags & (kSplitBaseLoss | kSplitQueryLoss)) {
     const float error = (s.flags & kSplitBaseLoss ? s.lost[0] * s.top[1] : 0.0f) +
                         (s.flags & kSplitQueryLoss ? s.lost[1] * s.top[0] : 0.0f);

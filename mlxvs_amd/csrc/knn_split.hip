@@ -34,12 +34,12 @@ constexpr float kUnitScale = 32768.0f;
 // flight together (values scattered one by one took it 50 us, not 5).
 __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArgs a) {
   constexpr int W = kSampleThreads / 64;
-  __shared__ float wmax[2][W], wspread[2][W];
-  __shared__ int wzero[2][W];
+  __shared__ float wmax[2][W], wspread[2][W], wsquare[2][W];
+  __shared__ int wunit[2][W], wzero[2][W];
   __shared__ uint32_t wflags[W];
   const int tid = threadIdx.x, wave = tid >> 6;
   float m[2] = {0.0f, 0.0f};
-  int zeros[2] = {0, 0};
+  int unit[2] = {0, 0}, zeros[2] = {0, 0};
   // what the sample's bits show already (values of more than 11 and 16 bits,
   // values that two pieces do not hold, fractions): set here, the workgroups of
   // the pass need not all report it at once
@@ -78,7 +78,14 @@ __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArg
       const uint32_t bits = __float_as_uint(x);
       m[side] = fmaxf(m[side], fabsf(x));
       zeros[side] += __popcll(__builtin_amdgcn_ballot_w64(x == 0.0f));
-      if (a.unit) continue;
+      if (a.unit) {
+        if (a.factors && (bits & 0x7fffu)) shown |= kSplitOver9;
+        // x = odd 2^low, |x| = man 2^(exponent - 150)
+        const uint32_t ex = bits >> 23 & 0xffu;
+        const uint32_t man = (bits & 0x7fffffu) | (ex ? 0x800000u : 0u);
+        if (man) unit[side] = min(unit[side], (int)max(ex, 1u) - 150 + __builtin_ctz(man));
+        continue;
+      }
       const float f = __builtin_amdgcn_frexp_mantf(x);  // (+-[1/2, 1))
       if (bits & 0x1fffu) shown |= side ? kSplitQueryLow : kSplitBaseLow;
       if (bits & 0xffu) shown |= side ? kSplitQueryLong : kSplitBaseLong;
@@ -113,19 +120,29 @@ __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArg
   // (squares past float32's ends: taken as spread evenly)
   const float sq = s1[0] * s1[0];
   float spread = s1[0] == 0.0f ? 0.0f : sq >= 0x1p-100f && sq < 0x1p120f ? sq / (64.0f * s2[0]) : 1.0f;
+  float square = s2[0];  // the largest row's
 #pragma unroll
-  for (int o = 1; o < kSamplePer; o <<= 1) spread += __shfl_xor(spread, o);
+  for (int o = 1; o < kSamplePer; o <<= 1) {
+    spread += __shfl_xor(spread, o);
+    square = fmaxf(square, __shfl_xor(square, o));
+  }
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
     m[0] = fmaxf(m[0], __shfl_xor(m[0], o));
     m[1] = fmaxf(m[1], __shfl_xor(m[1], o));
+    unit[0] = min(unit[0], __shfl_xor(unit[0], o));
+    unit[1] = min(unit[1], __shfl_xor(unit[1], o));
     shown |= __shfl_xor(shown, o);
   }
   static_assert(kSamplePer == 8, "lane 8: the first query row's");
-  if ((tid & 63) == 0 || (tid & 63) == 8) wspread[tid >> 3 & 1][wave] = spread;
+  if ((tid & 63) == 0 || (tid & 63) == 8) {
+    wspread[tid >> 3 & 1][wave] = spread;
+    wsquare[tid >> 3 & 1][wave] = square;
+  }
   if ((tid & 63) == 0) {
     for (int side = 0; side < 2; ++side) {
       wmax[side][wave] = m[side];
+      wunit[side][wave] = unit[side];
       wzero[side][wave] = zeros[side];
     }
     wflags[wave] = shown;
@@ -136,18 +153,24 @@ __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArg
   if (tid >= 64) return;
   static_assert(W == 16, "sixteen lanes a side");
   const int side = tid >> 4 & 1, w = tid & 15;
-  float x = wmax[side][w], part = wspread[side][w];
-  int z = wzero[side][w];
+  float x = wmax[side][w], part = wspread[side][w], sq2 = wsquare[side][w];
+  int u = wunit[side][w], z = wzero[side][w];
   uint32_t flags = wflags[w];
 #pragma unroll
   for (int o = 1; o < 16; o <<= 1) {
     x = fmaxf(x, __shfl_xor(x, o));
     part += __shfl_xor(part, o);
+    sq2 = fmaxf(sq2, __shfl_xor(sq2, o));
+    u = min(u, __shfl_xor(u, o));
     z += __shfl_xor(z, o);
     flags |= __shfl_xor(flags, o);
   }
   const float sp = part / (float)(kSamplePer * W);
   const float held = 1.0f - (float)z / (float)(kSamplePer * kSampleThreads);
+  const float fix = a.factors ? ldexpf(1.0f, min(-u, 100)) : 1.0f;
+  // (a row's sum of squares past 2^24, in these units and with a rounding: what
+  // the pass would find)
+  if (a.factors && !(sq2 * fix * fix < 0x1p25f)) flags |= kSplitFrac;
   float sc = a.unit ? kUnitScale : 1.0f;
   // both sides past 2^26: every value an integer, no sum exact
   const uint32_t large = !a.unit && x >= 0x1p26f;
@@ -161,7 +184,7 @@ __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArg
   }
   flags |= __shfl_xor(flags, 16);
   const float sp_q = __shfl_xor(sp, 16), held_q = __shfl_xor(held, 16);
-  const float sc_q = __shfl_xor(sc, 16);
+  const float sc_q = __shfl_xor(sc, 16), fix_q = __shfl_xor(fix, 16);
   const uint32_t large_q = __shfl_xor(large, 16);
   if (tid != 0) return;
   if (a.d < (a.l2 ? kSplitShortL2 : kSplitShortDot) ||
@@ -179,6 +202,8 @@ __global__ __launch_bounds__(kSampleThreads) void split_init_kernel(SplitInitArg
   // them are reported)
   st.cap = cap;
   st.room = (float)a.d * cap;
+  st.fix[0] = fix;
+  st.fix[1] = fix_q;
   for (int i = 0; i < 2; ++i) {
     st.lost[i] = 0x1p-25f;
     st.top[i] = 0x1p12f;
@@ -220,6 +245,12 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
   const float scale = a.query ? a.st->squery : a.st->sbase;
   const float seed_scale = a.st->sbase * a.st->squery;
   const float cap = a.st->cap;
+  const float fix = a.st->fix[a.query];
+  // (the values' own bits are looked at while the state does not show what they
+  // would)
+  const bool factors = a.st->flags & kSplitFactors;
+  const uint32_t shown = kSplitFrac | (factors ? kSplitOver9 : 0u);
+  const bool look = (a.st->flags & shown) != shown;
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   constexpr int EPV = F16 ? 8 : 4;
   constexpr int VPR = 32 / EPV;
@@ -271,6 +302,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
   uint32_t cutbits = 0;   // of what the pieces leave out: bit 30 (2 and above) only if
                           // a value is past binary16's range or not finite
   uint32_t fracbits = 0;  // of the values' fractions
+  uint32_t rawbits = 0;   // of the values (unit rows)
   bool rows32_seen = false;
   load_slab(0);
   for (int c0 = 0; c0 < a.out_ld; c0 += 32) {
@@ -311,11 +343,21 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
       float x[8];
       *(floatx4*)&x[0] = *(const floatx4*)&sh[r * SS + c];
       *(floatx4*)&x[4] = *(const floatx4*)&sh[r * SS + c + 4];
+      if (look && !a.unit_norms) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) fracbits |= __float_as_uint(__builtin_amdgcn_fractf(x[u]));
+        for (int u = 0; u < 8; ++u) fracbits |= __float_as_uint(__builtin_amdgcn_fractf(x[u]));
+      } else if (look) {
+        // (in units of the side's, SplitState::fix)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          fracbits |= __float_as_uint(__builtin_amdgcn_fractf(x[u] * fix));
+          rawbits |= __float_as_uint(x[u]);
+        }
+        const float nn = a.unit_norms[row];
+        if (!(nn * fix * fix < 0x1p24f)) fracbits = 1u;  // (the sums may pass 2^24)
+      }
       if (a.unit_norms) {
         const float nn = a.unit_norms[row];
-        if (!(nn < 0x1p24f)) fracbits = 1u;  // (the sums may pass 2^24)
         const float nrm = sqrtf(nn);
         const float den = nrm > 1e-30f ? nrm : 1e-30f;
 #pragma unroll
@@ -396,7 +438,8 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitRowsArgs ab, Split
       (any_of(lowbits & 0x7fff7fffu) ? (a.query ? kSplitQueryLow : kSplitBaseLow) : 0u) |
       (any_of(lowbits & 0x003f003fu) ? (a.query ? kSplitQueryLong : kSplitBaseLong) : 0u) |
       (any_of(rows32_seen || (cutbits & 0x40000000u)) ? kSplitRows32 : 0u) |
-      (any_of(fracbits & 0x7fffffffu) ? kSplitFrac : 0u) | (any_of(cutbits) ? kSplitCut : 0u) |
+      (any_of(fracbits & 0x7fffffffu) ? kSplitFrac : 0u) |
+      (any_of(rawbits & 0x7fffu) ? kSplitOver9 : 0u) | (any_of(cutbits) ? kSplitCut : 0u) |
       (any_of(worst > 0.0f) ? (a.query ? kSplitQueryLoss : kSplitBaseLoss) : 0u);
   __shared__ uint32_t rflags[4];
   __shared__ float red[3][4];

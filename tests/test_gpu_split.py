@@ -200,10 +200,11 @@ def test_integers_of_24_bits(engine, oracle, d):
     ("positive", "l2", 200), ("float", "l2", 768), ("float", "inner_product", 9),
     ("float", "inner_product", 33), ("positive", "inner_product", 300), ("float", "cosine", 96),
     ("float", "cosine", 384),
-    # few terms that count, in long rows too
+    # few terms that count, in long rows too; values whose products have few bits
     ("half zeros", "l2", 40), ("half zeros", "l2", 128), ("half zeros", "l2", 300),
     ("sparse", "l2", 96), ("sparse", "l2", 160), ("log-normal", "l2", 40),
     ("log-normal", "inner_product", 36), ("counts", "cosine", 36),
+    ("sixty-fourths", "cosine", 320), ("bfloat16", "cosine", 512),
 ])
 def test_errors_no_larger_than_the_float32_kernels(engine, kind, metric, d):
     """Errors against 64 bits of a batch and of its first 128 queries alone,
@@ -217,6 +218,9 @@ def test_errors_no_larger_than_the_float32_kernels(engine, kind, metric, d):
             "sparse": lambda *s: np.abs(r.standard_normal(s, np.float32)) * (r.random(s) < 0.05),
             "log-normal": lambda *s: np.exp(r.standard_normal(s, np.float32)),
             "counts": lambda *s: r.poisson(0.5, s).astype(np.float32),
+            "sixty-fourths": lambda *s: np.round(r.standard_normal(s, np.float32) * 64) / 64,
+            "bfloat16": lambda *s: (r.standard_normal(s, np.float32).view(np.uint32)
+                                    & np.uint32(0xffff0000)).view(np.float32),
             "float": lambda *s: r.standard_normal(s, np.float32)}[kind]
     base, q = make(n, d), make(nq, d)
 
