@@ -363,7 +363,7 @@ __global__ __launch_bounds__(256, (fused_min_blocks<F16, DH>())) void fused_kern
   };
   query_frags(a.queries, qf);
   if constexpr (NP == 2) query_frags(a.queries_lo, ql);
-  const bool lowlow = NP == 2 && (DH <= 32 || split_low_low(sflags));
+  const bool lowlow = NP == 2 && split_low_low(sflags);
   const char* lbase = NP == 2 ? (const char*)((const E*)a.base_lo + r0 * ld) : nullptr;
 
   // tile t into (dst, ldst, ndst)

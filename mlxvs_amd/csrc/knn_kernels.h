@@ -96,20 +96,25 @@ constexpr int kSplitShortL2 = 32, kSplitShortDot = 16;
 // rows' spread, (sum |x|)^2 / (d sum x^2), on both sides, over that of normal
 // values (2 / pi each), so that normal rows have d; `held`: the share of pairs of
 // values with none zero (from a sample, 64 values of a row: long tails count for
-// more than they are, log-normal rows for d / 2).  Rms errors, pieces over float32
-// kernels, 100k rows, 3,000 queries, at 36 / 50 / 96 dims:
-//   L2: log-normal rows (terms d / 2) 1.16 / 1.07 / 0.93; 30% zeros (terms and
-//   held d / 2) 1.16 / 1.06 / 0.96; columns whose scales vary by e^3 (terms below
-//   1) 1.30 / 1.18 / 1.02, 1.07 / 1.03 at 160 / 256 and 0.84 at 300 (the tile
-//   kernel's sums with the norms last); half zeros (held 1/4) 1.27 / 1.23 / 1.14,
-//   1.13 at 512, and 80% zeros 1.57 to 1.02: the float32 sums round only where a
-//   product is not zero, a sum of eight nearly always;
-//   inner products: log-normal 1.28 / 1.10 / 0.91; cosine: small counts (terms
-//   d / 4) 1.16 / 1.00 / 0.92.
+// more than they are).  Rms errors, pieces over float32 kernels, 100k rows, 3,000
+// queries:
+//   L2: log-normal rows (terms d / 2) 1.16 / 1.07 / 1.06 / 0.93 at 36 / 50 / 64 / 96
+//   dims; normal ones held at 0 (terms 0.55 d) 1.12 / 1.06 / 0.99 / 0.99; 30% zeros
+//   (d / 2) 1.16 / 1.06 / 1.00 / 0.96; Laplace (0.67 d) 0.98 / 0.92 / 0.83; columns
+//   whose scales vary by e^3 (below 1) 1.30 / 1.18 / - / 1.02, 1.07 / 1.03 at 160 /
+//   256 and 0.84 at 300 (the tile kernel's sums with the norms last); half zeros
+//   (held 1/4) 1.27 / 1.23 / - / 1.14, 1.13 at 512, and 80% zeros 1.57 to 1.02: the
+//   float32 sums round only where a product is not zero, a sum of eight nearly
+//   always;
+//   inner products: log-normal 1.72 / 1.28 / 1.10 / 1.00 at 16 / 36 / 56 / 64 dims,
+//   Laplace 1.00 / 0.72 / 0.70 / 0.64; cosine: small counts (d / 4) 1.16 at 36.
 constexpr float kSplitNormalSpread = 2.4674011f;  // (pi / 2)^2
 __host__ __device__ constexpr bool split_few_terms(int d, bool l2, float terms, float held) {
-  if (!l2) return d < 64 && terms < 26.0f && terms < 0.6f * (float)d;
-  return held < 0.3f || (d < 64 && terms < 30.0f) || (d <= 256 && terms < 4.0f);
+  const float share = terms / (float)d;
+  // (the spread of a few values comes out larger)
+  if (!l2) return d <= 64 && terms < 32.0f && share < (d < 24 ? 0.8f : 0.65f);
+  return held < 0.3f || (d <= 64 && (terms < 24.0f || (terms < 40.0f && share < 0.62f))) ||
+         (d <= 256 && terms < 4.0f);
 }
 // Values below 2^-2 in the pieces' scale lose more than their last bit: up to
 // 2^-25, whatever their size.  Under L2 that error meets |q| and stays below
@@ -154,9 +159,10 @@ __device__ inline int split_route(const SplitState& s) {
 }
 // The lo x lo products are at most 2^-22 of a value's product, 2^-25 of it on
 // average; they are formed when both sides have lo pieces and either one side
-// has short values only (at most 16 bits) or all values are integers -- sums that
-// can be exact in float32 --, and for rows of at most 64 values, whose sums have
-// few other roundings.
+// has short values only (at most 16 bits) or all values are integers: sums that
+// can be exact in float32.  (In all rows of at most 64 values they moved the rms
+// errors by 3% at most, 13 kinds of rows at 16 to 64 dims, for a third more
+// products: 135k x 53 cosine, each row a query, k = 35, 9.32 ms against 7.96.)
 __device__ inline bool split_low_low(uint32_t flags) {
   const uint32_t low = kSplitBaseLow | kSplitQueryLow, lng = kSplitBaseLong | kSplitQueryLong;
   return (flags & low) == low && ((flags & lng) != lng || !(flags & kSplitFrac));

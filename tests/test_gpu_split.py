@@ -202,8 +202,9 @@ def test_integers_of_24_bits(engine, oracle, d):
     ("float", "cosine", 384),
     # few terms that count, in long rows too; values whose products have few bits
     ("half zeros", "l2", 40), ("half zeros", "l2", 128), ("half zeros", "l2", 300),
-    ("sparse", "l2", 96), ("sparse", "l2", 160), ("log-normal", "l2", 40),
-    ("log-normal", "inner_product", 36), ("counts", "cosine", 36),
+    ("sparse", "l2", 96), ("sparse", "l2", 160), ("log-normal", "l2", 40), ("log-normal", "l2", 64),
+    ("log-normal", "inner_product", 16), ("log-normal", "inner_product", 36),
+    ("log-normal", "inner_product", 56), ("counts", "cosine", 36),
     ("sixty-fourths", "cosine", 320), ("bfloat16", "cosine", 512),
 ])
 def test_errors_no_larger_than_the_float32_kernels(engine, kind, metric, d):
